@@ -209,15 +209,23 @@ __global__ void icell_k(uint32_t* __restrict__ icell,
     }
 }
 
-// iHoc, LinkList.cl.in:32-42
+// iHoc, LinkList.cl.in:32-42.  The host knows the capacity of ihoc only; the
+// grid in use (n_cells[3], on the device) can be far smaller (a wide domain
+// box around a small tank), so the launch is bounded (IHOC_MAXB workgroups)
+// and strides over the cells in use instead of covering the capacity:
+// 276 -> 4 us for 8 k cells under a capacity of 332 M, and the same 4.3 us
+// as before for 0.3 M cells.
+constexpr unsigned IHOC_MAXB = 2048;
 __global__ void ihoc_fill(uint32_t* __restrict__ ihoc, uint32_t N,
                           const uint32_t* n_cells, uint32_t capacity,
                           const uint32_t* status)
 {
-    const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= capacity || c >= n_cells[3]) return;
     if (status && (*status & 1u)) return;
-    ihoc[c] = N;
+    const uint32_t nc = min(n_cells[3], capacity);
+    const uint32_t stride = gridDim.x * blockDim.x;
+    for (uint64_t c = blockIdx.x * blockDim.x + threadIdx.x; c < nc;
+         c += stride)
+        ihoc[c] = N;
 }
 
 // linkList, LinkList.cl.in:92-113
@@ -693,8 +701,9 @@ void linklist_ihoc(const uint32_t* icell, uint32_t* ihoc, uint32_t N,
                    const uint32_t* n_cells, uint32_t cap,
                    const uint32_t* status, hipStream_t s)
 {
-    hipLaunchKernelGGL(ihoc_fill, dim3(blocks_for(cap, 256)), dim3(256), 0, s,
-                       ihoc, N, n_cells, cap, status);
+    hipLaunchKernelGGL(ihoc_fill,
+                       dim3(std::min(IHOC_MAXB, blocks_for(cap, 256))),
+                       dim3(256), 0, s, ihoc, N, n_cells, cap, status);
     if (N > 1)
         hipLaunchKernelGGL(ihoc_heads, dim3(blocks_for(N - 1, 256)),
                            dim3(256), 0, s, icell, ihoc, N, status);
