@@ -1,0 +1,586 @@
+// Fused fluid walk with several lanes per particle (the same terms and sums
+// as fluid_pass_cells_k of walk_cells.hip, bit for bit).
+//
+// One lane per particle leaves a launch short of work when there are few
+// particles: a 2D cell holds some 16 of them for 64 lanes, and below a few
+// hundred thousand particles there are fewer cells than wavefronts the chip
+// holds, while each particle's pairs (50 in 2D, 250 in 3D) form a serial
+// chain.  Here Q lanes serve one particle: a wavefront takes 64 / Q fluid
+// particles of a cell, and a cell is cut into such groups, handed out to
+// different wavefronts.
+//   test     a chunk of 64 candidates is staged through LDS as in
+//            ring_walk (box prefilter, survivors compacted in order); lane
+//            q of a particle tests the survivors q, q + Q, ..., and every
+//            accepted one is appended, in candidate order, to the
+//            particle's list in LDS (its place from the ballots);
+//   consume  when a list has no room for another chunk (and at the end),
+//            the lanes of every particle with Q B listed take its next Q B,
+//            evaluate their terms, and all Q lanes add the terms in list
+//            order, each term broadcast from its lane by a DPP modifier of
+//            the addition: the Q copies of the sums stay equal, and every
+//            sum takes the terms of the one-lane walk in the same order.
+//            (The particles of a cell accept from different stretches of
+//            the candidate list; consuming only when a list fills up lets
+//            them work side by side.)
+#include "aq_device.hpp"
+#include "aq_internal.hpp"
+#include "walk_device.hpp"
+
+namespace aq {
+
+namespace {
+
+// Orders the LDS accesses of one wavefront (its LDS operations complete in
+// program order; nothing in flight from memory is waited for).
+__device__ __forceinline__ void lds_order()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The value of lane K of the caller's group of Q lanes: DPP quad_perm
+// (Q == 4) or row_newbcast (Q == 16).
+template <int Q, int K> __device__ __forceinline__ float lane_of(float v)
+{
+    static_assert(Q == 4 || Q == 16, "lanes per particle");
+    constexpr int ctrl = Q == 4 ? K * 0x55 : 0x150 + K;
+    return __int_as_float(__builtin_amdgcn_update_dpp(
+        0, __float_as_int(v), ctrl, 0xf, 0xf, true));
+}
+// f(lane 0's v), f(lane 1's v), ... of the caller's group, in that order
+template <int Q, int K = 0, class F>
+__device__ __forceinline__ void each_lane(float v, F f)
+{
+    if constexpr (K < Q) {
+        f(lane_of<Q, K>(v));
+        each_lane<Q, K + 1>(v, f);
+    }
+}
+
+template <int Q, int B, bool PER> struct CoopLds {
+    uint32_t start[27];
+    uint32_t cum[28];
+    float4 stage[64];
+    uint32_t candj[64];
+    // ring of accepted candidates of each particle
+    static constexpr uint32_t CAP = Q == 4 ? 128 : 256;
+    uint32_t list[64 / Q][CAP];
+    uint32_t owns[64 / Q];
+    float4 shift[PER ? 27 : 1];
+};
+
+// Walk the accepted candidates of one particle per group of Q lanes.  kind,
+// flag_el, el_near and the relative test (LOOSE): as in ring_walk.
+// round(n, cw): one round, in which lane q of the group takes the list
+// entries q + Q b < n (cw[b]); called by every lane.
+template <int D, int Q, int B, bool LOOSE, bool PER, class Round>
+__device__ __forceinline__ void
+coop_list_walk(CoopLds<Q, B, PER>& L, int lane, uint32_t total,
+               const f3& r_i, bool act, const f3& bmin, const f3& bmax,
+               float smax, const float* __restrict__ r,
+               const int* __restrict__ imove, int kind, bool flag_el,
+               bool& el_near, const float* __restrict__ per, Round round)
+{
+    static_assert(!(LOOSE && PER), "relative test: not for periodic walks");
+    const int q = lane & (Q - 1), o = lane / Q;
+    uint32_t* list = L.list[o];
+    f3 cen = { 0.f, 0.f, 0.f }, rio = r_i;
+    float ai = 0.f, smaxl = smax;
+    if constexpr (LOOSE) {
+        if (bmin.x <= bmax.x) {
+            cen = f3{ uni_f(0.5f * (bmin.x + bmax.x)),
+                      uni_f(0.5f * (bmin.y + bmax.y)),
+                      D == 3 ? uni_f(0.5f * (bmin.z + bmax.z)) : 0.f };
+            const f3 hd = sub<D>(bmax, cen);
+            const float rb = sqrtf(dot<D>(hd, hd)) * 1.0001f + sqrtf(smax);
+            smaxl = uni_f(smax + rb * rb * 0x1p-14f);
+        }
+        rio = sub<D>(r_i, cen);
+        ai = dot<D>(rio, rio);
+    }
+    int kl = 0;         // neighbour cell of the lane's next candidate
+    uint32_t head = 0, pend = 0;  // the particle's ring: first entry, entries
+    constexpr uint32_t CAP = CoopLds<Q, B, PER>::CAP;
+    bool eln = false;
+    // the loads of the next chunk are issued before a chunk is tested
+    uint32_t j = 0;
+    int klj = 0, im_j = 0;
+    f3 rj = { 0.f, 0.f, 0.f };
+    auto fetch = [&](uint32_t cb) {
+        const uint32_t t = cb + (uint32_t)lane;
+        im_j = 0;
+        if (t < total) {
+            while (t >= L.cum[kl + 1]) kl++;
+            j = L.start[kl] + (t - L.cum[kl]);
+            klj = kl;
+            rj = ldv_o<D>(r, j);
+            im_j = ldi_o(imove, j);
+        }
+    };
+    // rounds while some particle has `most` or more listed; those with a
+    // whole round's worth (any, at the end) take part
+    auto consume = [&](uint32_t most, uint32_t least) {
+        while (__ballot(pend >= most) != 0) {
+            const uint32_t n =
+                pend >= least ? min(pend, (uint32_t)(Q * B)) : 0u;
+            uint32_t cw[B];
+#pragma unroll
+            for (int b = 0; b < B; b++)
+                cw[b] = list[(head + (uint32_t)(q + Q * b)) & (CAP - 1)];
+            round(n, cw);
+            head += n;
+            pend -= n;
+        }
+    };
+    fetch(0);
+    for (uint32_t cb = 0; cb < total; cb += 64) {
+        // stage the chunk
+        bool take = false, is_el = false;
+        float4 st = make_float4(0.f, 0.f, 0.f, 0.f);
+        const uint32_t word =
+            PER ? (j | ((uint32_t)klj << PER_KL_SHIFT)) : j;
+        if (cb + (uint32_t)lane < total) {
+            if constexpr (PER) {
+                const float4 sh = L.shift[klj];
+                rj = per_shift<D>(rj, f3{ sh.x, sh.y, sh.z }, per);
+            }
+            is_el = (im_j == -3);
+            take = kind ? is_el : (im_j == 1 || (flag_el && is_el));
+            if (take) {
+                const float dx =
+                    fmaxf(fmaxf(bmin.x - rj.x, rj.x - bmax.x), 0.f);
+                const float dy =
+                    fmaxf(fmaxf(bmin.y - rj.y, rj.y - bmax.y), 0.f);
+                float d2 = dx * dx;
+                d2 = d2 + dy * dy;
+                if constexpr (D == 3) {
+                    const float dz =
+                        fmaxf(fmaxf(bmin.z - rj.z, rj.z - bmax.z), 0.f);
+                    d2 = d2 + dz * dz;
+                }
+                take = !(d2 > smax);
+            }
+            if constexpr (LOOSE) {
+                const f3 rjo = sub<D>(rj, cen);
+                float bj = rjo.x * rjo.x;
+                bj = __builtin_fmaf(rjo.y, rjo.y, bj);
+                if constexpr (D == 3) bj = __builtin_fmaf(rjo.z, rjo.z, bj);
+                st = make_float4(rjo.x, rjo.y, rjo.z, is_el ? -bj : bj);
+            } else {
+                st = make_float4(rj.x, rj.y, rj.z, is_el ? -1.f : 1.f);
+            }
+        }
+        const uint64_t tm = __ballot(take);
+        const uint32_t cnt = (uint32_t)__popcll(tm);
+        if (cnt != 0) {
+            const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
+                (uint32_t)(tm >> 32),
+                __builtin_amdgcn_mbcnt_lo((uint32_t)tm, 0u));
+            if (take) {
+                L.stage[rank] = st;
+                L.candj[rank] = word;
+            }
+        }
+        if (cb + 64 < total) fetch(cb + 64);
+        if (cnt == 0) continue;
+        lds_order();
+        const bool els = !kind && __ballot(take && is_el) != 0;
+        // survivors q, q + Q, ...: the bits of the group's lanes are the
+        // accept flags of Q successive survivors
+        const uint32_t sh = ((uint32_t)(o * Q)) & 31u;
+        const bool upper = o * Q >= 32;
+        const uint32_t below = (1u << q) - 1u;
+        for (uint32_t t = 0; t < cnt; t += Q) {
+            const uint32_t k = t + (uint32_t)q;
+            const float4 c = L.stage[k & 63u];
+            bool acc;
+            if constexpr (LOOSE) {
+                float d = rio.x * c.x;
+                d = __builtin_fmaf(rio.y, c.y, d);
+                if constexpr (D == 3) d = __builtin_fmaf(rio.z, c.z, d);
+                const float s = __builtin_fmaf(-2.f, d, ai + fabsf(c.w));
+                acc = !(s > smaxl);
+            } else {
+                const f3 r_ij = sub<D>(f3{ c.x, c.y, c.z }, r_i);
+                const float s = dot<D>(r_ij, r_ij);
+                acc = !(s > smax);
+            }
+            acc = acc && act && k < cnt;
+            if (els) {
+                // wall elements in range: flagged, then dropped
+                const bool e = (__float_as_uint(c.w) >> 31) != 0u;
+                eln = eln || (acc && e);
+                acc = acc && !e;
+            }
+            const uint64_t bm = __ballot(acc);
+            const uint32_t half =
+                upper ? (uint32_t)(bm >> 32) : (uint32_t)bm;
+            const uint32_t mine =
+                Q == 4 ? (half >> sh) & 15u : (half >> sh) & 0xFFFFu;
+            if (acc)
+                list[(head + pend + (uint32_t)__popc(mine & below)) &
+                     (CAP - 1)] = L.candj[k];
+            pend += (uint32_t)__popc(mine);
+        }
+        lds_order();
+        consume(CAP - 63, Q * B);  // room for the next chunk
+    }
+    consume(1, 1);
+    // every lane of the group learns what one of them saw
+    const uint64_t em = __ballot(eln);
+    constexpr uint64_t grp = Q == 4 ? 15ull : 0xFFFFull;
+    el_near = ((em >> (o * Q)) & grp) != 0;
+    lds_order();
+}
+
+// See fluid_pass_cells_k.  Item k of the launch is group k % S of the fluid
+// particles of the k / S-th cell: its particles (S t + k % S) OW + 0 .. OW -
+// 1 for t = 0, 1, ..., OW = 64 / Q.  nlist gets one entry per item with a
+// near particle: the runs of particles of different items do not overlap,
+// so BI Interactions meets every near particle once.
+template <int D, int SHEP, int MATH, bool PER, int Q, int B>
+__global__ void __launch_bounds__(64 * WC_WAVES)
+    fluid_coop_k(const int* __restrict__ imove, const float* __restrict__ r,
+                 const float* __restrict__ u, const float* __restrict__ rho,
+                 const float* __restrict__ m, const float* __restrict__ p,
+                 const float* __restrict__ normal,
+                 const float* __restrict__ tangent,
+                 const float* __restrict__ binormal,
+                 float* __restrict__ shepard, float* __restrict__ grad_p,
+                 float* __restrict__ lap_u, float* __restrict__ div_u,
+                 float* __restrict__ lap_p, uint8_t* __restrict__ near,
+                 WalkArgs w, float H, float CONW, float CONF, float DIMS,
+                 float smax, const uint32_t* __restrict__ rec, int lapf,
+                 int lapp_, uint32_t S)
+{
+    constexpr int OW = 64 / Q;
+    constexpr bool LOOSE = !PER;
+    const bool lapp = lapp_ != 0;
+    __shared__ CoopLds<Q, B, PER> lds[WC_WAVES];
+    const int lane = threadIdx.x & 63;
+    const int wv = threadIdx.x >> 6;
+    const int q = lane & (Q - 1), o = lane / Q;
+    CoopLds<Q, B, PER>& L = lds[wv];
+    if (w.status && (*w.status & 1u)) return;
+    const uint32_t n_items = uni(*w.n_heads) * S;
+    const float eps = 1E-8f * H;
+    const bool flag_el = (SHEP == 2) || (near != nullptr);
+    const uint32_t nwv = gridDim.x * WC_WAVES;
+    uint32_t item = blockIdx.x * WC_WAVES + (uint32_t)wv;
+    if (item >= n_items) return;
+    float fdT = 0.f;
+    if (rec) fdT = fast_threshold<D>(rec, H, CONF, smax, lapf, lapp);
+    const bool fastdiv = fdT > 0.f;
+    const Rcp RH = rcp_nr(H);
+    auto rjof = [&](uint32_t j, uint32_t kl) {
+        f3 v = ldv_o<D>(r, j);
+        if constexpr (PER) {
+            const float4 s = L.shift[kl];
+            v = per_shift<D>(v, f3{ s.x, s.y, s.z }, w.per);
+        }
+        return v;
+    };
+    for (; item < n_items; item += nwv) {
+        const uint32_t hk = item / S, sub_i = item % S;
+        uint32_t cstart, c_i, ce;
+        if (w.blist) {
+            cstart = uni(w.blist[3 * hk]);
+            c_i = uni(w.blist[3 * hk + 1]);
+            ce = uni(w.blist[3 * hk + 2]);
+        } else {
+            cstart = uni(w.heads[hk]);
+            c_i = uni(w.icell[cstart]);
+            ce = uni(w.cell_end[c_i]);
+        }
+        const uint32_t cend = ce & AQ_CELL_END;
+        if (w.flagged && !(ce & AQ_CELL_FLUID)) continue;  // no fluid here
+        for (uint32_t lo = sub_i * OW;; lo += S * OW) {
+            // fluid particles lo .. lo + OW - 1 of the cell
+            uint32_t seen = 0, nf = 0;
+            for (uint32_t pos = cstart; pos < cend && nf < (uint32_t)OW;
+                 pos += 64) {
+                const uint32_t ii = pos + (uint32_t)lane;
+                const bool fl = ii < cend && imove[ii] == 1;
+                const uint64_t bm = __ballot(fl);
+                const uint32_t rank =
+                    seen + __builtin_amdgcn_mbcnt_hi(
+                               (uint32_t)(bm >> 32),
+                               __builtin_amdgcn_mbcnt_lo((uint32_t)bm, 0u));
+                if (fl && rank >= lo && rank < lo + OW)
+                    L.owns[rank - lo] = ii;
+                seen += (uint32_t)__popcll(bm);
+                nf = seen > lo ? min(seen - lo, (uint32_t)OW) : 0u;
+            }
+            if (nf == 0) break;
+            const uint32_t total = neighbour_table<D, PER>(
+                w, c_i, L, lane,
+                AQ_CELL_FLUID | (flag_el ? AQ_CELL_ELEM : 0u));
+            const bool act = (uint32_t)o < nf;
+            const uint32_t i = act ? L.owns[o] : cstart;
+            f3 r_i = { 0.f, 0.f, 0.f }, u_i = { 0.f, 0.f, 0.f };
+            float p_i = 0.f, rho_i = 1.f;
+            f3 gp = { 0.f, 0.f, 0.f }, lu = { 0.f, 0.f, 0.f };
+            float dv = 0.f, lp = 0.f, sh = 0.f;
+            f3 cgp = { 0.f, 0.f, 0.f }, clu = { 0.f, 0.f, 0.f };
+            float cdv = 0.f, clp = 0.f;
+            if (act) {
+                r_i = ldv<D>(r, i);
+                u_i = ldv<D>(u, i);
+                p_i = p[i];
+                rho_i = rho[i];
+                gp = ldv<D>(grad_p, i);
+                lu = ldv<D>(lap_u, i);
+                dv = div_u[i];
+                if (lapp) lp = lap_p[i];
+                sh = (SHEP == 2) ? 1.f : (SHEP == 1 ? shepard[i] : 0.f);
+            }
+            bool nearw = false;
+            f3 bmin, bmax;
+            wave_box<D>(r_i, act, bmin, bmax);
+            auto acc1 = [&](float& s, float& c, float v) {
+                each_lane<Q>(v, [&](float x) {
+                    if constexpr (MATH == 2) nsum(s, c, x);
+                    else s += x;
+                });
+            };
+            // ---- fluid neighbours ------------------------------------------
+            // A lane without a candidate adds zeros, and so does a candidate
+            // of the relative test's shell beyond the support (zero mass):
+            // the sums are never -0 (they start at +0, or 1, and an exact
+            // cancellation rounds to +0), so +-0 leaves them unchanged.
+            auto round = [&](uint32_t n, const uint32_t (&cw)[B]) {
+                f3 rc[B], uc[B];
+                float mc[B], rhoc[B], pc[B];
+#pragma unroll
+                for (int b = 0; b < B; b++) {
+                    if ((uint32_t)(q + Q * b) >= n) continue;
+                    const uint32_t j = PER ? cw[b] & PER_J_MASK : cw[b];
+                    rc[b] = rjof(j, PER ? cw[b] >> PER_KL_SHIFT : 0u);
+                    mc[b] = ldf_o(m, j);
+                    rhoc[b] = ldf_o(rho, j);
+                    pc[b] = ldf_o(p, j);
+                    uc[b] = ldv_o<D>(u, j);
+                }
+#pragma unroll
+                for (int b = 0; b < B; b++) {
+                    PairTerms t{ 0.f, 0.f, 0.f, 0.f, 0.f };
+                    f3 g = { 0.f, 0.f, 0.f }, l = { 0.f, 0.f, 0.f };
+                    if ((uint32_t)(q + Q * b) < n) {
+                        const f3 r_ij = sub<D>(rc[b], r_i);
+                        const float s = dot<D>(r_ij, r_ij);
+                        float m_j = mc[b];
+                        if (LOOSE) m_j = (s > smax) ? 0.f : m_j;
+                        const f3 u_ij = sub<D>(uc[b], u_i);
+                        const float udr = dot<D>(u_ij, r_ij);
+                        const bool fd =
+                            fastdiv && !(((s < 0x1p-96f) & (s != 0.f)) |
+                                         ((udr != 0.f) & (fabsf(udr) < fdT)));
+                        if (fd)
+                            t = fluid_pair<D, SHEP, true>(
+                                lapf, lapp, div_nr(sqrt_nr(s), RH), m_j,
+                                rhoc[b], pc[b], udr, p_i, rho_i, H, CONW,
+                                CONF);
+                        else
+                            t = fluid_pair<D, SHEP, false>(
+                                lapf, lapp, sqrtf(s) / H, m_j, rhoc[b], pc[b],
+                                udr, p_i, rho_i, H, CONW, CONF);
+                        const f3 v = lapf == AQ_LAP_MONAGHAN ? r_ij : u_ij;
+                        g = scl<D>(t.sg, r_ij);
+                        l = scl<D>(t.sl, v);
+                    }
+                    if constexpr (SHEP == 1)
+                        each_lane<Q>(t.sh, [&](float x) { sh += x; });
+                    acc1(gp.x, cgp.x, g.x);
+                    acc1(gp.y, cgp.y, g.y);
+                    if constexpr (D == 3) acc1(gp.z, cgp.z, g.z);
+                    acc1(lu.x, clu.x, l.x);
+                    acc1(lu.y, clu.y, l.y);
+                    if constexpr (D == 3) acc1(lu.z, clu.z, l.z);
+                    acc1(dv, cdv, t.td);
+                    acc1(lp, clp, t.tl);  // zeros without lap p
+                }
+            };
+            coop_list_walk<D, Q, B, LOOSE, PER>(
+                L, lane, total, r_i, act, bmin, bmax, smax, r, imove, 0,
+                flag_el, nearw, w.per, round);
+            // ---- wall elements (boundary-integral Shepard) ------------------
+            if constexpr (SHEP == 2) {
+                if (__ballot(nearw) != 0) {
+                    bool self_added = false, unused = false;
+                    const uint32_t total_el =
+                        neighbour_table<D, PER>(w, c_i, L, lane, AQ_CELL_ELEM);
+                    auto round_el = [&](uint32_t n, const uint32_t (&cw)[B]) {
+#pragma unroll
+                        for (int b = 0; b < B; b++) {
+                            // v: the element's part; on: the particle lies on
+                            // the element (1/2, once)
+                            float v = 0.f;
+                            bool on = false;
+                            if ((uint32_t)(q + Q * b) < n) {
+                                const uint32_t j = cw[b];
+                                const f3 r_ij = sub<D>(ldv_o<D>(r, j), r_i);
+                                const float s = dot<D>(r_ij, r_ij);
+                                const f3 n_j = ldv_o<D>(normal, j);
+                                const f3 t_j = ldv_o<D>(tangent, j);
+                                const f3 b_j = ldv_o<D>(binormal, j);
+                                const float area_j = ldf_o(m, j);
+                                const float qq = sqrtf(s) / H;
+                                const float r_n = dot<D>(r_ij, n_j);
+                                const float r_t = fabsf(dot<D>(r_ij, t_j));
+                                const float r_b = fabsf(dot<D>(r_ij, b_j));
+                                if (LOOSE && s > smax) {
+                                } else if ((r_n > -eps) && (r_n < eps)) {
+                                    const float dr =
+                                        0.55f *
+                                        pow_cl(area_j, 1.f / (DIMS - 1.f));
+                                    on = (r_t <= dr) && (r_b <= dr);
+                                } else {
+                                    v = r_n * CONW * kernelS_P<D>(qq) *
+                                            area_j +
+                                        kernelS_D<D>(fabsf(r_n), r_t, r_b,
+                                                     area_j);
+                                }
+                            }
+                            if (__ballot(on) == 0) {
+                                each_lane<Q>(v, [&](float x) { sh += x; });
+                            } else {
+                                // the half angle in its place in the order
+                                float f = on ? 1.f : 0.f;
+                                float xs[Q], fs[Q];
+                                int k = 0;
+                                each_lane<Q>(v, [&](float x) { xs[k++] = x; });
+                                k = 0;
+                                each_lane<Q>(f, [&](float x) { fs[k++] = x; });
+#pragma unroll
+                                for (int e = 0; e < Q; e++) {
+                                    if (fs[e] != 0.f) {
+                                        if (!self_added) {
+                                            self_added = true;
+                                            sh -= 0.5f;
+                                        }
+                                    } else {
+                                        sh += xs[e];
+                                    }
+                                }
+                            }
+                        }
+                    };
+                    coop_list_walk<D, Q, B, LOOSE, PER>(
+                        L, lane, total_el, r_i, act && nearw, bmin, bmax,
+                        smax, r, imove, 1, false, unused, w.per, round_el);
+                }
+            }
+            if (act && q == 0) {
+                if constexpr (MATH == 2) {
+                    gp = { gp.x + cgp.x, gp.y + cgp.y, gp.z + cgp.z };
+                    lu = { lu.x + clu.x, lu.y + clu.y, lu.z + clu.z };
+                    dv += cdv;
+                    lp += clp;
+                }
+                stxyz<D>(grad_p, i, gp);
+                stxyz<D>(lap_u, i, lu);
+                div_u[i] = dv;
+                if (lapp) lap_p[i] = lp;
+                if (SHEP) shepard[i] = sh;
+                if (near) near[i] = nearw ? 1 : 0;
+            }
+            if (w.nlist && __ballot(act && nearw) != 0 && lane == 0) {
+                uint32_t* cnt =
+                    const_cast<uint32_t*>(w.n_heads) + AQ_CL_NNCELLS;
+                const uint32_t k = atomicAdd(cnt, 1u);
+                w.nlist[3 * k] = L.owns[0];
+                w.nlist[3 * k + 1] = c_i;
+                w.nlist[3 * k + 2] =
+                    (L.owns[nf - 1] + 1u) | (ce & ~AQ_CELL_END);
+            }
+            lds_order();
+            if (nf < (uint32_t)OW) break;
+        }
+    }
+}
+
+}  // namespace
+
+// Lanes per particle of the fused walk for N particles (the host knows no
+// other count); 0: the one-lane walk of walk_cells.hip.  Walk times in us,
+// one lane / 4 lanes / 16 lanes, on dam breaks with their walls:
+//   2D      2 k 107 / 34 / 27     8 k 104 / 35 / 28    31 k 101 / 38 / 45
+//         184 k 185 / 92 / 159   1.1 M 820 / 435 / 869
+//   3D      9 k 513 / 120 / 71   20 k 532 / 126 / 115   38 k 533 / 146 / 162
+//         135 k 634 / 326 / 440  240 k 651 / 535 / 714  394 k 880 / 791 / -
+//         627 k 1144 / 1269 / -
+// A 2D cell has 16 particles, so four lanes each fill a wavefront at any
+// size; a 3D cell has 64, and one lane each wins once the cells fill the
+// chip: 4096 wavefronts, 262 k fluid particles, where four still gain on a
+// flow out of lattice order and lose on the lattice (periodic cube of 262 k:
+// 764 / 669 and 584 / 633).  The
+// compensated sums (math == 2) take their six operations per term on every
+// lane of the group, which moves that line down (135 k 693 / 455, 240 k
+// 746 / 760); 16 lanes pay it 16 times (2D 8 k 109 / 39 / 37, 31 k 107 / 44
+// / 72; 3D 9 k 558 / 154 / 114, 20 k 576 / 165 / 192).
+int fluid_coop_lanes(int dims, uint32_t N, int math)
+{
+    const bool comp = math == 2;
+    if (dims == 2) return N <= (comp ? 8000u : 16000u) ? 16 : 4;
+    if (N <= (comp ? 12000u : 24000u)) return 16;
+    return N <= (comp ? 200000u : 250000u) ? 4 : 0;
+}
+
+void launch_fluid_coop(int dims, int shep, bool lapp, int q,
+                       const int32_t* imove, const float* r, const float* u,
+                       const float* rho, const float* m, const float* p,
+                       const float* normal, const float* tangent,
+                       const float* binormal, float* shepard, float* grad_p,
+                       float* lap_u, float* div_u, float* lap_p,
+                       uint8_t* near, const WalkArgs& w, aq_defs d,
+                       float smax, int math, const uint32_t* rec,
+                       hipStream_t s)
+{
+    // a 2D cell holds one group of 16 particles, a 3D cell four
+    const uint32_t S = q == 16 ? (dims == 2 ? 4u : 16u)
+                               : (dims == 2 ? 1u : 4u);
+#define AQ_CO4(DD, SH, MM, PR, QQ, BB)                                         \
+    do {                                                                       \
+        auto* ker = fluid_coop_k<DD, SH, MM, PR, QQ, BB>;                      \
+        const unsigned nb =                                                    \
+            std::min(resident_blocks((const void*)ker, 64 * WC_WAVES),         \
+                     std::max(1u, blocks_for((size_t)w.N * QQ * 2,             \
+                                             64 * WC_WAVES)));                 \
+        hipLaunchKernelGGL(ker, dim3(nb), dim3(64 * WC_WAVES), 0, s, imove, r, \
+                           u, rho, m, p, normal, tangent, binormal, shepard,   \
+                           grad_p, lap_u, div_u, lap_p, near, w, d.H, d.CONW,  \
+                           d.CONF, d.DIMS, smax, rec, d.lap_formulation,       \
+                           lapp ? 1 : 0, S);                                   \
+    } while (0)
+#define AQ_CO3(DD, SH, MM, PR)                                                 \
+    do {                                                                       \
+        if (q == 16) AQ_CO4(DD, SH, MM, PR, 16, 1);                            \
+        else AQ_CO4(DD, SH, MM, PR, 4, 1);                                     \
+    } while (0)
+#define AQ_CO2(DD, SH, MM)                                                     \
+    do {                                                                       \
+        if (w.per && SH != 2) AQ_CO3(DD, SH, MM, (SH != 2));                   \
+        else AQ_CO3(DD, SH, MM, false);                                        \
+    } while (0)
+#define AQ_CO1(DD, SH)                                                         \
+    do {                                                                       \
+        if (math == 2) AQ_CO2(DD, SH, 2);                                      \
+        else AQ_CO2(DD, SH, 0);                                                \
+    } while (0)
+    if (dims == 2) {
+        if (shep == 0) AQ_CO1(2, 0);
+        else if (shep == 1) AQ_CO1(2, 1);
+        else AQ_CO1(2, 2);
+    } else {
+        if (shep == 0) AQ_CO1(3, 0);
+        else if (shep == 1) AQ_CO1(3, 1);
+        else AQ_CO1(3, 2);
+    }
+#undef AQ_CO1
+#undef AQ_CO2
+#undef AQ_CO3
+#undef AQ_CO4
+}
+
+}  // namespace aq

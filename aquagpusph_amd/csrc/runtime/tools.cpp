@@ -582,17 +582,21 @@ class LinkListTool : public Tool {
                 c.cell_end = nullptr;
                 AQ_HIP(hipMalloc(&c.cell_end, ihoc_->length * 4));
                 c.cap = ihoc_->length;
-                // cell triplets: at most one per non-empty cell, and the
-                // owner lists one more per AQ_OWNER_CHUNK non-fluid
-                // particles of the cells split into runs
+                // cell triplets: at most one per non-empty cell, the owner
+                // lists one more per AQ_OWNER_CHUNK non-fluid particles of
+                // the cells split into runs, and the near list one per group
+                // of at least 4 fluid particles (each group but a cell's
+                // last is full)
                 const size_t ncap = std::min<size_t>(S.N, c.cap);
                 for (uint32_t** l : { &c.ocells, &c.wcells, &c.nlist,
                                       &c.bcells }) {
                     if (*l) AQ_HIP(hipFree(*l));
                     *l = nullptr;
                     const bool own = l == &c.ocells || l == &c.wcells;
-                    AQ_HIP(hipMalloc(
-                        l, (own ? aq_owner_list_cap(ncap, S.N) : ncap) * 12));
+                    const size_t n =
+                        own ? aq_owner_list_cap(ncap, S.N)
+                            : l == &c.nlist ? ncap + S.N / 4 + 1 : ncap;
+                    AQ_HIP(hipMalloc(l, n * 12));
                 }
                 // the blocked order's per-block counters (zero between
                 // steps) and bases

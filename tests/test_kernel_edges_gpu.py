@@ -45,3 +45,69 @@ def test_ihoc_table_of_wide_grids(cuda, cells, cap):
     got = ihoc.cpu().numpy()
     np.testing.assert_array_equal(got[:cells], want)
     assert (got[cells:] == -7).all()
+
+
+def _run(tmp_path, case, presets, tag, steps=3):
+    from aquagpusph_amd import casefiles
+    from aquagpusph_amd.sim import Simulation
+    d = tmp_path / tag
+    sim = Simulation(casefiles.write_case(case, str(d), presets=presets,
+                                          load=False), case["dims"])
+    casefiles.upload(sim, case)
+    sim.step(steps, graph=True)
+    out = {k: sim.get(k) for k in ("id", "r", "u", "rho", "p", "dudt",
+                                   "drhodt", "grad_p", "lap_u", "div_u",
+                                   "lap_p", "shepard")}
+    sim.close()
+    return out
+
+
+def _stir(case, seed):
+    """Displaced fluid particles and a velocity field (a flow out of its
+    lattice order, so that cells hold uneven numbers of particles)."""
+    rng = np.random.default_rng(seed)
+    fl, D = case["imove"] == 1, case["dims"]
+    n = int(fl.sum())
+    case["r"][fl, :D] += 0.3 * case["params"]["dr"] * rng.uniform(
+        -1, 1, (n, D))
+    case["u"][fl, :D] = rng.normal(0, 0.3, (n, D))
+    return case
+
+
+# sizes on both sides of the lines between 16, 4 and one lane per particle
+@pytest.mark.parametrize("dims,dr,kind", [
+    (2, 0.06, "wall"), (2, 0.011, "wall"), (2, 0.0028, "wall"),
+    (2, 0.011, "kahan"), (2, 0.0031, "kahan"), (3, 0.05, "wall"),
+    (3, 0.031, "wall"), (3, 0.0187, "wall"), (3, 0.031, "kahan"),
+    (3, 0.0187, "kahan"), (2, 1 / 41, "box"), (2, 1 / 160, "box"),
+    (3, 1 / 17, "box"), (3, 1 / 33, "box"), (2, 0.011, "morris"),
+    (3, 0.031, "morris")])
+def test_lanes_per_particle_are_bit_identical(cuda, tmp_path, monkeypatch,
+                                              dims, dr, kind):
+    """The fused walk with 4 or 16 lanes per particle against the one-lane
+    walk (asked for by an explicit grid), bit for bit: every sum takes the
+    same terms in the same order."""
+    from aquagpusph_amd import casefiles, cases
+    pres = casefiles.PBI_PRESETS
+    if kind == "box":
+        case = cases.periodic_box(dims, int(round(1 / dr)), seed=3)
+        pres = casefiles.PPER_PRESETS
+    else:
+        case = cases.dam_break(dims, dr)
+        if kind == "kahan":
+            pres = pres + ("resources/Presets/precision.xml",)
+    case = _stir(case, 7)
+    extra = ""
+    if kind == "morris":
+        from aquagpusph_amd import casefiles as cf
+        orig = cf.write_case
+        extra = ('    <Definitions><Define name="__LAP_FORMULATION__" '
+                 'value="2" evaluate="false"/></Definitions>')
+        monkeypatch.setattr(
+            cf, "write_case",
+            lambda *a, **k: orig(*a, **dict(k, extra_xml=extra)))
+    got = _run(tmp_path, case, pres, "lanes")
+    monkeypatch.setenv("AQ_WALK_BLOCKS", "300")
+    want = _run(tmp_path, case, pres, "one")
+    for k in want:
+        np.testing.assert_array_equal(got[k], want[k], err_msg=k)
