@@ -74,10 +74,6 @@ inline size_t aq_owner_list_cap(size_t cells, size_t N)
 // particle within the support of a wall element, listed by the fused walk).
 #define AQ_CL_NNCELLS 514u
 #define AQ_CL_WORDS 1024u  // size of the n_heads buffer in words
-// Hand-out counters of the walks launched on the side stream beside the
-// fused walk (8 counters, 32 words apart, from this word on); the walks of
-// the main stream use the counters from word 32.
-#define AQ_CL_SIDE 544u
 struct CellArgs {
     const uint32_t* icell;
     const uint32_t* ihoc;
@@ -95,9 +91,8 @@ struct CellArgs {
     const uint32_t* wcells = nullptr;  // the wet owner cells
     const uint32_t* nlist = nullptr;   // the near cells (fused walk)
     const uint32_t* blist = nullptr;   // every non-empty cell, blocked order
-    // word of the n_heads buffer where the walk's hand-out counters start
-    // (0: word 32, the main stream's)
-    uint32_t next_off = 0;
+    // the walk runs on the side stream, beside the fused walk
+    uint32_t side = 0;
 };
 
 // Optional aids of the per-particle walk kernels, supplied by the runtime:

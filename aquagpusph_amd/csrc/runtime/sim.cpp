@@ -689,7 +689,7 @@ CellArgs Sim::cell_args()
                          ? clist.nlist
                          : nullptr,
                      (clist.blocked && clist.kinds) ? clist.bcells : nullptr,
-                     in_side ? AQ_CL_SIDE : 0u };
+                     in_side ? 1u : 0u };
 }
 
 void Sim::join_side(hipStream_t s)

@@ -30,6 +30,7 @@
 
 #include "aq_device.hpp"
 #include "aq_internal.hpp"
+#include "coop_device.hpp"
 #include "walk_device.hpp"
 
 namespace aq {
@@ -758,9 +759,12 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
 //   pol.owner(i, im_i)  the particles that run the kernel (the reference
 //                       kernel's early exits)
 //   Pol::State          per-particle accumulators
-//   pol.init(i, r_i, st), pol.pair<NRQ>(i, j, r_i, st), pol.finish(i, st)
-//                       (NRQ: q by div_nr, see qof)
-// pair() is called for the accepted candidates of each particle in the
+//   pol.init(i, r_i, st), pol.finish(i, st)
+//   pol.load(j)         a candidate's fields (Pol::Cand)
+//   pol.use<NRQ>(i, j, cand, r_i, st)
+//                       its terms added to the accumulators (NRQ: q by
+//                       div_nr, see qof)
+// use() is called for the accepted candidates of each particle in the
 // reference walk order, so every sum is bit-identical to the per-particle
 // kernel of sph.hip.
 // ---------------------------------------------------------------------------
@@ -773,9 +777,7 @@ template <bool NRQ> __device__ __forceinline__ float qof(float s, float H)
     else return sqrtf(s) / H;
 }
 
-// Candidate fields loaded ahead of their use (NB > 1): the policy's
-// Cand load(j) and use<NRQ>(i, j, cand, r_i, st), which together are its
-// pair<NRQ>(i, j, r_i, st).
+// A policy as ring_walk's batched pair: fields loaded ahead of their use.
 template <class Pol, bool NRQ> struct BatchPair {
     const Pol& pol;
     uint32_t i;
@@ -792,46 +794,29 @@ template <class Pol, bool NRQ> struct BatchPair {
     }
 };
 
-// Pol::STATIC_CELLS when the policy declares it (else false): static
-// hand-out of the listed cells in cell_kernel_k
-template <class P, class = void> struct StaticCells : std::false_type {};
-template <class P>
-struct StaticCells<P, std::void_t<decltype(P::STATIC_CELLS)>>
-    : std::integral_constant<bool, P::STATIC_CELLS> {};
-
-// PER: a periodic box; the policy's pair_p<NRQ>(i, j, shift, r_i, st) gets
-// the shift of j's neighbour cell.  NB > 1: batched consume (ring_walk).
-// olist: walk the cells it lists ((first particle, cell, cell_end)
-// triplets, counted in n_heads[count_word]: the owner-cell lists, the
-// near-cell list) instead of every non-empty cell.
-template <int D, int SEGW, class Pol, bool PER = false, int NB = 1>
+// Batched consume (ring_walk, NB candidates).  olist: walk the cells it lists
+// ((first particle, cell, cell_end) triplets, counted in
+// n_heads[count_word]) instead of every non-empty cell.
+template <int D, int SEGW, class Pol, int NB>
 __global__ void __launch_bounds__(64 * WC_WAVES)
     cell_kernel_k(Pol pol, const int* __restrict__ imove,
                   const float* __restrict__ r, WalkArgs w, float smax,
                   int nrq, const uint32_t* __restrict__ olist,
                   uint32_t count_word)
 {
-    __shared__ WaveLds<SEGW, PER> lds[WC_WAVES];
+    __shared__ WaveLds<SEGW, false> lds[WC_WAVES];
     const int lane = threadIdx.x & 63;
-    WaveLds<SEGW, PER>& L = lds[threadIdx.x >> 6];
+    WaveLds<SEGW, false>& L = lds[threadIdx.x >> 6];
     if (w.status && (*w.status & 1u)) return;
     const uint32_t n_heads =
         olist ? uni(w.n_heads[count_word]) : uni(*w.n_heads);
-    uint32_t range = blockIdx.x % w.ranges;
-    // static hand-out of a policy's listed cells (wave v takes v, v + W,
-    // ...; no atomic per cell)
-    const bool stat = StaticCells<Pol>::value && olist != nullptr;
+    // static hand-out: wavefront v takes the cells v, v + W, ...  (One
+    // counter per XCD costs an atomic per cell on 8 cache lines, some 16 ns
+    // each: 217 against 84 us for BI Interactions over the 66 k cells of 64
+    // sloshing tanks.)
     const uint32_t nwv = gridDim.x * WC_WAVES;
-    uint32_t hs = blockIdx.x * WC_WAVES + (threadIdx.x >> 6);
-    while (true) {
-        uint32_t hk;
-        if (stat) {
-            hk = hs;
-            hs += nwv;
-        } else {
-            hk = next_cell(w, n_heads, lane, range);
-        }
-        if (hk >= n_heads) break;
+    for (uint32_t hk = blockIdx.x * WC_WAVES + (threadIdx.x >> 6);
+         hk < n_heads; hk += nwv) {
         uint32_t cstart, c_i, ce;
         if (olist) {
             // (first particle, cell, cell_end) triplets: one round trip
@@ -852,7 +837,7 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
             const bool act = (i < cend) && pol.owner(i, imove[i]);
             if (__ballot(act) == 0) continue;
             if (!table) {
-                total = neighbour_table<D, PER>(
+                total = neighbour_table<D, false>(
                     w, c_i, L, lane,
                     Pol::KIND ? AQ_CELL_ELEM : AQ_CELL_FLUID);
                 table = true;
@@ -866,43 +851,16 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
             bool unused = false;
             f3 bmin, bmax;
             wave_box<D>(r_i, act, bmin, bmax);
-            auto call = [&](auto nrqc, uint32_t j, uint32_t kl) {
-                constexpr bool NRQ = decltype(nrqc)::value;
-                if constexpr (PER) {
-                    const float4 sh = L.shift[kl];
-                    pol.template pair_p<NRQ>(i, j, f3{ sh.x, sh.y, sh.z },
-                                             r_i, st);
-                } else {
-                    pol.template pair<NRQ>(i, j, r_i, st);
-                }
-            };
-            if constexpr (NB > 1) {
-                if (nrq)
-                    ring_walk<D, SEGW, NB>(
-                        L, lane, total, r_i, act, bmin, bmax, smax, r, imove,
-                        Pol::KIND, false, unused,
-                        BatchPair<Pol, true>{ pol, i, r_i, st }, w.per);
-                else
-                    ring_walk<D, SEGW, NB>(
-                        L, lane, total, r_i, act, bmin, bmax, smax, r, imove,
-                        Pol::KIND, false, unused,
-                        BatchPair<Pol, false>{ pol, i, r_i, st }, w.per);
-            } else if (nrq)
-                ring_walk<D, SEGW>(
+            if (nrq)
+                ring_walk<D, SEGW, NB>(
                     L, lane, total, r_i, act, bmin, bmax, smax, r, imove,
                     Pol::KIND, false, unused,
-                    [&](uint32_t j, uint32_t kl) {
-                        call(std::true_type{}, j, kl);
-                    },
-                    w.per);
+                    BatchPair<Pol, true>{ pol, i, r_i, st }, w.per);
             else
-                ring_walk<D, SEGW>(
+                ring_walk<D, SEGW, NB>(
                     L, lane, total, r_i, act, bmin, bmax, smax, r, imove,
                     Pol::KIND, false, unused,
-                    [&](uint32_t j, uint32_t kl) {
-                        call(std::false_type{}, j, kl);
-                    },
-                    w.per);
+                    BatchPair<Pol, false>{ pol, i, r_i, st }, w.per);
             if (act) pol.finish(i, st);
             __builtin_amdgcn_wave_barrier();
         }
@@ -910,262 +868,43 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
 }
 
 // ---------------------------------------------------------------------------
-// Cooperative cell kernel: Q lanes per owner.
+// Group kernel: Q lanes per owner (coop_device.hpp).
 //
 // A wall cell holds few owners (the 16 elements of a 3D wall plane in a cell
-// of side 2h at h = 2 dr), so a wavefront with one owner per lane leaves
-// most lanes idle, and the few wet wall cells (about a fifth) each form a
-// long chain of candidate tests and pair terms.  Here a pass takes up to
-// OW = 64 / Q owners of the cell and gives each Q lanes (lane q OW + o
-// serves owner o):
-//   test     every chunk of 64 candidates is staged as in ring_walk; lane
-//            (q, o) tests the q-th 64/Q of the chunk's survivors against
-//            owner o, and the Q pieces are assembled into the owner's
-//            accept bits, which all Q lanes hold;
-//   consume  in each round the Q lanes of an owner take its next Q accepted
-//            candidates, lane q evaluates the q-th one's term (Pol::term, a
-//            pure function of the owner and the candidate), the terms go
-//            through LDS and lane 0 of the owner adds them to the
-//            accumulator in candidate order (Pol::add).
-// Every owner's accumulator thus takes the terms of the one-lane walk in the
-// same order: the sums are bit-identical.
+// of side 2h at h = 2 dr), and a launch over the wall cells, or over the
+// cells of a small case, has too few of them to hide the latency of each
+// owner's chain of pair terms, so every owner gets Q lanes, and a listed
+// cell is cut into S groups of 64 / Q owners handed out to different
+// wavefronts: item k is group k % S of entry k / S, wavefront v takes the
+// items v, v + W, ... (no atomic per item).  The policy splits its pair
+// into load(j) (the candidate's fields), term<NRQ>(i, j, cand, r_i, st) (a
+// pure function of the owner and the candidate) and add_group<Q>(st, term),
+// which adds the terms of the group's lanes in lane order on all of them:
+// every owner's sums take the terms of the one-lane walk in the same order.
+// PER: the candidate's position is moved to its periodic image first.
+// olist as in cell_kernel_k, its count in n_heads[count_word].
 // ---------------------------------------------------------------------------
-// B: candidates per lane and round (Q B per owner), whose loads are issued
-// together; tsl holds B x 64 terms.
-template <int D, int SEGW, int Q, int B, class Term, class LoadFn,
-          class TermFn, class AddFn>
-__device__ __forceinline__ void coop_walk(WaveLds<SEGW, false>& L,
-                                          Term* tsl, int lane,
-                                          uint32_t total, const f3& r_i,
-                                          bool act, const f3& bmin,
-                                          const f3& bmax, float smax,
-                                          const float* __restrict__ r,
-                                          const int* __restrict__ imove,
-                                          int kind, LoadFn load, TermFn term,
-                                          AddFn add)
-{
-    static_assert(Q == 1 || Q == 2 || Q == 4, "lanes per owner");
-    static_assert(B >= 1 && B <= 4, "candidates per lane and round");
-    constexpr int OW = 64 / Q;   // owners per pass
-    constexpr int TPL = 64 / Q;  // survivors tested per lane and chunk
-    constexpr uint32_t SEG = SEGW * 32;
-    constexpr uint32_t RING = 2 * SEGW;
-    const int q = lane / OW, o = lane % OW;
-    const uint32_t nsegs = (total + SEG - 1) / SEG;
-    const uint32_t nwords = (total + 31) >> 5;
-    const uint32_t* bits = &L.bits[0][0][0];
-    const uint32_t* cand = &L.cand[0][0];
-    int kl = 0;
-    uint32_t nw = 0, bw = 0, tested = 0;
-    auto advance = [&]() {
-        const uint32_t tw = min(tested * SEGW, nwords);
-        while (bw == 0 && nw < tw) {
-            bw = bits[(nw % RING) * 64 + lane];
-            nw++;
-        }
-    };
-    auto go = [&]() {
-        advance();
-        if (tested < nsegs &&
-            (tested < 2 ||
-             __ballot(bw != 0 && nw <= (tested - 1) * SEGW) == 0))
-            return false;
-        return __ballot(bw != 0) != 0;
-    };
-    while (true) {
-        for (bool more = go(); more; more = go()) {
-            // one round: the next Q B accepted candidates of every owner
-            // (the Q lanes of an owner hold the same bits and step alike);
-            // lane q takes the candidates k = q + Q b
-            uint32_t myj[B];
-            bool mine[B];
-#pragma unroll
-            for (int b = 0; b < B; b++) {
-                myj[b] = 0;
-                mine[b] = false;
-            }
-            int n = 0;
-#pragma unroll
-            for (int k = 0; k < Q * B; k++) {
-                if (bw == 0) advance();
-                if (bw != 0) {
-                    const uint32_t b = __builtin_clz(bw);
-                    bw ^= 0x80000000u >> b;
-                    const uint32_t jj = cand[((nw - 1) % RING) * 32 + b];
-                    if (k % Q == q) {
-                        myj[k / Q] = jj;
-                        mine[k / Q] = true;
-                    }
-                    n = k + 1;
-                }
-            }
-            decltype(load(0u)) cd[B];
-#pragma unroll
-            for (int b = 0; b < B; b++)
-                if (mine[b]) cd[b] = load(myj[b]);
-            if constexpr (Q == 1 && B == 1) {
-                if (mine[0]) add(term(myj[0], cd[0]));
-            } else {
-#pragma unroll
-                for (int b = 0; b < B; b++) {
-                    Term t{};
-                    if (mine[b]) t = term(myj[b], cd[b]);
-                    tsl[b * 64 + lane] = t;
-                }
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_s_waitcnt(0);
-                if (q == 0) {
-#pragma unroll
-                    for (int k = 0; k < Q * B; k++)
-                        if (k < n) add(tsl[(k / Q) * 64 + (k % Q) * OW + o]);
-                }
-                __builtin_amdgcn_wave_barrier();
-            }
-        }
-        if (tested >= nsegs) break;  // and no lane has a candidate left
-        // refill the oldest slot: the segment's candidate loads are issued
-        // together, then its chunks of 64 are tested
-        const uint32_t seg = tested * SEG;
-        const uint32_t nseg = min(SEG, total - seg);
-        const int slot = tested & 1;
-        constexpr uint32_t NCH = SEG / 64;
-        uint32_t pj[NCH];
-        f3 prj[NCH];
-        int pim[NCH];
-#pragma unroll
-        for (uint32_t ch = 0; ch < NCH; ch++) {
-            pj[ch] = 0;
-            const uint32_t t = seg + ch * 64 + lane;
-            if (ch * 64 + lane < nseg) {
-                while (t >= L.cum[kl + 1]) kl++;
-                pj[ch] = L.start[kl] + (t - L.cum[kl]);
-            }
-        }
-#pragma unroll
-        for (uint32_t ch = 0; ch < NCH; ch++) {
-            prj[ch] = f3{ 0.f, 0.f, 0.f };
-            pim[ch] = 0;
-            if (ch * 64 + lane < nseg) {
-                prj[ch] = ldv_o<D>(r, pj[ch]);
-                pim[ch] = ldi_o(imove, pj[ch]);
-            }
-        }
-#pragma unroll
-        for (uint32_t ch = 0; ch < NCH; ch++) {
-            const uint32_t cb = ch * 64;
-            if (cb >= nseg) break;
-            float4 st = make_float4(0.f, 0.f, 0.f, 0.f);
-            bool take = false;
-            const uint32_t j = pj[ch];
-            if (cb + lane < nseg) {
-                const f3 rj = prj[ch];
-                const int im_j = pim[ch];
-                take = kind ? (im_j == -3) : (im_j == 1);
-                if (take) {
-                    const float dx =
-                        fmaxf(fmaxf(bmin.x - rj.x, rj.x - bmax.x), 0.f);
-                    const float dy =
-                        fmaxf(fmaxf(bmin.y - rj.y, rj.y - bmax.y), 0.f);
-                    float d2 = dx * dx;
-                    d2 = d2 + dy * dy;
-                    if constexpr (D == 3) {
-                        const float dz =
-                            fmaxf(fmaxf(bmin.z - rj.z, rj.z - bmax.z), 0.f);
-                        d2 = d2 + dz * dz;
-                    }
-                    take = !(d2 > smax);
-                }
-                st = make_float4(rj.x, rj.y, rj.z, 0.f);
-            }
-            const uint64_t tm = __ballot(take);
-            const uint32_t cnt = (uint32_t)__popcll(tm);
-            uint32_t lo = 0, hi = 0;
-            if (cnt != 0) {
-                // compact the survivors into stage[0 .. cnt), in order
-                const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
-                    (uint32_t)(tm >> 32),
-                    __builtin_amdgcn_mbcnt_lo((uint32_t)tm, 0u));
-                if (take) {
-                    L.stage[rank] = st;
-                    L.cand[slot][cb + rank] = j;
-                }
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_s_waitcnt(0);
-                // lane (q, o): survivors q TPL .. q TPL + TPL - 1
-                const uint32_t k0 = (uint32_t)(q * TPL);
-                const uint32_t kn =
-                    cnt > k0 ? min(cnt - k0, (uint32_t)TPL) : 0u;
-                uint64_t piece = 0;
-                for (uint32_t k = 0; k < kn; k++) {
-                    const float4 c = L.stage[k0 + k];
-                    const f3 r_ij = sub<D>(f3{ c.x, c.y, c.z }, r_i);
-                    const float s = dot<D>(r_ij, r_ij);
-                    piece = (piece << 1) | (!(s > smax) ? 1u : 0u);
-                }
-                if (kn == 0u || !act) piece = 0;
-                else if (kn < (uint32_t)TPL) piece <<= (uint32_t)TPL - kn;
-                // the owner's accept bits of the whole chunk, MSB first
-                uint64_t mask = 0;
-#pragma unroll
-                for (int qq = 0; qq < Q; qq++) {
-                    const uint64_t pc =
-                        (Q == 1) ? piece
-                                 : (uint64_t)(uint32_t)__shfl(
-                                       (int)(uint32_t)piece, qq * OW + o);
-                    mask |= pc << (64 - TPL * (qq + 1));
-                }
-                lo = (uint32_t)(mask >> 32);
-                hi = (uint32_t)mask;
-            }
-            L.bits[slot][cb >> 5][lane] = lo;
-            if (nseg - cb > 32) L.bits[slot][(cb >> 5) + 1][lane] = hi;
-            __builtin_amdgcn_wave_barrier();
-        }
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_s_waitcnt(0);
-        tested++;
-    }
-    __builtin_amdgcn_wave_barrier();
-}
-
-// Owners of each listed cell in passes of up to 64 / Q; the policy splits
-// its pair into load(j) (the candidate's fields), term<NRQ>(i, j, cand,
-// r_i, st) (pure) and add(st, term), applied in candidate order.  olist as
-// in cell_kernel_k, its count in n_heads[count_word].
-template <int D, int SEGW, int Q, class Pol>
+template <int D, int Q, class Pol, bool PER>
 __global__ void __launch_bounds__(64 * WC_WAVES)
-    cell_coop_k(Pol pol, const int* __restrict__ imove,
-                const float* __restrict__ r, WalkArgs w, float smax, int nrq,
-                const uint32_t* __restrict__ olist, uint32_t count_word)
+    cell_group_k(Pol pol, const int* __restrict__ imove,
+                 const float* __restrict__ r, WalkArgs w, float smax, int nrq,
+                 const uint32_t* __restrict__ olist, uint32_t count_word,
+                 uint32_t S)
 {
     constexpr int OW = 64 / Q;
     using Term = typename Pol::Term;
-    constexpr int B = Pol::COOP_B;
-    __shared__ WaveLds<SEGW, false> lds[WC_WAVES];
-    __shared__ uint32_t owns[WC_WAVES][OW];
-    __shared__ Term tsl[WC_WAVES][B * 64];
+    __shared__ CoopLds<Q, 1, PER> lds[WC_WAVES];
     const int lane = threadIdx.x & 63;
     const int wv = threadIdx.x >> 6;
-    const int q = lane / OW, o = lane % OW;
-    WaveLds<SEGW, false>& L = lds[wv];
+    const int q = lane & (Q - 1), o = lane / Q;
+    CoopLds<Q, 1, PER>& L = lds[wv];
     if (w.status && (*w.status & 1u)) return;
-    const uint32_t n_heads =
-        olist ? uni(w.n_heads[count_word]) : uni(*w.n_heads);
-    uint32_t range = blockIdx.x % w.ranges;
-    // static hand-out (Pol::STATIC_CELLS): wave v takes the cells
-    // v, v + W, v + 2W, ... (no atomic per cell), for lists whose cells cost
-    // alike
+    const uint32_t n_items =
+        (olist ? uni(w.n_heads[count_word]) : uni(*w.n_heads)) * S;
     const uint32_t nwv = gridDim.x * WC_WAVES;
-    uint32_t hs = blockIdx.x * WC_WAVES + (uint32_t)wv;
-    while (true) {
-        uint32_t hk;
-        if (Pol::STATIC_CELLS) {
-            hk = hs;
-            hs += nwv;
-        } else {
-            hk = next_cell(w, n_heads, lane, range);
-        }
-        if (hk >= n_heads) break;
+    for (uint32_t item = blockIdx.x * WC_WAVES + (uint32_t)wv; item < n_items;
+         item += nwv) {
+        const uint32_t hk = item / S;
         uint32_t cstart, c_i, ce;
         if (olist) {
             cstart = uni(olist[3 * hk]);
@@ -1178,44 +917,15 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
         }
         const uint32_t cend = ce & AQ_CELL_END;
         if (w.flagged && Pol::OWNERS && !(ce & Pol::OWNERS)) continue;
-        bool table = false;
-        uint32_t total = 0;
-        uint32_t pos = cstart;  // scan cursor (uniform)
-        while (pos < cend) {
-            // collect up to OW owners
-            uint32_t nf = 0;
-            while (nf < (uint32_t)OW && pos < cend) {
-                const uint32_t ii = pos + (uint32_t)lane;
-                const bool own = ii < cend && pol.owner(ii, imove[ii]);
-                const uint64_t bm = __ballot(own);
-                const uint32_t c = (uint32_t)__popcll(bm);
-                const uint32_t room = (uint32_t)OW - nf;
-                const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
-                    (uint32_t)(bm >> 32),
-                    __builtin_amdgcn_mbcnt_lo((uint32_t)bm, 0u));
-                if (own && rank < room) owns[wv][nf + rank] = ii;
-                if (c <= room) {
-                    nf += c;
-                    pos += 64;
-                } else {
-                    // resume at the first owner not taken
-                    uint64_t m = bm;
-                    for (uint32_t k = 0; k < room; k++) m &= m - 1ull;
-                    pos += (uint32_t)__builtin_ctzll(m);
-                    nf = OW;
-                }
-            }
+        for (uint32_t lo = (item % S) * OW;; lo += S * OW) {
+            const uint32_t nf = group_owners<Q>(
+                L, lane, cstart, cend, lo, imove,
+                [&](uint32_t ii, int im) { return pol.owner(ii, im); });
             if (nf == 0) break;
-            if (!table) {
-                total = neighbour_table<D, false>(
-                    w, c_i, L, lane,
-                    Pol::KIND ? AQ_CELL_ELEM : AQ_CELL_FLUID);
-                table = true;
-            }
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_s_waitcnt(0);
+            const uint32_t total = neighbour_table<D, PER>(
+                w, c_i, L, lane, Pol::KIND ? AQ_CELL_ELEM : AQ_CELL_FLUID);
             const bool act = (uint32_t)o < nf;
-            const uint32_t i = act ? owns[wv][o] : 0u;
+            const uint32_t i = act ? L.owns[o] : cstart;
             typename Pol::State st{};
             f3 r_i = { 0.f, 0.f, 0.f };
             if (act) {
@@ -1224,55 +934,54 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
             }
             f3 bmin, bmax;
             wave_box<D>(r_i, act, bmin, bmax);
-            auto add = [&](const Term& t) { pol.add(st, t); };
-            auto load = [&](uint32_t j) { return pol.load(j); };
-            using Cand = typename Pol::Cand;
-            if (nrq)
-                coop_walk<D, SEGW, Q, B>(
-                    L, &tsl[wv][0], lane, total, r_i, act, bmin, bmax, smax,
-                    r, imove, Pol::KIND, load,
-                    [&](uint32_t j, const Cand& c) {
-                        return pol.template term<true>(i, j, c, r_i, st);
-                    },
-                    add);
-            else
-                coop_walk<D, SEGW, Q, B>(
-                    L, &tsl[wv][0], lane, total, r_i, act, bmin, bmax, smax,
-                    r, imove, Pol::KIND, load,
-                    [&](uint32_t j, const Cand& c) {
-                        return pol.template term<false>(i, j, c, r_i, st);
-                    },
-                    add);
+            auto round = [&](uint32_t n, const uint32_t (&cw)[1]) {
+                Term t = Pol::none();
+                if ((uint32_t)q < n) {
+                    const uint32_t j = PER ? cw[0] & PER_J_MASK : cw[0];
+                    auto c = pol.load(j);
+                    if constexpr (PER) {
+                        const float4 sh = L.shift[cw[0] >> PER_KL_SHIFT];
+                        c.r = per_shift<D>(c.r, f3{ sh.x, sh.y, sh.z },
+                                           w.per);
+                    }
+                    t = nrq ? pol.template term<true>(i, j, c, r_i, st)
+                            : pol.template term<false>(i, j, c, r_i, st);
+                }
+                pol.template add_group<Q>(st, t);
+            };
+            bool unused = false;
+            coop_list_walk<D, Q, 1, false, PER>(
+                L, lane, total, r_i, act, bmin, bmax, smax, r, imove,
+                Pol::KIND, false, unused, w.per, round);
             if (act && q == 0) pol.finish(i, st);
-            __builtin_amdgcn_wave_barrier();
+            lds_order();
+            if (nf < (uint32_t)OW) break;
         }
     }
 }
 
+// a += the values v of the group's lanes, in lane order
+template <int Q> __device__ __forceinline__ void add_lanes(float& a, float v)
+{
+    each_lane<Q>(v, [&](float x) { a += x; });
+}
+
 // The element-owner policies below split each pair into load(j) (the
 // candidate's fields), term<NRQ>(i, j, cand, r_i, st) (a pure function of
-// the owner's state and the candidate) and add(st, term); pair and use
-// apply them in that order, so every walk form adds the same terms.
-#define AQ_POL_PAIR_FROM_TERM                                                  \
+// the owner's state and the candidate) and add(st, term); use applies them
+// in that order, so every walk form adds the same terms.
+#define AQ_POL_USE_FROM_TERM                                                  \
     template <bool NRQ>                                                        \
     __device__ void use(uint32_t i, uint32_t j, const Cand& c,                 \
                         const f3& r_i, State& st) const                        \
     {                                                                          \
         add(st, term<NRQ>(i, j, c, r_i, st));                                  \
-    }                                                                          \
-    template <bool NRQ>                                                        \
-    __device__ void pair(uint32_t i, uint32_t j, const f3& r_i, State& st)     \
-        const                                                                  \
-    {                                                                          \
-        use<NRQ>(i, j, load(j), r_i, st);                                      \
     }
 
 // cfd/Boundary/BI/Shepard.cl:61-150 (compute) for the non-fluid particles
 // (skip_fluid) or all of them
 template <int D> struct PolBiShepard {
     static constexpr int BATCH = 4;  // candidates loaded together
-    static constexpr bool STATIC_CELLS = true;  // coop walk hand-out
-    static constexpr int COOP_B = 1;  // per lane and round (coop walk)
     static constexpr int KIND = 1;
     static constexpr uint32_t OWNERS = 0;  // elements, sensors, ...
     const int* imove;
@@ -1339,7 +1048,25 @@ template <int D> struct PolBiShepard {
             st.acc -= 0.5f;
         }
     }
-    AQ_POL_PAIR_FROM_TERM
+    __device__ static Term none() { return Term{ 0.f, 2u }; }
+    template <int Q>
+    __device__ void add_group(State& st, const Term& t) const
+    {
+        // (v is 0 where kind != 0, and acc is never -0)
+        if (__ballot(t.kind == 1u) == 0) {
+            add_lanes<Q>(st.acc, t.v);
+            return;
+        }
+        // the half angle in its place in the order
+        float v[Q], k[Q];
+        int e = 0;
+        each_lane<Q>(t.v, [&](float x) { v[e++] = x; });
+        e = 0;
+        each_lane<Q>((float)t.kind, [&](float x) { k[e++] = x; });
+#pragma unroll
+        for (int l = 0; l < Q; l++) add(st, Term{ v[l], (uint32_t)k[l] });
+    }
+    AQ_POL_USE_FROM_TERM
     __device__ void finish(uint32_t i, const State& st) const
     {
         shepard[i] = st.acc;
@@ -1350,8 +1077,6 @@ template <int D> struct PolBiShepard {
 // cfd/Boundary/BI/LapU.cl:58-123 (freeslip)
 template <int D> struct PolBiLapU {
     static constexpr int BATCH = 4;  // candidates loaded together
-    static constexpr bool STATIC_CELLS = true;  // coop walk hand-out
-    static constexpr int COOP_B = 2;  // per lane and round (coop walk)
     static constexpr int KIND = 0;
     static constexpr uint32_t OWNERS = AQ_CELL_ELEM;
     const float *r_, *u, *rho, *m;
@@ -1412,7 +1137,15 @@ template <int D> struct PolBiLapU {
         st.lu.y += t.v.y;
         if constexpr (D == 3) st.lu.z += t.v.z;
     }
-    AQ_POL_PAIR_FROM_TERM
+    __device__ static Term none() { return Term{ f3{ 0.f, 0.f, 0.f }, 0u }; }
+    template <int Q>
+    __device__ void add_group(State& st, const Term& t) const
+    {
+        add_lanes<Q>(st.lu.x, t.v.x);
+        add_lanes<Q>(st.lu.y, t.v.y);
+        if constexpr (D == 3) add_lanes<Q>(st.lu.z, t.v.z);
+    }
+    AQ_POL_USE_FROM_TERM
     __device__ void finish(uint32_t i, const State& st) const
     {
         stxyz<D>(lap_u, i, st.lu);
@@ -1422,8 +1155,6 @@ template <int D> struct PolBiLapU {
 // cfd/Boundary/BI/Interpolation.cl:54-107
 template <int D> struct PolBiInterp {
     static constexpr int BATCH = 4;  // candidates loaded together
-    static constexpr bool STATIC_CELLS = true;  // coop walk hand-out
-    static constexpr int COOP_B = 2;  // per lane and round (coop walk)
     static constexpr int KIND = 0;
     static constexpr uint32_t OWNERS = AQ_CELL_ELEM;
     const float *r_, *m, *rho, *grad_p;
@@ -1464,20 +1195,23 @@ template <int D> struct PolBiInterp {
         return (c.p - dot<D>(st.gp_i, r_ij)) * w_ij;
     }
     __device__ void add(State& st, const Term& t) const { st.acc += t; }
-    AQ_POL_PAIR_FROM_TERM
+    __device__ static Term none() { return 0.f; }
+    template <int Q>
+    __device__ void add_group(State& st, const Term& t) const
+    {
+        add_lanes<Q>(st.acc, t);
+    }
+    AQ_POL_USE_FROM_TERM
     __device__ void finish(uint32_t i, const State& st) const
     {
         p[i] = st.acc;
     }
 };
-#undef AQ_POL_PAIR_FROM_TERM
 
 // cfd/Boundary/BI/Interactions.cl:51-133, for the fluid particles with an
 // element inside the support (near flags of the fused walk) or all of them
 template <int D> struct PolBiInteractions {
     static constexpr int BATCH = 4;  // candidates loaded together
-    // the near cells cost about alike: static hand-out over the near list
-    static constexpr bool STATIC_CELLS = true;
     static constexpr int KIND = 1;
     static constexpr uint32_t OWNERS = AQ_CELL_FLUID;
     const float *r_, *normal, *u, *rho, *m, *p;
@@ -1509,27 +1243,37 @@ template <int D> struct PolBiInteractions {
         return Cand{ ldv_o<D>(r_, j), ldv_o<D>(normal, j), ldv_o<D>(u, j),
                      ldf_o(m, j), ldf_o(p, j) };
     }
+    struct Term {
+        f3 g;  // the rounded products of the axpy
+        float d;
+    };
     template <bool NRQ>
-    __device__ void pair(uint32_t i, uint32_t j, const f3& r_i,
-                         State& st) const
-    {
-        use<NRQ>(i, j, load(j), r_i, st);
-    }
-    template <bool NRQ>
-    __device__ void use(uint32_t, uint32_t, const Cand& c, const f3& r_i,
-                        State& st) const
+    __device__ Term term(uint32_t, uint32_t, const Cand& c, const f3& r_i,
+                         const State& st) const
     {
         const f3 r_ij = sub<D>(c.r, r_i);
         const float s = dot<D>(r_ij, r_ij);
         const float q = qof<NRQ>(s, H);
-        const f3 n_j = c.n;
-        const float area_j = c.area;
-        const float p_j = c.p;
         const f3 du = sub<D>(c.u, st.u_i);
-        const float w_ij = kernelW<D>(q) * CONW * area_j;
-        axpy<D>(st.gp, (st.p_i + p_j) / st.rho_i * w_ij, n_j);
-        st.dv += st.rho_i * dot<D>(du, n_j) * w_ij;
+        const float w_ij = kernelW<D>(q) * CONW * c.area;
+        return Term{ scl<D>((st.p_i + c.p) / st.rho_i * w_ij, c.n),
+                     st.rho_i * dot<D>(du, c.n) * w_ij };
     }
+    __device__ void add(State& st, const Term& t) const
+    {
+        st.gp = add3<D>(st.gp, t.g);
+        st.dv += t.d;
+    }
+    __device__ static Term none() { return Term{ f3{ 0.f, 0.f, 0.f }, 0.f }; }
+    template <int Q>
+    __device__ void add_group(State& st, const Term& t) const
+    {
+        add_lanes<Q>(st.gp.x, t.g.x);
+        add_lanes<Q>(st.gp.y, t.g.y);
+        if constexpr (D == 3) add_lanes<Q>(st.gp.z, t.g.z);
+        add_lanes<Q>(st.dv, t.d);
+    }
+    AQ_POL_USE_FROM_TERM
     __device__ void finish(uint32_t i, const State& st) const
     {
         stxyz<D>(grad_p, i, st.gp);
@@ -1537,13 +1281,15 @@ template <int D> struct PolBiInteractions {
     }
 };
 
+#undef AQ_POL_USE_FROM_TERM
+
 // ---- LES closure pair kernels (cfd/LES/GradU.cl, cfd/LES/Interactions.cl
 // of Presets/cfd/LES.xml; no counterpart in the reference) -------------------
 // The SPH velocity gradient of the fluid particles,
 //   G_i = sum_j m_j / rho_j (u_j - u_i) (x) F_ij r_ij,
 // grad_u[a n + b] = du_a / dx_b (row stride n = 2 in 2D, 4 in 3D), summed
-// in the walk order; pair_p: the same at a periodic image.  The non-fluid
-// particles' rows are cleared by the launcher.
+// in the walk order.  The non-fluid particles' rows are cleared by the
+// launcher.  (Group kernel only.)
 template <int D> struct PolLesGradU {
     static constexpr int KIND = 0;
     static constexpr uint32_t OWNERS = AQ_CELL_FLUID;
@@ -1551,7 +1297,6 @@ template <int D> struct PolLesGradU {
     const float *r_, *u, *rho, *m;
     float* grad_u;
     float H, CONF;
-    const float* per;
     struct State {
         f3 u_i;
         float G[D * D];
@@ -1563,37 +1308,48 @@ template <int D> struct PolLesGradU {
 #pragma unroll
         for (int k = 0; k < D * D; k++) st.G[k] = 0.f;
     }
-    __device__ void add(uint32_t j, const f3& r_j, const f3& r_i, float q,
-                        State& st) const
+    struct Cand {
+        f3 r, u;
+        float m, rho;
+    };
+    struct Term {
+        float g[D * D];
+    };
+    __device__ Cand load(uint32_t j) const
     {
-        const f3 r_ij = sub<D>(r_j, r_i);
-        const float w = kernelF<D>(q) * CONF * ldf_o(m, j) / ldf_o(rho, j);
-        const f3 du = sub<D>(ldv_o<D>(u, j), st.u_i);
+        return Cand{ ldv_o<D>(r_, j), ldv_o<D>(u, j), ldf_o(m, j),
+                     ldf_o(rho, j) };
+    }
+    template <bool NRQ>
+    __device__ Term term(uint32_t i, uint32_t j, const Cand& c,
+                         const f3& r_i, const State& st) const
+    {
+        Term t = none();
+        if (i == j) return t;
+        const f3 r_ij = sub<D>(c.r, r_i);
+        const float q = qof<NRQ>(dot<D>(r_ij, r_ij), H);
+        const float w = kernelF<D>(q) * CONF * c.m / c.rho;
+        const f3 du = sub<D>(c.u, st.u_i);
         const float dv[3] = { du.x, du.y, du.z };
         const float rv[3] = { r_ij.x, r_ij.y, r_ij.z };
 #pragma unroll
         for (int a = 0; a < D; a++)
 #pragma unroll
-            for (int b = 0; b < D; b++)
-                st.G[a * D + b] += dv[a] * (w * rv[b]);
+            for (int b = 0; b < D; b++) t.g[a * D + b] = dv[a] * (w * rv[b]);
+        return t;
     }
-    template <bool NRQ>
-    __device__ void pair(uint32_t i, uint32_t j, const f3& r_i,
-                         State& st) const
+    __device__ static Term none()
     {
-        if (i == j) return;
-        const f3 r_j = ldv_o<D>(r_, j);
-        const f3 r_ij = sub<D>(r_j, r_i);
-        add(j, r_j, r_i, qof<NRQ>(dot<D>(r_ij, r_ij), H), st);
+        Term t;
+#pragma unroll
+        for (int k = 0; k < D * D; k++) t.g[k] = 0.f;
+        return t;
     }
-    template <bool NRQ>
-    __device__ void pair_p(uint32_t i, uint32_t j, const f3& sh,
-                           const f3& r_i, State& st) const
+    template <int Q>
+    __device__ void add_group(State& st, const Term& t) const
     {
-        if (i == j) return;
-        const f3 r_j = per_shift<D>(ldv_o<D>(r_, j), sh, per);
-        const f3 r_ij = sub<D>(r_j, r_i);
-        add(j, r_j, r_i, qof<NRQ>(dot<D>(r_ij, r_ij), H), st);
+#pragma unroll
+        for (int k = 0; k < D * D; k++) add_lanes<Q>(st.G[k], t.g[k]);
     }
     __device__ void finish(uint32_t i, const State& st) const
     {
@@ -1620,7 +1376,6 @@ template <int D> struct PolLesInteractions {
     const float *r_, *u, *rho, *m, *nu_t;
     float* dudt;
     float H, CONF;
-    const float* per;
     struct State {
         f3 u_i, acc;
         float rho_i, mu_i;
@@ -1633,29 +1388,35 @@ template <int D> struct PolLesInteractions {
         st.mu_i = st.rho_i * nu_t[i];
         st.acc = f3{ 0.f, 0.f, 0.f };
     }
-    __device__ void add(uint32_t j, float q, State& st) const
+    struct Cand {
+        f3 r, u;
+        float m, rho, nu;
+    };
+    using Term = f3;
+    __device__ Cand load(uint32_t j) const
     {
-        const float rho_j = ldf_o(rho, j);
-        const float f = kernelF<D>(q) * CONF * ldf_o(m, j);
+        return Cand{ ldv_o<D>(r_, j), ldv_o<D>(u, j), ldf_o(m, j),
+                     ldf_o(rho, j), ldf_o(nu_t, j) };
+    }
+    template <bool NRQ>
+    __device__ Term term(uint32_t i, uint32_t j, const Cand& c,
+                         const f3& r_i, const State& st) const
+    {
+        if (i == j) return none();
+        const f3 r_ij = sub<D>(c.r, r_i);
+        const float q = qof<NRQ>(dot<D>(r_ij, r_ij), H);
+        const float f = kernelF<D>(q) * CONF * c.m;
         const float sc =
-            f * (st.mu_i + rho_j * ldf_o(nu_t, j)) / (st.rho_i * rho_j);
-        axpy<D>(st.acc, sc, sub<D>(ldv_o<D>(u, j), st.u_i));
+            f * (st.mu_i + c.rho * c.nu) / (st.rho_i * c.rho);
+        return scl<D>(sc, sub<D>(c.u, st.u_i));
     }
-    template <bool NRQ>
-    __device__ void pair(uint32_t i, uint32_t j, const f3& r_i,
-                         State& st) const
+    __device__ static Term none() { return f3{ 0.f, 0.f, 0.f }; }
+    template <int Q>
+    __device__ void add_group(State& st, const Term& t) const
     {
-        if (i == j) return;
-        const f3 r_ij = sub<D>(ldv_o<D>(r_, j), r_i);
-        add(j, qof<NRQ>(dot<D>(r_ij, r_ij), H), st);
-    }
-    template <bool NRQ>
-    __device__ void pair_p(uint32_t i, uint32_t j, const f3& sh,
-                           const f3& r_i, State& st) const
-    {
-        if (i == j) return;
-        const f3 r_ij = sub<D>(per_shift<D>(ldv_o<D>(r_, j), sh, per), r_i);
-        add(j, qof<NRQ>(dot<D>(r_ij, r_ij), H), st);
+        add_lanes<Q>(st.acc.x, t.x);
+        add_lanes<Q>(st.acc.y, t.y);
+        if constexpr (D == 3) add_lanes<Q>(st.acc.z, t.z);
     }
     __device__ void finish(uint32_t i, const State& st) const
     {
@@ -1763,7 +1524,7 @@ static unsigned reserved_grid(unsigned resident, unsigned reserve)
 static unsigned walk_grid(const void* ker, const CellArgs& c)
 {
     const unsigned res = resident_blocks(ker, 64 * WC_WAVES);
-    if (c.next_off != AQ_CL_SIDE) return res;
+    if (!c.side) return res;
     return std::min(res, std::max(1u, side_wgs_per_cu()) * cu_count());
 }
 
@@ -1885,50 +1646,68 @@ void launch_fluid_pass_cells(int dims, int shep, bool lapp,
 
 
 // ---- launchers of the generic cell kernels ---------------------------------
-template <int D, class Pol, bool PER = false, int NB = 1>
-static void launch_cells(const Pol& pol, const int32_t* imove, const float* r,
-                         const CellArgs& c, float smax, hipStream_t s,
-                         const float* per = nullptr,
-                         const uint32_t* olist = nullptr,
-                         uint32_t count_word = AQ_CL_NOCELLS)
-{
-    AQ_REQUIRE(c.N < (1u << 28), "cell-parallel walk: more than 2^28 particles");
-    uint32_t* next = const_cast<uint32_t*>(c.n_heads) +
-                     (c.next_off ? c.next_off : RSTRIDE);
-    hipLaunchKernelGGL(zero_u32_k, dim3(1), dim3(64), 0, s, next,
-                       (uint32_t*)nullptr);
-    WalkArgs w{ c.icell,   c.ihoc,   c.n_cells, c.cell_end, c.heads,
-                c.n_heads, next,     c.status,  c.N,        c.flagged,
-                walk_ranges(), per };
-    if (!olist && c.blist) {
-        // every non-empty cell, in blocked order (n_heads[0] of them)
-        olist = c.blist;
-        count_word = 0;
-    }
-    auto* ker = cell_kernel_k<D, 8, Pol, PER, NB>;
-    const unsigned nb = walk_grid((const void*)ker, c);
-    const int nrq = (pol.H >= 0x1p-40f && pol.H <= 0x1p40f) ? 1 : 0;
-    hipLaunchKernelGGL(ker, dim3(nb), dim3(64 * WC_WAVES), 0, s, pol, imove,
-                       r, w, smax, nrq, olist, count_word);
-}
-
-// The boundary-integral element kernels: batched consume; the kernels whose
-// owners are wall elements or other non-fluid particles (owner_cells) walk
-// the owner-cell list when the link-list built it.
-// Kernels whose owners are wall elements or other non-fluid particles
-// (owner_cells) run the cooperative walk over the owner-cell list when the
-// link-list built it (4 lanes per owner); the others, and all of them
-// without the list, the one-owner-per-lane walk with batched loads.
+// One owner per lane over every non-empty cell (in blocked order when the
+// link-list built it), batched loads.
 template <int D, class Pol>
 static void launch_bi_cells(const Pol& pol, const int32_t* imove,
                             const float* r, const CellArgs& c, float smax,
                             hipStream_t s)
 {
-    launch_cells<D, Pol, false, Pol::BATCH>(pol, imove, r, c, smax, s);
+    AQ_REQUIRE(c.N < (1u << 28), "cell-parallel walk: more than 2^28 particles");
+    WalkArgs w{ c.icell,   c.ihoc,   c.n_cells, c.cell_end, c.heads,
+                c.n_heads, nullptr,  c.status,  c.N,        c.flagged,
+                walk_ranges() };
+    auto* ker = cell_kernel_k<D, 8, Pol, Pol::BATCH>;
+    const unsigned nb = walk_grid((const void*)ker, c);
+    const int nrq = (pol.H >= 0x1p-40f && pol.H <= 0x1p40f) ? 1 : 0;
+    hipLaunchKernelGGL(ker, dim3(nb), dim3(64 * WC_WAVES), 0, s, pol, imove,
+                       r, w, smax, nrq, c.blist, 0u);
+}
+
+// The group kernel with `wide` ? 16 : 4 lanes per owner over `olist`
+// (nullptr: every non-empty cell, in blocked order when there is one);
+// `per_cell`: owners of a full entry.  Measured in us, 4 / 16 lanes:
+//   BI LapU          3D  29 k particles 46 / 25   394 k 52 / 34
+//                        1.2 M 57 / 62   4.5 M 113 / 126
+//                    2D  21 k 13 / 11   1.2 M (64 tanks) 23 / 28
+//   BI Interactions  3D  29 k 25 / 34   1.2 M 72 / 126   4.5 M 136 / 245
+//   LES grad u       3D  9 k 219 / 101   64 k 204 / 248   262 k 570 / 862
+// The elements are few and hold a fifth of their neighbours' particles each,
+// so 16 lanes pay as long as latency rules; fluid owners fill the chip much
+// earlier.  (Before, in us at 4.5 M / 1.2 M / 29 k: 4 lanes with the terms
+// through LDS and a full wait per segment, LapU 240 / 134 / 127,
+// Interpolation 200 / 119 / 113; one lane per owner, Interactions 132 / 75 /
+// 65; LES grad u at 262 k one lane 667.)
+template <int D, class Pol, bool PER = false>
+static void launch_groups(const Pol& pol, const int32_t* imove,
+                          const float* r, const CellArgs& c, float smax,
+                          hipStream_t s, bool wide, const uint32_t* olist,
+                          uint32_t count_word, uint32_t per_cell,
+                          const float* per = nullptr)
+{
+    AQ_REQUIRE(c.N < (1u << 28), "cell-parallel walk: more than 2^28 particles");
+    WalkArgs w{ c.icell,   c.ihoc,   c.n_cells, c.cell_end, c.heads,
+                c.n_heads, nullptr,  c.status,  c.N,        c.flagged,
+                walk_ranges(), per };
+    if (!olist && c.blist) {
+        olist = c.blist;
+        count_word = 0;
+    }
+    const int nrq = (pol.H >= 0x1p-40f && pol.H <= 0x1p40f) ? 1 : 0;
+    auto launch = [&](auto* ker, unsigned q) {
+        const unsigned nb = std::min(walk_grid((const void*)ker, c),
+                                     blocks_for((size_t)c.N * q * 2,
+                                                64 * WC_WAVES));
+        hipLaunchKernelGGL(ker, dim3(nb), dim3(64 * WC_WAVES), 0, s, pol,
+                           imove, r, w, smax, nrq, olist, count_word,
+                           std::max(1u, per_cell * q / 64u));
+    };
+    if (wide) launch(cell_group_k<D, 16, Pol, PER>, 16);
+    else launch(cell_group_k<D, 4, Pol, PER>, 4);
 }
 
 // list: 0 every non-empty cell (one owner per lane), 1 the owner cells,
-// 2 the wet owner cells (cooperative walk)
+// 2 the wet owner cells (group kernel)
 template <int D, class Pol>
 static void launch_bi_coop(const Pol& pol, const int32_t* imove,
                            const float* r, const CellArgs& c, float smax,
@@ -1938,24 +1717,13 @@ static void launch_bi_coop(const Pol& pol, const int32_t* imove,
                          : list == 1 ? c.ocells
                          : list == 2 ? c.wcells
                                      : nullptr;
-    if (!ol) {
+    if (!ol)
         launch_bi_cells<D>(pol, imove, r, c, smax, s);
-        return;
-    }
-    AQ_REQUIRE(c.N < (1u << 28), "cell-parallel walk: more than 2^28 particles");
-    uint32_t* next = const_cast<uint32_t*>(c.n_heads) +
-                     (c.next_off ? c.next_off : RSTRIDE);
-    hipLaunchKernelGGL(zero_u32_k, dim3(1), dim3(64), 0, s, next,
-                       (uint32_t*)nullptr);
-    WalkArgs w{ c.icell,   c.ihoc,   c.n_cells, c.cell_end, c.heads,
-                c.n_heads, next,     c.status,  c.N,        c.flagged,
-                walk_ranges(), nullptr };
-    auto* ker = cell_coop_k<D, 8, 4, Pol>;
-    const unsigned nb = walk_grid((const void*)ker, c);
-    const int nrq = (pol.H >= 0x1p-40f && pol.H <= 0x1p40f) ? 1 : 0;
-    hipLaunchKernelGGL(ker, dim3(nb), dim3(64 * WC_WAVES), 0, s, pol, imove,
-                       r, w, smax, nrq, ol,
-                       list == 1 ? AQ_CL_NOCELLS : AQ_CL_NWCELLS);
+    else
+        launch_groups<D>(pol, imove, r, c, smax, s,
+                         c.N <= (D == 2 ? 100000u : 600000u), ol,
+                         list == 1 ? AQ_CL_NOCELLS : AQ_CL_NWCELLS,
+                         AQ_OWNER_CHUNK);
 }
 
 // p = 0 for the wall elements (imove == -3): the value BI Interpolation
@@ -2029,19 +1797,37 @@ void launch_bi_interactions_cells(int dims, const int32_t* imove,
 {
     // with the near flags, only the cells the fused walk listed as near
     const uint32_t* ol = (near && c.flagged) ? c.nlist : nullptr;
-    if (dims == 2) {
-        PolBiInteractions<2> q{ r, normal, u, rho, m, p, grad_p, div_u,
-                                near, d.H, d.CONW };
-        launch_cells<2, PolBiInteractions<2>, false,
-                     PolBiInteractions<2>::BATCH>(q, imove, r, c, smax, s,
-                                                  nullptr, ol, AQ_CL_NNCELLS);
-    } else {
-        PolBiInteractions<3> q{ r, normal, u, rho, m, p, grad_p, div_u,
-                                near, d.H, d.CONW };
-        launch_cells<3, PolBiInteractions<3>, false,
-                     PolBiInteractions<3>::BATCH>(q, imove, r, c, smax, s,
-                                                  nullptr, ol, AQ_CL_NNCELLS);
-    }
+    auto go = [&](const auto& pol, auto dim) {
+        constexpr int D = decltype(dim)::value;
+        if (ol)
+            launch_groups<D>(pol, imove, r, c, smax, s, false, ol,
+                             AQ_CL_NNCELLS, D == 2 ? 16 : 64);
+        else
+            launch_bi_cells<D>(pol, imove, r, c, smax, s);
+    };
+    if (dims == 2)
+        go(PolBiInteractions<2>{ r, normal, u, rho, m, p, grad_p, div_u, near,
+                                 d.H, d.CONW },
+           std::integral_constant<int, 2>{});
+    else
+        go(PolBiInteractions<3>{ r, normal, u, rho, m, p, grad_p, div_u, near,
+                                 d.H, d.CONW },
+           std::integral_constant<int, 3>{});
+}
+
+// LES kernels: groups over every cell
+template <int D, class Pol>
+static void launch_les(const Pol& pol, const int32_t* imove, const float* r,
+                       const CellArgs& c, float smax, const float* per,
+                       hipStream_t s)
+{
+    const bool wide = c.N <= (D == 2 ? 16000u : 24000u);
+    const uint32_t full = D == 2 ? 16 : 64;
+    if (per)
+        launch_groups<D, Pol, true>(pol, imove, r, c, smax, s, wide, nullptr,
+                                    0, full, per);
+    else
+        launch_groups<D>(pol, imove, r, c, smax, s, wide, nullptr, 0, full);
 }
 
 void launch_les_gradu_cells(int dims, const int32_t* imove, const float* r,
@@ -2053,15 +1839,13 @@ void launch_les_gradu_cells(int dims, const int32_t* imove, const float* r,
     if (dims == 2) {
         hipLaunchKernelGGL(les_gradu_clear_k<2>, g, b, 0, s, imove, grad_u,
                            c.N);
-        PolLesGradU<2> p{ r, u, rho, m, grad_u, d.H, d.CONF, per };
-        if (per) launch_cells<2, PolLesGradU<2>, true>(p, imove, r, c, smax, s, per);
-        else launch_cells<2>(p, imove, r, c, smax, s);
+        PolLesGradU<2> p{ r, u, rho, m, grad_u, d.H, d.CONF };
+        launch_les<2>(p, imove, r, c, smax, per, s);
     } else {
         hipLaunchKernelGGL(les_gradu_clear_k<3>, g, b, 0, s, imove, grad_u,
                            c.N);
-        PolLesGradU<3> p{ r, u, rho, m, grad_u, d.H, d.CONF, per };
-        if (per) launch_cells<3, PolLesGradU<3>, true>(p, imove, r, c, smax, s, per);
-        else launch_cells<3>(p, imove, r, c, smax, s);
+        PolLesGradU<3> p{ r, u, rho, m, grad_u, d.H, d.CONF };
+        launch_les<3>(p, imove, r, c, smax, per, s);
     }
 }
 
@@ -2073,17 +1857,11 @@ void launch_les_interactions_cells(int dims, const int32_t* imove,
                                    const float* per, hipStream_t s)
 {
     if (dims == 2) {
-        PolLesInteractions<2> p{ r, u, rho, m, nu_t, dudt, d.H, d.CONF, per };
-        if (per)
-            launch_cells<2, PolLesInteractions<2>, true>(p, imove, r, c, smax,
-                                                         s, per);
-        else launch_cells<2>(p, imove, r, c, smax, s);
+        PolLesInteractions<2> p{ r, u, rho, m, nu_t, dudt, d.H, d.CONF };
+        launch_les<2>(p, imove, r, c, smax, per, s);
     } else {
-        PolLesInteractions<3> p{ r, u, rho, m, nu_t, dudt, d.H, d.CONF, per };
-        if (per)
-            launch_cells<3, PolLesInteractions<3>, true>(p, imove, r, c, smax,
-                                                         s, per);
-        else launch_cells<3>(p, imove, r, c, smax, s);
+        PolLesInteractions<3> p{ r, u, rho, m, nu_t, dudt, d.H, d.CONF };
+        launch_les<3>(p, imove, r, c, smax, per, s);
     }
 }
 

@@ -111,3 +111,46 @@ def test_lanes_per_particle_are_bit_identical(cuda, tmp_path, monkeypatch,
     want = _run(tmp_path, case, pres, "one")
     for k in want:
         np.testing.assert_array_equal(got[k], want[k], err_msg=k)
+
+
+# element kernels: 16 lanes per owner below 100 k (2D) / 600 k (3D)
+# particles, 4 above; wall edges and corners hold more than one group
+@pytest.mark.parametrize("dims,dr,hfac", [(2, 0.06, 2.0), (2, 0.011, 2.0),
+                                          (2, 0.00135, 2.0), (3, 0.05, 2.0),
+                                          (3, 0.031, 3.3), (3, 0.0061, 2.0)])
+def test_element_groups_match_one_lane_walks(cuda, tmp_path, monkeypatch,
+                                             dims, dr, hfac):
+    """The boundary-integral element kernels with 4 or 16 lanes per owner
+    over the owner, wet and near lists against one lane per owner over every
+    cell (AQ_BI_WALK=cells), bit for bit."""
+    from aquagpusph_amd import casefiles, cases
+    case = _stir(cases.dam_break(dims, dr, hfac=hfac), 11)
+    got = _run(tmp_path, case, casefiles.PBI_PRESETS, "groups", 2)
+    monkeypatch.setenv("AQ_BI_WALK", "cells")
+    want = _run(tmp_path, case, casefiles.PBI_PRESETS, "cells", 2)
+    for k in want:
+        np.testing.assert_array_equal(got[k], want[k], err_msg=k)
+
+
+@pytest.mark.parametrize("dims,n", [(2, 23), (2, 150), (3, 17), (3, 30)])
+def test_les_groups_match_oracle(cuda, tmp_path, dims, n):
+    """The LES gradient and viscous term (periodic box, Smagorinsky) with 16
+    and with 4 lanes per particle (2D above 16 k, 3D above 24 k particles)
+    against the oracle's float32 walk, bit for bit."""
+    from aquagpusph_amd import casefiles, cases
+    from aquagpusph_amd.sim import Simulation
+    from oracle import pipeline as op
+    case = _stir(cases.periodic_box(dims, n), 5)
+    sim = Simulation(casefiles.write_case(
+        case, str(tmp_path), load=False, presets=casefiles.PPER_PRESETS +
+        ("resources/Presets/cfd/LES-smagorinsky.xml",)), dims)
+    casefiles.upload(sim, case)
+    o = op.OracleSim(case, bi=False, domain=False, les={"Cs": 0.15},
+                     periodic=case["params"]["periodic"])
+    for _ in range(2):
+        o.step()
+    sim.step(2)
+    for k in ("grad_u", "nu_t", "dudt", "u", "r"):
+        np.testing.assert_array_equal(sim.get(k).ravel(), o.f[k].ravel(),
+                                      err_msg=k)
+    sim.close()
