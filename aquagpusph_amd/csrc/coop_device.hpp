@@ -61,7 +61,8 @@ template <int Q, int B, bool PER> struct CoopLds {
 };
 
 // Walk the accepted candidates of one particle per group of Q lanes.  kind,
-// flag_el, el_near and the relative test (LOOSE): as in ring_walk.
+// flag_el, el_near and the relative test (LOOSE): as in ring_walk (kind 2:
+// candidates with imove < 3).
 // round(n, cw): one round, in which lane q of the group takes the list
 // entries q + Q b < n (cw[b]); called by every lane.
 template <int D, int Q, int B, bool LOOSE, bool PER, class Round>
@@ -136,7 +137,9 @@ coop_list_walk(CoopLds<Q, B, PER>& L, int lane, uint32_t total,
                 rj = per_shift<D>(rj, f3{ sh.x, sh.y, sh.z }, per);
             }
             is_el = (im_j == -3);
-            take = kind ? is_el : (im_j == 1 || (flag_el && is_el));
+            take = kind == 1   ? is_el
+                   : kind == 2 ? im_j < 3
+                               : (im_j == 1 || (flag_el && is_el));
             if (take) {
                 const float dx =
                     fmaxf(fmaxf(bmin.x - rj.x, rj.x - bmax.x), 0.f);
@@ -175,7 +178,7 @@ coop_list_walk(CoopLds<Q, B, PER>& L, int lane, uint32_t total,
         if (cb + 64 < total) fetch(cb + 64);
         if (cnt == 0) continue;
         lds_order();
-        const bool els = !kind && __ballot(take && is_el) != 0;
+        const bool els = kind == 0 && __ballot(take && is_el) != 0;
         // survivors q, q + Q, ...: the bits of the group's lanes are the
         // accept flags of Q successive survivors
         const uint32_t sh = ((uint32_t)(o * Q)) & 31u;

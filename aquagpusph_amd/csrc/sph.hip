@@ -1827,6 +1827,24 @@ void launch_bi_interp_shepard(const uint32_t* iset, const int32_t* imove,
                        rho, p, refd, N, cs, p0);
 }
 
+// pair_groups.hip
+bool shepard_groups(int dims, const int32_t* imove, const float* r,
+                    const float* rho, const float* m, float* shepard,
+                    uint32_t N, const uint32_t* icell, const uint32_t* ihoc,
+                    const uint32_t* n_cells, aq_defs d, int cfd,
+                    hipStream_t s);
+bool interactions_groups(int dims, const int32_t* imove, const float* r,
+                         const float* u, const float* rho, const float* m,
+                         const float* p, float* grad_p, float* lap_u,
+                         float* div_u, uint32_t N, const uint32_t* icell,
+                         const uint32_t* ihoc, const uint32_t* n_cells,
+                         aq_defs d, hipStream_t s);
+bool lapp_groups(int dims, const int32_t* imove, const float* r,
+                 const float* rho, const float* m, const float* p,
+                 float* lap_p, uint32_t N, const uint32_t* icell,
+                 const uint32_t* ihoc, const uint32_t* n_cells, aq_defs d,
+                 hipStream_t s);
+
 void launch_shepard(int dims, const int32_t* imove, const float* r,
                     const float* rho, const float* m, float* shepard,
                     uint32_t N, const uint32_t* icell, const uint32_t* ihoc,
@@ -2226,9 +2244,11 @@ AQ_API int aq_shepard(int dims, const int32_t* imove, const float* r,
         check_defs(defs);
         if (!N) return;
         AQ_PTRS(imove, r, rho, m, shepard, icell, ihoc, n_cells);
-        launch_shepard(dims, imove, r, rho, m, shepard, N, icell, ihoc,
-                       n_cells, nullptr, defs, cfd_variant ? 1 : 0,
-                       S(stream), nullptr);
+        if (!shepard_groups(dims, imove, r, rho, m, shepard, N, icell, ihoc,
+                            n_cells, defs, cfd_variant, S(stream)))
+            launch_shepard(dims, imove, r, rho, m, shepard, N, icell, ihoc,
+                           n_cells, nullptr, defs, cfd_variant ? 1 : 0,
+                           S(stream), nullptr);
     });
 }
 
@@ -2245,9 +2265,12 @@ AQ_API int aq_interactions(int dims, const int32_t* imove, const float* r,
         if (!N) return;
         AQ_PTRS(imove, r, u, rho, m, p, grad_p, lap_u, div_u, icell, ihoc,
                 n_cells);
-        launch_interactions(dims, imove, r, u, rho, m, p, grad_p, lap_u, div_u,
-                            N, icell, ihoc, n_cells, nullptr, defs,
-                            S(stream));
+        if (!interactions_groups(dims, imove, r, u, rho, m, p, grad_p, lap_u,
+                                 div_u, N, icell, ihoc, n_cells, defs,
+                                 S(stream)))
+            launch_interactions(dims, imove, r, u, rho, m, p, grad_p, lap_u,
+                                div_u, N, icell, ihoc, n_cells, nullptr, defs,
+                                S(stream));
     });
 }
 
@@ -2262,8 +2285,10 @@ AQ_API int aq_lapp(int dims, const int32_t* imove, const float* r,
         check_defs(defs);
         if (!N) return;
         AQ_PTRS(imove, r, rho, m, p, lap_p, icell, ihoc, n_cells);
-        launch_lapp(dims, imove, r, rho, m, p, lap_p, N, icell, ihoc, n_cells,
-                    nullptr, defs, S(stream));
+        if (!lapp_groups(dims, imove, r, rho, m, p, lap_p, N, icell, ihoc,
+                         n_cells, defs, S(stream)))
+            launch_lapp(dims, imove, r, rho, m, p, lap_p, N, icell, ihoc,
+                        n_cells, nullptr, defs, S(stream));
     });
 }
 

@@ -154,3 +154,81 @@ def test_les_groups_match_oracle(cuda, tmp_path, dims, n):
         np.testing.assert_array_equal(sim.get(k).ravel(), o.f[k].ravel(),
                                       err_msg=k)
     sim.close()
+
+
+# around the line between 16 and 4 lanes per particle, single particles and
+# cells of more than 64
+@pytest.mark.parametrize("dims,n,cell,lap", [
+    (2, 1, 3, 1), (2, 65, 3, 2), (2, 16384, 4, 1), (2, 16385, 4, 2),
+    (2, 30011, 12, 1), (3, 1, 3, 1), (3, 63, 2, 1), (3, 5000, 6, 2),
+    (3, 16384, 4, 1), (3, 20011, 4, 1)])
+def test_abi_pair_kernels_match_oracle(cuda, dims, n, cell, lap):
+    """aq_shepard (both variants), aq_interactions and aq_lapp on disordered
+    particles of every kind, about cell^dims of them per cell, against the
+    oracle's float32 walk, bit for bit, accumulating onto given values."""
+    from oracle import pipeline as op
+    rng = np.random.default_rng(n + dims)
+    vs = 2 if dims == 2 else 4
+    side = max(1.0, (n / cell ** dims) ** (1 / dims))  # in cells
+    h = np.float32(0.05)
+    r = np.zeros((n, vs), np.float32)
+    r[:, :dims] = rng.uniform(0, side * 2 * h, (n, dims))
+    u = np.zeros_like(r)
+    u[:, :dims] = rng.normal(0, 1, (n, dims))
+    f32 = lambda a: np.ascontiguousarray(a, np.float32)  # noqa: E731
+    rho = f32(1000 + rng.normal(0, 5, n))
+    m = f32(rng.uniform(0.5, 1.5, n))
+    p = f32(rng.normal(0, 100, n))
+    im = rng.choice(np.array([1, 1, 1, 1, 1, 0, -3, 2, 3, -256], np.int32), n)
+    cap = int(side + 8) ** dims
+    d = {k: _dev(v) for k, v in dict(
+        lo=np.zeros(vs, np.float32), hi=np.zeros(vs, np.float32),
+        sup=f32([2]), h=f32([h]), nc=np.zeros(4, np.int32),
+        ic=np.zeros(n, np.int32), pu=np.zeros(n, np.int32),
+        ps=np.zeros(n, np.int32), hoc=np.zeros(cap, np.int32),
+        st=np.zeros(1, np.int32), r=r).items()}
+    ws = torch.empty(int(_lib.lib().aq_linklist_workspace(
+        ctypes.c_uint32(n))), dtype=torch.uint8, device="cuda")
+    _lib.call("aq_linklist", dims, _dp(d["r"]), n, _dp(d["lo"]),
+              _dp(d["hi"]), _dp(d["sup"]), _dp(d["h"]), _dp(d["nc"]),
+              _dp(d["ic"]), _dp(d["pu"]), _dp(d["ps"]), _dp(d["hoc"]), cap,
+              _dp(d["st"]), _dp(ws), _stream())
+    perm = d["pu"].cpu().numpy()
+    assert int(d["st"].item()) == 0
+    r, u, rho, m, p, im = (np.ascontiguousarray(a[perm])
+                           for a in (r, u, rho, m, p, im))
+    H = op.definition(h)
+    CONW = op.definition(1.0 / float(h) ** dims)
+    CONF = op.definition(1.0 / float(h) ** (dims + 2))
+    D = _lib.Defs(H, CONW, CONF, float(dims), lap)
+    g = {k: _dev(v) for k, v in dict(r=r, u=u, rho=rho, m=m, p=p,
+                                     im=im).items()}
+    ll = (n, _dp(d["ic"]), _dp(d["hoc"]), _dp(d["nc"]), D)
+    hic, hhoc, hnc = (d[k].cpu().numpy() for k in ("ic", "hoc", "nc"))
+    oll = tuple(op._p(a) for a in (hic, hhoc, hnc))
+    fn = lambda k: getattr(op.lib(), "orc_%s_f32_%dd" % (k, dims))  # noqa
+    cf, cu = ctypes.c_float, ctypes.c_uint
+    for cfd in (0, 1):
+        want = f32(rng.normal(0, 1, n))
+        got = _dev(want)
+        _lib.call("aq_shepard", dims, _dp(g["im"]), _dp(g["r"]),
+                  _dp(g["rho"]), _dp(g["m"]), _dp(got), *ll, cfd, _stream())
+        fn("shepard")(op._p(im), op._p(r), op._p(rho), op._p(m),
+                      op._p(want), cu(n), *oll, cf(H), cf(CONW),
+                      ctypes.c_int(cfd))
+        np.testing.assert_array_equal(got.cpu().numpy(), want)
+    w = [f32(rng.normal(0, 1, (n, vs))), f32(rng.normal(0, 1, (n, vs))),
+         f32(rng.normal(0, 1, n)), f32(rng.normal(0, 1, n))]
+    t = [_dev(a) for a in w]
+    _lib.call("aq_interactions", dims, _dp(g["im"]), _dp(g["r"]),
+              _dp(g["u"]), _dp(g["rho"]), _dp(g["m"]), _dp(g["p"]),
+              *(_dp(a) for a in t[:3]), *ll, _stream())
+    _lib.call("aq_lapp", dims, _dp(g["im"]), _dp(g["r"]), _dp(g["rho"]),
+              _dp(g["m"]), _dp(g["p"]), _dp(t[3]), *ll, _stream())
+    fn("interactions")(op._p(im), op._p(r), op._p(u), op._p(rho), op._p(m),
+                       op._p(p), *(op._p(a) for a in w[:3]), cu(n), *oll,
+                       cf(H), cf(CONF), ctypes.c_int(lap))
+    fn("lapp")(op._p(im), op._p(r), op._p(rho), op._p(m), op._p(p),
+               op._p(w[3]), cu(n), *oll, cf(H), cf(CONF))
+    for a, b in zip(t, w):
+        np.testing.assert_array_equal(a.cpu().numpy(), b)
