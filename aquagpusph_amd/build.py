@@ -23,9 +23,10 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # -ffp-contract=off: the kernels keep the reference's rounded products and
 # sums (no silent FMA contraction), which the bit-exact parity tests rely on.
 # -packed-fp32-ops: no packed FP32 (v_pk_*_f32) code generation.
+# -amdgpu-mfma-vgpr-form: matrix instructions write VGPRs (no AGPR copies).
 COMMON = ["-O3", "-std=c++17", "-fPIC", "--offload-arch=gfx950",
           "-ffp-contract=off", "-Xclang", "-target-feature", "-Xclang",
-          "-packed-fp32-ops", "-Wall", "-Wno-unused-function",
+          "-packed-fp32-ops", "-mllvm", "-amdgpu-mfma-vgpr-form", "-Wall", "-Wno-unused-function",
           "-Wno-pass-failed",
           "-Wno-unused-variable", "-I" + os.path.join(ROOT, "include")]
 

@@ -39,7 +39,6 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
                  int lapp_, uint32_t S)
 {
     constexpr int OW = 64 / Q;
-    constexpr bool LOOSE = !PER;
     const bool lapp = lapp_ != 0;
     __shared__ CoopLds<Q, B, PER> lds[WC_WAVES];
     const int lane = threadIdx.x & 63;
@@ -142,7 +141,7 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
                         const f3 r_ij = sub<D>(rc[b], r_i);
                         const float s = dot<D>(r_ij, r_ij);
                         float m_j = mc[b];
-                        if (LOOSE) m_j = (s > smax) ? 0.f : m_j;
+                        m_j = (s > smax) ? 0.f : m_j;
                         const f3 u_ij = sub<D>(uc[b], u_i);
                         const float udr = dot<D>(u_ij, r_ij);
                         const bool fd =
@@ -173,7 +172,7 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
                     acc1(lp, clp, t.tl);  // zeros without lap p
                 }
             };
-            coop_list_walk<D, Q, B, LOOSE, PER>(
+            coop_list_walk<D, Q, B, PER>(
                 L, lane, total, r_i, act, bmin, bmax, smax, r, imove, 0,
                 flag_el, nearw, w.per, round);
             // ---- wall elements (boundary-integral Shepard) ------------------
@@ -201,7 +200,7 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
                                 const float r_n = dot<D>(r_ij, n_j);
                                 const float r_t = fabsf(dot<D>(r_ij, t_j));
                                 const float r_b = fabsf(dot<D>(r_ij, b_j));
-                                if (LOOSE && s > smax) {
+                                if (s > smax) {
                                 } else if ((r_n > -eps) && (r_n < eps)) {
                                     const float dr =
                                         0.55f *
@@ -238,7 +237,7 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
                             }
                         }
                     };
-                    coop_list_walk<D, Q, B, LOOSE, PER>(
+                    coop_list_walk<D, Q, B, PER>(
                         L, lane, total_el, r_i, act && nearw, bmin, bmax,
                         smax, r, imove, 1, false, unused, w.per, round_el);
                 }

@@ -93,8 +93,9 @@ __device__ __forceinline__ uint32_t run_table(const RunArgs& w, uint32_t c_i,
 }
 
 // Policies: KIND of the candidates (coop_list_walk), owner(im), State,
-// init(i, st), load(j) (Cand, its position in r), term(i, j, cand, r_ij, s,
-// st), add_group<Q>(st, term), finish(i, st).
+// init(i, st), load(j) (Cand: position r, mass m, ...), term(cand, r_ij, s,
+// st) (carries the mass as a factor), add_group<Q>(st, term), finish(i, st);
+// NO_SELF: a particle is not its own candidate.
 template <int D, int Q, class Pol>
 __global__ void __launch_bounds__(64 * WC_WAVES)
     run_group_k(Pol pol, const int* __restrict__ imove,
@@ -138,16 +139,18 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
             typename Pol::Term t = Pol::none();
             if ((uint32_t)q < n) {
                 const uint32_t j = cw[0];
-                const typename Pol::Cand cd = pol.load(j);
+                typename Pol::Cand cd = pol.load(j);
                 const f3 r_ij = sub<D>(cd.r, r_i);
                 const float s = dot<D>(r_ij, r_ij);
-                // (the relative test accepts a thin shell beyond)
-                if (!(s > smax)) t = pol.term(i, j, cd, r_ij, s, st);
+                // the walk's test accepts a thin shell beyond: no mass (a
+                // select, so that every load of the pair is issued at once)
+                if (s > smax || (Pol::NO_SELF && j == i)) cd.m = 0.f;
+                t = pol.term(cd, r_ij, s, st);
             }
             pol.template add_group<Q>(st, t);
         };
         bool unused = false;
-        coop_list_walk<D, Q, 1, true, false>(
+        coop_list_walk<D, Q, 1, false>(
             L, lane, total, r_i, act, bmin, bmax, smax, r, imove, Pol::KIND,
             false, unused, nullptr, round);
         if (act && q == 0) pol.finish(i, st);
@@ -164,6 +167,7 @@ template <int Q> __device__ __forceinline__ void add_lanes(float& a, float v)
 // other positive imove among the owners), KIND 2: imove < 3
 template <int D, int K> struct PolShepard {
     static constexpr int KIND = K;
+    static constexpr bool NO_SELF = false;
     const float *r, *rho, *m;
     float* shepard;
     float H, CONW;
@@ -184,8 +188,8 @@ template <int D, int K> struct PolShepard {
     {
         return Cand{ ldv_o<D>(r, j), ldf_o(rho, j), ldf_o(m, j) };
     }
-    __device__ Term term(uint32_t, uint32_t, const Cand& c, const f3&,
-                         float s, const State&) const
+    __device__ Term term(const Cand& c, const f3&, float s,
+                         const State&) const
     {
         return kernelW<D>(sqrtf(s) / H) * CONW * c.m / c.rho;
     }
@@ -204,6 +208,7 @@ template <int D, int K> struct PolShepard {
 // cfd/Interactions.cl:60-145
 template <int D> struct PolInteractions {
     static constexpr int KIND = 0;
+    static constexpr bool NO_SELF = true;
     const float *r, *u, *rho, *m, *p;
     float *grad_p, *lap_u, *div_u;
     float H, CONF;
@@ -235,10 +240,9 @@ template <int D> struct PolInteractions {
         return Cand{ ldv_o<D>(r, j), ldv_o<D>(u, j), ldf_o(rho, j),
                      ldf_o(m, j), ldf_o(p, j) };
     }
-    __device__ Term term(uint32_t i, uint32_t j, const Cand& c,
-                         const f3& r_ij, float s, const State& st) const
+    __device__ Term term(const Cand& c, const f3& r_ij, float s,
+                         const State& st) const
     {
-        if (i == j) return none();
         const f3 u_ij = sub<D>(c.u, st.u_i);
         const float udr = dot<D>(u_ij, r_ij);
         const PairTerms t = fluid_pair<D, 0, false>(
@@ -274,6 +278,7 @@ template <int D> struct PolInteractions {
 // basic/deltaSPH.cl:191-242 (lapp), fluid only
 template <int D> struct PolLapP {
     static constexpr int KIND = 0;
+    static constexpr bool NO_SELF = true;
     const float *r, *rho, *m, *p;
     float* lap_p;
     float H, CONF;
@@ -296,10 +301,9 @@ template <int D> struct PolLapP {
         return Cand{ ldv_o<D>(r, j), ldf_o(rho, j), ldf_o(m, j),
                      ldf_o(p, j) };
     }
-    __device__ Term term(uint32_t i, uint32_t j, const Cand& c, const f3&,
-                         float s, const State& st) const
+    __device__ Term term(const Cand& c, const f3&, float s,
+                         const State& st) const
     {
-        if (i == j) return none();
         const float f_ij = kernelF<D>(sqrtf(s) / H) * CONF * c.m / c.rho;
         return (c.p - st.p_i) * f_ij;
     }

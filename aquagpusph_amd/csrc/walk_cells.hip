@@ -944,13 +944,21 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
                         c.r = per_shift<D>(c.r, f3{ sh.x, sh.y, sh.z },
                                            w.per);
                     }
+                    // the walk's test accepts a thin shell beyond: such a
+                    // candidate gets no weight (a select, so that every
+                    // load of the pair is issued at once)
+                    const f3 r_ij = sub<D>(c.r, r_i);
+                    const bool out = dot<D>(r_ij, r_ij) > smax ||
+                                     (Pol::NO_SELF && j == i);
+                    pol.weigh(c, out);
                     t = nrq ? pol.template term<true>(i, j, c, r_i, st)
                             : pol.template term<false>(i, j, c, r_i, st);
+                    pol.weigh(t, out);
                 }
                 pol.template add_group<Q>(st, t);
             };
             bool unused = false;
-            coop_list_walk<D, Q, 1, false, PER>(
+            coop_list_walk<D, Q, 1, PER>(
                 L, lane, total, r_i, act, bmin, bmax, smax, r, imove,
                 Pol::KIND, false, unused, w.per, round);
             if (act && q == 0) pol.finish(i, st);
@@ -965,6 +973,15 @@ template <int Q> __device__ __forceinline__ void add_lanes(float& a, float v)
 {
     each_lane<Q>(v, [&](float x) { a += x; });
 }
+
+// weigh(x, out): takes the weight of an `out` candidate (its mass or area,
+// which every product of the term carries) or of its term
+#define AQ_POL_WEIGH_MASS                                                      \
+    __device__ static void weigh(Cand& c, bool out)                            \
+    {                                                                          \
+        c.m = out ? 0.f : c.m;                                                 \
+    }                                                                          \
+    __device__ static void weigh(Term&, bool) {}
 
 // The element-owner policies below split each pair into load(j) (the
 // candidate's fields), term<NRQ>(i, j, cand, r_i, st) (a pure function of
@@ -983,6 +1000,7 @@ template <int Q> __device__ __forceinline__ void add_lanes(float& a, float v)
 template <int D> struct PolBiShepard {
     static constexpr int BATCH = 4;  // candidates loaded together
     static constexpr int KIND = 1;
+    static constexpr bool NO_SELF = false;  // its own element counts (term)
     static constexpr uint32_t OWNERS = 0;  // elements, sensors, ...
     const int* imove;
     const float *normal, *tangent, *binormal, *m;
@@ -1049,6 +1067,11 @@ template <int D> struct PolBiShepard {
         }
     }
     __device__ static Term none() { return Term{ 0.f, 2u }; }
+    __device__ static void weigh(Cand&, bool) {}
+    __device__ static void weigh(Term& t, bool out)
+    {
+        if (out) t = none();
+    }
     template <int Q>
     __device__ void add_group(State& st, const Term& t) const
     {
@@ -1078,6 +1101,7 @@ template <int D> struct PolBiShepard {
 template <int D> struct PolBiLapU {
     static constexpr int BATCH = 4;  // candidates loaded together
     static constexpr int KIND = 0;
+    static constexpr bool NO_SELF = false;  // never its own candidate
     static constexpr uint32_t OWNERS = AQ_CELL_ELEM;
     const float *r_, *u, *rho, *m;
     float* lap_u;
@@ -1138,6 +1162,7 @@ template <int D> struct PolBiLapU {
         if constexpr (D == 3) st.lu.z += t.v.z;
     }
     __device__ static Term none() { return Term{ f3{ 0.f, 0.f, 0.f }, 0u }; }
+    AQ_POL_WEIGH_MASS
     template <int Q>
     __device__ void add_group(State& st, const Term& t) const
     {
@@ -1156,6 +1181,7 @@ template <int D> struct PolBiLapU {
 template <int D> struct PolBiInterp {
     static constexpr int BATCH = 4;  // candidates loaded together
     static constexpr int KIND = 0;
+    static constexpr bool NO_SELF = false;  // never its own candidate
     static constexpr uint32_t OWNERS = AQ_CELL_ELEM;
     const float *r_, *m, *rho, *grad_p;
     float* p;
@@ -1196,6 +1222,7 @@ template <int D> struct PolBiInterp {
     }
     __device__ void add(State& st, const Term& t) const { st.acc += t; }
     __device__ static Term none() { return 0.f; }
+    AQ_POL_WEIGH_MASS
     template <int Q>
     __device__ void add_group(State& st, const Term& t) const
     {
@@ -1213,6 +1240,7 @@ template <int D> struct PolBiInterp {
 template <int D> struct PolBiInteractions {
     static constexpr int BATCH = 4;  // candidates loaded together
     static constexpr int KIND = 1;
+    static constexpr bool NO_SELF = false;  // never its own candidate
     static constexpr uint32_t OWNERS = AQ_CELL_FLUID;
     const float *r_, *normal, *u, *rho, *m, *p;
     float *grad_p, *div_u;
@@ -1265,6 +1293,11 @@ template <int D> struct PolBiInteractions {
         st.dv += t.d;
     }
     __device__ static Term none() { return Term{ f3{ 0.f, 0.f, 0.f }, 0.f }; }
+    __device__ static void weigh(Cand& c, bool out)
+    {
+        c.area = out ? 0.f : c.area;
+    }
+    __device__ static void weigh(Term&, bool) {}
     template <int Q>
     __device__ void add_group(State& st, const Term& t) const
     {
@@ -1292,6 +1325,7 @@ template <int D> struct PolBiInteractions {
 // launcher.  (Group kernel only.)
 template <int D> struct PolLesGradU {
     static constexpr int KIND = 0;
+    static constexpr bool NO_SELF = true;
     static constexpr uint32_t OWNERS = AQ_CELL_FLUID;
     static constexpr int NR = (D == 2) ? 2 : 4;
     const float *r_, *u, *rho, *m;
@@ -1321,11 +1355,10 @@ template <int D> struct PolLesGradU {
                      ldf_o(rho, j) };
     }
     template <bool NRQ>
-    __device__ Term term(uint32_t i, uint32_t j, const Cand& c,
-                         const f3& r_i, const State& st) const
+    __device__ Term term(uint32_t, uint32_t, const Cand& c, const f3& r_i,
+                         const State& st) const
     {
-        Term t = none();
-        if (i == j) return t;
+        Term t;
         const f3 r_ij = sub<D>(c.r, r_i);
         const float q = qof<NRQ>(dot<D>(r_ij, r_ij), H);
         const float w = kernelF<D>(q) * CONF * c.m / c.rho;
@@ -1345,6 +1378,7 @@ template <int D> struct PolLesGradU {
         for (int k = 0; k < D * D; k++) t.g[k] = 0.f;
         return t;
     }
+    AQ_POL_WEIGH_MASS
     template <int Q>
     __device__ void add_group(State& st, const Term& t) const
     {
@@ -1372,6 +1406,7 @@ template <int D> struct PolLesGradU {
 // summed in the walk order and added to dudt at the end.
 template <int D> struct PolLesInteractions {
     static constexpr int KIND = 0;
+    static constexpr bool NO_SELF = true;
     static constexpr uint32_t OWNERS = AQ_CELL_FLUID;
     const float *r_, *u, *rho, *m, *nu_t;
     float* dudt;
@@ -1399,10 +1434,9 @@ template <int D> struct PolLesInteractions {
                      ldf_o(rho, j), ldf_o(nu_t, j) };
     }
     template <bool NRQ>
-    __device__ Term term(uint32_t i, uint32_t j, const Cand& c,
-                         const f3& r_i, const State& st) const
+    __device__ Term term(uint32_t, uint32_t, const Cand& c, const f3& r_i,
+                         const State& st) const
     {
-        if (i == j) return none();
         const f3 r_ij = sub<D>(c.r, r_i);
         const float q = qof<NRQ>(dot<D>(r_ij, r_ij), H);
         const float f = kernelF<D>(q) * CONF * c.m;
@@ -1411,6 +1445,7 @@ template <int D> struct PolLesInteractions {
         return scl<D>(sc, sub<D>(c.u, st.u_i));
     }
     __device__ static Term none() { return f3{ 0.f, 0.f, 0.f }; }
+    AQ_POL_WEIGH_MASS
     template <int Q>
     __device__ void add_group(State& st, const Term& t) const
     {
