@@ -60,15 +60,15 @@ __device__ __forceinline__ uint32_t next_cell(const WalkArgs& w,
     return uni(hk);
 }
 
-// Shared state of one wavefront: neighbour-cell table, the candidate chunk
-// being tested and the two segment slots (candidate indices, accept bits;
-// SEGW 32-bit words of bits per lane and slot).
-template <int SEGW, bool PER = false> struct WaveLds {
+// Shared state of one wavefront of the fused walk: neighbour-cell table,
+// staged candidates (two chunks of 64, see dist_tile) and the ring of tested
+// chunks (candidate words, SEGW words of accept bits per lane).
+template <int SEGW, bool PER = false> struct RingLds {
     uint32_t start[27];
     uint32_t cum[28];
-    float4 stage[64];
-    uint32_t cand[2][SEGW * 32];
-    uint32_t bits[2][SEGW][64];
+    float4 stage[2][80];
+    uint32_t cand[SEGW * 32];
+    uint32_t bits[SEGW][64];
     // periodic box: the shift of each neighbour cell's particles
     float4 shift[PER ? 27 : 1];
 };
@@ -76,8 +76,10 @@ template <int SEGW, bool PER = false> struct WaveLds {
 // Walk the accepted candidates of one particle per lane.  `kind` selects
 // the candidates (0: fluid particles, imove == 1; 1: wall elements,
 // imove == -3); with kind 0 and `flag_el`, wall elements in range are also
-// tested and reported through `el_near`.  pair(j) is called for the
-// accepted candidates of each lane in increasing candidate order.
+// tested and reported through `el_near`.  pair(j, kl) is called for the
+// accepted candidates of each lane in increasing candidate order; kl is the
+// neighbour-table entry the candidate came from (its shift in a periodic
+// walk; 0 otherwise).
 //
 // (A branch-free variant, calling pair() on every lane at every step with a
 // dummy index on the idle lanes, measured 25% slower on the 3D dam break:
@@ -86,16 +88,225 @@ template <int SEGW, bool PER = false> struct WaveLds {
 //
 // Box prefilter: a candidate farther than the support from the bounding box
 // of the active lanes' positions is accepted by no lane, so it is not
-// staged; the survivors of each 64-candidate chunk are compacted in their
-// order (each lane's accepted candidates keep their order, so the sums are
-// unchanged).  The box distance is computed like the lanes' own test, one
+// staged.  The box distance is computed like the lanes' own test, one
 // rounded subtraction, square and sum per axis in the same order, and
 // rounding is monotone, so it never exceeds a lane's s: the prefilter
-// drops only candidates every lane would reject.
-// pair(j, kl): kl is the neighbour-table entry the candidate came from
-// (its shift in a periodic walk; 0 otherwise).
+// drops only candidates every lane would reject.  The survivors are packed,
+// in their order, into chunks of 64 across the cells' ends (a quarter of an
+// interior 3D cell's candidates is dropped), and a chunk is refilled as soon
+// as no lane reads from it.  The window of the ring sets the pace both ways:
+// the lanes of a cell accept from different stretches of the list, so a
+// narrow one leaves lanes idle, and a wide one scatters their gathers over
+// more lines than the cache holds for 16 wavefronts.  3D dam break, 1.2 M /
+// 4.5 M particles, walk in us by survivors in the ring: 128: 1867 / 6439,
+// 192: 1816 / 6439, 256: 1789 / 6382, 384: 2099 / 7567, 512: 2359 / 8936
+// (two slots of 256 list entries, refilled whole: 2014 / 6924).
 //
-// NB > 1 (batched consume, not periodic): `pair` has load(j), returning
+// Test: the squared distances of a chunk to the 64 particles by matrix
+// instructions (dist_tile), on coordinates relative to the box centre c:
+// s' = |r_i - c|^2 + |r_j - c|^2 - 2 (r_i - c).(r_j - c), within 64 ulp of
+// R^2 (R bounds |r - c| for every owner and survivor: the half diagonal of
+// the box plus the support radius) of the reference's s.  The test s' <=
+// smax + 2^-14 R^2 accepts every candidate the exact test accepts, and a few
+// within a relative 2^-14 R^2 / smax beyond; the consume repeats the exact
+// test (s <= smax) before adding a pair, so the sums are unchanged.
+template <int D, int SEGW, bool PER, class Pair>
+__device__ __forceinline__ void
+ring_walk_m(RingLds<SEGW, PER>& L, int lane, uint32_t total, const f3& r_i,
+            bool act, const f3& bmin, const f3& bmax, float smax,
+            const float* __restrict__ r, const int* __restrict__ imove,
+            int kind, bool flag_el, bool& el_near, Pair pair,
+            const float* __restrict__ per)
+{
+    constexpr uint32_t RING = SEGW;  // words of accept bits per lane
+    f3 cen = { 0.f, 0.f, 0.f };
+    float limit = smax;
+    if (bmin.x <= bmax.x) {
+        cen = f3{ uni_f(0.5f * (bmin.x + bmax.x)),
+                  uni_f(0.5f * (bmin.y + bmax.y)),
+                  D == 3 ? uni_f(0.5f * (bmin.z + bmax.z)) : 0.f };
+        const f3 hd = sub<D>(bmax, cen);
+        const float rb = sqrtf(dot<D>(hd, hd)) * 1.0001f + sqrtf(smax);
+        limit = uni_f(smax + rb * rb * 0x1p-14f);
+    }
+    // lane (g, o): B and C of the particles o, 16 + o, 32 + o, 48 + o
+    const int g = lane >> 4, o = lane & 15;
+    float mB[4], mC[4];
+    {
+        const f3 rio = sub<D>(r_i, cen);
+        const float ai = dot<D>(rio, rio);
+#pragma unroll
+        for (int n = 0; n < 4; n++) {
+            const f3 v = { __shfl(rio.x, 16 * n + o),
+                           __shfl(rio.y, 16 * n + o),
+                           __shfl(rio.z, 16 * n + o) };
+            const float av = __shfl(ai, 16 * n + o);
+            mB[n] = dist_b(g, v, av);
+            mC[n] = dist_c(av, limit);
+        }
+    }
+    uint16_t* half = reinterpret_cast<uint16_t*>(&L.bits[0][0]);
+    int kl = 0;        // per-lane cursor: neighbour cell of a candidate
+    uint32_t nw = 0;   // next word to load (the current one is nw - 1)
+    uint32_t bw = 0;   // remaining bits of the current word
+    uint32_t wt = 0;   // words tested
+    uint32_t cb = 0;   // candidates read
+    uint32_t ns = 0;   // survivors staged
+    bool done = false; // every survivor is tested
+    uint64_t elm[2] = { 0, 0 };  // wall elements of the staged chunks
+    bool eln = false;
+    auto advance = [&]() {
+        const uint32_t tw = act ? wt : 0u;
+        while (bw == 0 && nw < tw) {
+            bw = L.bits[nw % RING][lane];
+            nw++;
+        }
+    };
+    // consume while no chunk can be refilled (a lane still reads from the
+    // oldest) and some lane has a candidate left
+    auto go = [&]() {
+        advance();
+        if (!done && (wt < RING ||
+                      __ballot(bw != 0 && nw <= wt - RING + 2) == 0))
+            return false;
+        return __ballot(bw != 0) != 0;
+    };
+    while (true) {
+        // the test sits at the bottom of the consume loop, so the pair sums
+        // leave it from where they are updated (no copies at the back edge)
+        for (bool more = go(); more; more = go()) {
+            if (bw != 0) {
+                const uint32_t b = __builtin_clz(bw);
+                bw ^= 0x80000000u >> b;
+                const uint32_t cw = L.cand[((nw - 1) % RING) * 32 + b];
+                if constexpr (PER)
+                    pair(cw & PER_J_MASK, cw >> PER_KL_SHIFT);
+                else
+                    pair(cw, 0u);
+            }
+        }
+        if (done) break;  // and no lane has a candidate left
+        // stage survivors up to a whole chunk (or the candidates' end)
+        while (ns < wt * 32 + 64 && cb < total) {
+            const uint32_t t = cb + (uint32_t)lane;
+            bool take = false, is_el = false;
+            uint32_t word = 0;
+            float4 st = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (t < total) {
+                while (t >= L.cum[kl + 1]) kl++;
+                const uint32_t j = L.start[kl] + (t - L.cum[kl]);
+                f3 rj = ldv_o<D>(r, j);
+                const int im_j = ldi_o(imove, j);
+                word = PER ? (j | ((uint32_t)kl << PER_KL_SHIFT)) : j;
+                if constexpr (PER) {
+                    const float4 sh = L.shift[kl];
+                    rj = per_shift<D>(rj, f3{ sh.x, sh.y, sh.z }, per);
+                }
+                is_el = (im_j == -3);
+                take = kind ? is_el : (im_j == 1 || (flag_el && is_el));
+                if (take) {
+                    const float dx =
+                        fmaxf(fmaxf(bmin.x - rj.x, rj.x - bmax.x), 0.f);
+                    const float dy =
+                        fmaxf(fmaxf(bmin.y - rj.y, rj.y - bmax.y), 0.f);
+                    float d2 = dx * dx;
+                    d2 = d2 + dy * dy;
+                    if constexpr (D == 3) {
+                        const float dz =
+                            fmaxf(fmaxf(bmin.z - rj.z, rj.z - bmax.z), 0.f);
+                        d2 = d2 + dz * dz;
+                    }
+                    take = !(d2 > smax);
+                }
+                st = dist_stage<D>(sub<D>(rj, cen));
+            }
+            const uint64_t tm = __ballot(take);
+            const uint32_t rank =
+                ns + __builtin_amdgcn_mbcnt_hi(
+                         (uint32_t)(tm >> 32),
+                         __builtin_amdgcn_mbcnt_lo((uint32_t)tm, 0u));
+            if (take) {
+                float4* sg = L.stage[(rank >> 6) & 1];
+                sg[dist_slot(rank & 63u)] = st;
+                *dist_word<4>(sg, rank & 63u) = word;
+            }
+            if (!kind) {
+                uint64_t e = __ballot(take && is_el);
+                while (e != 0) {
+                    const int b = __builtin_ctzll(e);
+                    const uint32_t k =
+                        ns + (uint32_t)__popcll(tm & ((1ull << b) - 1ull));
+                    if ((k >> 6) & 1) elm[1] |= 1ull << (k & 63u);
+                    else elm[0] |= 1ull << (k & 63u);
+                    e &= e - 1ull;
+                }
+            }
+            ns += (uint32_t)__popcll(tm);
+            cb += 64;
+        }
+        lds_order();
+        const uint32_t have = min(ns - wt * 32, 64u);
+        done = cb >= total && ns <= wt * 32 + 64;
+        if (have != 0) {
+            // the chunk's accept bits: candidates 16 g .. in the upper (g
+            // even) or lower half of word wt + g / 2
+            const uint32_t hf = (wt >> 1) & 1;
+            float4* sg = L.stage[hf];
+            const float* row = dist_row(sg, lane);
+            const float A[4] = { row[0], row[16], row[32], row[48] };
+            const uint64_t valid =
+                have < 64 ? (1ull << have) - 1ull : ~0ull;
+            const uint32_t vb = dist_bits(valid, g);
+            const uint32_t at =
+                2u * (((wt + (uint32_t)(g >> 1)) % RING) * 64u +
+                      (uint32_t)o) + ((g & 1) ? 0u : 1u);
+#pragma unroll
+            for (int n = 0; n < 4; n++) {
+                half[at + 32u * (uint32_t)n] =
+                    (uint16_t)(dist_tile(A, mB[n], mC[n]) & vb);
+                // one tile's results live at a time (registers)
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            L.cand[(wt % RING) * 32 + (uint32_t)lane] =
+                *dist_word<4>(sg, (uint32_t)lane);
+            lds_order();
+            const uint64_t em = hf ? elm[1] : elm[0];
+            if (!kind && em != 0) {
+                // wall elements in range: flagged, then dropped
+                const uint32_t el =
+                    __builtin_bitreverse32((uint32_t)em);
+                const uint32_t eh =
+                    __builtin_bitreverse32((uint32_t)(em >> 32));
+                const uint32_t lo = L.bits[wt % RING][lane];
+                const uint32_t hi = L.bits[(wt + 1) % RING][lane];
+                eln = eln || (act && ((lo & el) | (hi & eh)) != 0);
+                L.bits[wt % RING][lane] = lo & ~el;
+                L.bits[(wt + 1) % RING][lane] = hi & ~eh;
+                if (hf) elm[1] = 0;
+                else elm[0] = 0;
+            }
+            wt += 2;
+        }
+    }
+    el_near = eln;
+    lds_order();
+}
+
+// ---- one owner per lane over a ring of segments (cell_kernel_k) -------------
+// Shared state of one wavefront: neighbour-cell table, the candidate chunk
+// being tested and the two segment slots (candidate indices, accept bits;
+// SEGW 32-bit words of bits per lane and slot).
+template <int SEGW> struct WaveLds {
+    uint32_t start[27];
+    uint32_t cum[28];
+    float4 stage[64];
+    uint32_t cand[2][SEGW * 32];
+    uint32_t bits[2][SEGW][64];
+};
+
+// ring_walk: as ring_walk_m with the exact distances on the vector ALU, for
+// candidates of one kind (0 fluid, 1 wall elements).  Batched consume:
+// `pair` has load(j), returning
 // the candidate's fields, and use(j, fields); each step takes up to NB
 // accepted candidates of the lane's current bit word, issues all their
 // loads, then uses them in increasing candidate order.  A lane's pair
@@ -105,28 +316,14 @@ template <int SEGW, bool PER = false> struct WaveLds {
 // candidates instead of one per candidate, with the same terms in the same
 // order.
 //
-// LOOSE (the fused fluid walk, not periodic): the per-lane test runs on
-// coordinates relative to the box centre c, s' = |r_i - c|^2 + |r_j - c|^2
-// - 2 (r_i - c).(r_j - c), with |r_j - c|^2 computed once per staged
-// candidate: 5 operations per lane and candidate instead of 8.  s' is
-// within 64 ulp of R^2 (R bounds |r - c| for every owner and survivor:
-// the half diagonal of the box plus the support radius) of the reference's
-// s, so the test s' <= smax + 2^-14 R^2 accepts every candidate the exact
-// test accepts, and a few within a relative 2^-14 R^2 / smax beyond; the
-// consume repeats the exact test (s <= smax) before adding a pair, so the
-// sums are unchanged.  The staged record's w carries |r_j - c|^2 with the
-// sign bit set for wall elements.
-template <int D, int SEGW, int NB = 1, bool LOOSE = false, bool PER,
-          class Pair>
-__device__ __forceinline__ void ring_walk(WaveLds<SEGW, PER>& L, int lane,
+template <int D, int SEGW, int NB, class Pair>
+__device__ __forceinline__ void ring_walk(WaveLds<SEGW>& L, int lane,
                                           uint32_t total, const f3& r_i,
                                           bool act, const f3& bmin,
                                           const f3& bmax, float smax,
                                           const float* __restrict__ r,
                                           const int* __restrict__ imove,
-                                          int kind, bool flag_el,
-                                          bool& el_near, Pair pair,
-                                          const float* __restrict__ per)
+                                          int kind, Pair pair)
 {
     constexpr uint32_t SEG = SEGW * 32;
     const uint32_t nsegs = (total + SEG - 1) / SEG;
@@ -136,28 +333,10 @@ __device__ __forceinline__ void ring_walk(WaveLds<SEGW, PER>& L, int lane,
     constexpr uint32_t RING = 2 * SEGW;
     const uint32_t* bits = &L.bits[0][0][0];
     const uint32_t* cand = &L.cand[0][0];
-    static_assert(!(LOOSE && PER), "relative test: not for periodic walks");
-    // LOOSE: the reference point, the owner's relative position and the
-    // widened threshold
-    f3 cen = { 0.f, 0.f, 0.f }, rio = { 0.f, 0.f, 0.f };
-    float ai = 0.f, smaxl = smax;
-    if constexpr (LOOSE) {
-        if (bmin.x <= bmax.x) {
-            cen = f3{ uni_f(0.5f * (bmin.x + bmax.x)),
-                      uni_f(0.5f * (bmin.y + bmax.y)),
-                      D == 3 ? uni_f(0.5f * (bmin.z + bmax.z)) : 0.f };
-            const f3 hd = sub<D>(bmax, cen);
-            const float rb = sqrtf(dot<D>(hd, hd)) * 1.0001f + sqrtf(smax);
-            smaxl = uni_f(smax + rb * rb * 0x1p-14f);
-        }
-        rio = sub<D>(r_i, cen);
-        ai = dot<D>(rio, rio);
-    }
     int kl = 0;          // per-lane cursor: neighbour cell of a staged candidate
     uint32_t nw = 0;     // next word to load (the current one is nw - 1)
     uint32_t bw = 0;     // remaining bits of the current word
     uint32_t tested = 0;
-    bool eln = false;
     auto advance = [&]() {
         const uint32_t tw = min(tested * SEGW, nwords);
         while (bw == 0 && nw < tw) {
@@ -179,38 +358,25 @@ __device__ __forceinline__ void ring_walk(WaveLds<SEGW, PER>& L, int lane,
         // the test sits at the bottom of the consume loop, so the pair sums
         // leave it from where they are updated (no copies at the back edge)
         for (bool more = go(); more; more = go()) {
-            if constexpr (NB == 1) {
+            uint32_t jb[NB];
+            int nb = 0;
+#pragma unroll
+            for (int k = 0; k < NB; k++) {
+                jb[k] = 0;
                 if (bw != 0) {
                     const uint32_t b = __builtin_clz(bw);
                     bw ^= 0x80000000u >> b;
-                    const uint32_t cw = cand[((nw - 1) % RING) * 32 + b];
-                    if constexpr (PER)
-                        pair(cw & PER_J_MASK, cw >> PER_KL_SHIFT);
-                    else
-                        pair(cw, 0u);
+                    jb[k] = cand[((nw - 1) % RING) * 32 + b];
+                    nb = k + 1;
                 }
-            } else {
-                static_assert(!PER, "batched consume: not for periodic walks");
-                uint32_t jb[NB];
-                int nb = 0;
-#pragma unroll
-                for (int k = 0; k < NB; k++) {
-                    jb[k] = 0;
-                    if (bw != 0) {
-                        const uint32_t b = __builtin_clz(bw);
-                        bw ^= 0x80000000u >> b;
-                        jb[k] = cand[((nw - 1) % RING) * 32 + b];
-                        nb = k + 1;
-                    }
-                }
-                decltype(pair.load(0u)) cd[NB];
-#pragma unroll
-                for (int k = 0; k < NB; k++)
-                    if (k < nb) cd[k] = pair.load(jb[k]);
-#pragma unroll
-                for (int k = 0; k < NB; k++)
-                    if (k < nb) pair.use(jb[k], cd[k]);
             }
+            decltype(pair.load(0u)) cd[NB];
+#pragma unroll
+            for (int k = 0; k < NB; k++)
+                if (k < nb) cd[k] = pair.load(jb[k]);
+#pragma unroll
+            for (int k = 0; k < NB; k++)
+                if (k < nb) pair.use(jb[k], cd[k]);
         }
         if (tested >= nsegs) break;  // and no lane has a candidate left
         // refill the oldest slot: chunk(cb, ...) tests the candidates
@@ -222,10 +388,9 @@ __device__ __forceinline__ void ring_walk(WaveLds<SEGW, PER>& L, int lane,
         auto chunk = [&](uint32_t cb, bool have, uint32_t j, f3 rj,
                          int im_j) {
             float4 st = make_float4(0.f, 0.f, 0.f, 0.f);
-            bool take = false, is_el = false;
+            bool take = false;
             if (have) {
-                is_el = (im_j == -3);
-                take = kind ? is_el : (im_j == 1 || (flag_el && is_el));
+                take = kind ? (im_j == -3) : (im_j == 1);
                 if (take) {
                     const float dx =
                         fmaxf(fmaxf(bmin.x - rj.x, rj.x - bmax.x), 0.f);
@@ -240,29 +405,13 @@ __device__ __forceinline__ void ring_walk(WaveLds<SEGW, PER>& L, int lane,
                     }
                     take = !(d2 > smax);
                 }
-                if constexpr (LOOSE) {
-                    const f3 rjo = sub<D>(rj, cen);
-                    float bj = rjo.x * rjo.x;
-                    bj = __builtin_fmaf(rjo.y, rjo.y, bj);
-                    if constexpr (D == 3) bj = __builtin_fmaf(rjo.z, rjo.z, bj);
-                    st = make_float4(rjo.x, rjo.y, rjo.z, is_el ? -bj : bj);
-                } else {
-                    st = make_float4(rj.x, rj.y, rj.z, is_el ? 1.f : 0.f);
-                }
+                st = make_float4(rj.x, rj.y, rj.z, 0.f);
             }
             // the per-lane test of a staged candidate
             auto accept = [&](const float4& c) {
-                if constexpr (LOOSE) {
-                    float t = rio.x * c.x;
-                    t = __builtin_fmaf(rio.y, c.y, t);
-                    if constexpr (D == 3) t = __builtin_fmaf(rio.z, c.z, t);
-                    const float s = __builtin_fmaf(-2.f, t, ai + fabsf(c.w));
-                    return !(s > smaxl);
-                } else {
-                    const f3 r_ij = sub<D>(f3{ c.x, c.y, c.z }, r_i);
-                    const float s = dot<D>(r_ij, r_ij);
-                    return !(s > smax);
-                }
+                const f3 r_ij = sub<D>(f3{ c.x, c.y, c.z }, r_i);
+                const float s = dot<D>(r_ij, r_ij);
+                return !(s > smax);
             };
             const uint64_t tm = __ballot(take);
             const uint32_t cnt = (uint32_t)__popcll(tm);
@@ -274,8 +423,7 @@ __device__ __forceinline__ void ring_walk(WaveLds<SEGW, PER>& L, int lane,
                     __builtin_amdgcn_mbcnt_lo((uint32_t)tm, 0u));
                 if (take) {
                     L.stage[rank] = st;
-                    L.cand[slot][cb + rank] =
-                        PER ? (j | ((uint32_t)kl << PER_KL_SHIFT)) : j;
+                    L.cand[slot][cb + rank] = j;
                 }
                 __builtin_amdgcn_wave_barrier();
                 __builtin_amdgcn_s_waitcnt(0);
@@ -291,98 +439,47 @@ __device__ __forceinline__ void ring_walk(WaveLds<SEGW, PER>& L, int lane,
                     if (cnt < 64u) hi <<= 64u - cnt;
                 }
                 if (!act) lo = hi = 0;
-                if (!kind && __ballot(take && is_el) != 0) {
-                    // wall elements in range: flagged, then dropped
-                    uint32_t el = 0, eh = 0;
-                    for (uint32_t k = 0; k < cnt; k++) {
-                        const float w = L.stage[k].w;
-                        if (LOOSE ? !(__float_as_uint(w) >> 31) : w == 0.f)
-                            continue;
-                        if (k < 32u) el |= 0x80000000u >> k;
-                        else eh |= 0x80000000u >> (k - 32u);
-                    }
-                    eln = eln || ((lo & el) | (hi & eh)) != 0;
-                    lo &= ~el;
-                    hi &= ~eh;
-                }
             }
             L.bits[slot][cb >> 5][lane] = lo;
             if (nseg - cb > 32) L.bits[slot][(cb >> 5) + 1][lane] = hi;
             __builtin_amdgcn_wave_barrier();
         };
-        if constexpr (NB > 1) {
-            // the whole segment's candidate loads issued together
-            constexpr uint32_t NCH = SEG / 64;
-            uint32_t pj[NCH];
-            f3 prj[NCH];
-            int pim[NCH];
+        // the whole segment's candidate loads issued together
+        constexpr uint32_t NCH = SEG / 64;
+        uint32_t pj[NCH];
+        f3 prj[NCH];
+        int pim[NCH];
 #pragma unroll
-            for (uint32_t ch = 0; ch < NCH; ch++) {
-                pj[ch] = 0;
-                const uint32_t t = seg + ch * 64 + lane;
-                if (ch * 64 + lane < nseg) {
-                    while (t >= L.cum[kl + 1]) kl++;
-                    pj[ch] = L.start[kl] + (t - L.cum[kl]);
-                }
+        for (uint32_t ch = 0; ch < NCH; ch++) {
+            pj[ch] = 0;
+            const uint32_t t = seg + ch * 64 + lane;
+            if (ch * 64 + lane < nseg) {
+                while (t >= L.cum[kl + 1]) kl++;
+                pj[ch] = L.start[kl] + (t - L.cum[kl]);
             }
+        }
 #pragma unroll
-            for (uint32_t ch = 0; ch < NCH; ch++) {
-                prj[ch] = f3{ 0.f, 0.f, 0.f };
-                pim[ch] = 0;
-                if (ch * 64 + lane < nseg) {
-                    prj[ch] = ldv_o<D>(r, pj[ch]);
-                    pim[ch] = ldi_o(imove, pj[ch]);
-                }
+        for (uint32_t ch = 0; ch < NCH; ch++) {
+            prj[ch] = f3{ 0.f, 0.f, 0.f };
+            pim[ch] = 0;
+            if (ch * 64 + lane < nseg) {
+                prj[ch] = ldv_o<D>(r, pj[ch]);
+                pim[ch] = ldi_o(imove, pj[ch]);
             }
+        }
 #pragma unroll
-            for (uint32_t ch = 0; ch < NCH; ch++) {
-                if (ch * 64 >= nseg) break;
-                chunk(ch * 64, ch * 64 + lane < nseg, pj[ch], prj[ch],
-                      pim[ch]);
-            }
-        } else {
-            for (uint32_t cb = 0; cb < nseg; cb += 64) {
-                const uint32_t t = seg + cb + lane;
-                uint32_t j = 0;
-                f3 rj = { 0.f, 0.f, 0.f };
-                int im_j = 0;
-                const bool have = cb + lane < nseg;
-                if (have) {
-                    while (t >= L.cum[kl + 1]) kl++;
-                    j = L.start[kl] + (t - L.cum[kl]);
-                    rj = ldv_o<D>(r, j);
-                    if constexpr (PER) {
-                        const float4 sh = L.shift[kl];
-                        rj = per_shift<D>(rj, f3{ sh.x, sh.y, sh.z }, per);
-                    }
-                    im_j = ldi_o(imove, j);
-                }
-                chunk(cb, have, j, rj, im_j);
-            }
+        for (uint32_t ch = 0; ch < NCH; ch++) {
+            if (ch * 64 >= nseg) break;
+            chunk(ch * 64, ch * 64 + lane < nseg, pj[ch], prj[ch],
+                  pim[ch]);
         }
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_s_waitcnt(0);
         tested++;
     }
-    el_near = eln;
     __builtin_amdgcn_wave_barrier();
 }
 
-// The fused walk's form of ring_walk (one candidate per consume step).
-template <int D, int SEGW, bool LOOSE = false, bool PER, class Pair>
-__device__ __forceinline__ void ring_walk_l(WaveLds<SEGW, PER>& L, int lane,
-                                            uint32_t total, const f3& r_i,
-                                            bool act, const f3& bmin,
-                                            const f3& bmax, float smax,
-                                            const float* __restrict__ r,
-                                            const int* __restrict__ imove,
-                                            int kind, bool flag_el,
-                                            bool& el_near, Pair pair,
-                                            const float* __restrict__ per)
-{
-    ring_walk<D, SEGW, 1, LOOSE>(L, lane, total, r_i, act, bmin, bmax, smax,
-                                 r, imove, kind, flag_el, el_near, pair, per);
-}
 // ---------------------------------------------------------------------------
 // Fused fluid walk (same terms as fluid_pass_k in sph.hip).
 //   MATH 0: IEEE-754 terms and sums, bit-identical to the oracle;
@@ -494,10 +591,10 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
                        float smax, float iH, const uint32_t* __restrict__ rec)
 {
     constexpr float CLEARY = (D == 2) ? 8.f : 10.f;
-    __shared__ WaveLds<SEGW, PER> lds[WC_WAVES];
+    __shared__ RingLds<SEGW, PER> lds[WC_WAVES];
     const int lane = threadIdx.x & 63;
     const int wv = threadIdx.x >> 6;
-    WaveLds<SEGW, PER>& L = lds[wv];
+    RingLds<SEGW, PER>& L = lds[wv];
     // a candidate's position, at its nearest image in a periodic box
     auto rjof = [&](uint32_t j, uint32_t kl) {
         f3 v = ldv_o<D>(r, j);
@@ -602,20 +699,19 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
             // div_nr / sqrt_nr where the per-pair bounds hold (s == 0 or
             // s >= 2^-96, udr == 0 or |udr| >= T), the IEEE sequences for
             // the other pairs
-            // The relative-coordinate test (LOOSE) accepts a thin shell
-            // beyond the support.  Such a candidate is given zero mass here
+            // The relative-coordinate test accepts a thin shell beyond the
+            // support.  Such a candidate is given zero mass here
             // (the reference's test, s <= smax, as a select rather than a
             // branch, so every load of the pair is issued at once): its
             // terms are then +-0 (finite fields), and adding +-0 leaves the
             // sums unchanged, since they are never -0 (they start at +0, or
             // 1, and an exact cancellation rounds to +0).
-            constexpr bool LOOSE = (MATH != 1) && !PER;
             auto pair_fd = [&](uint32_t j, uint32_t kl) {
                 const f3 r_ij = sub<D>(rjof(j, kl), r_i);
                 const float s = dot<D>(r_ij, r_ij);
                 const float qf = div_nr(sqrt_nr(s), RH);
                 float m_j = ldf_o(m, j);
-                if (LOOSE) m_j = (s > smax) ? 0.f : m_j;
+                m_j = (s > smax) ? 0.f : m_j;
                 const float rho_j = ldf_o(rho, j);
                 const float p_j = ldf_o(p, j);
                 const f3 u_ij = sub<D>(ldv_o<D>(u, j), u_i);
@@ -637,7 +733,8 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
                         const f3 r_ij = sub<D>(rjof(j, kl), r_i);
                         const float s = fdot<D>(r_ij, r_ij);
                         const float q = __builtin_amdgcn_sqrtf(s) * iH;
-                        const float m_j = ldf_o(m, j);
+                        float m_j = ldf_o(m, j);
+                        m_j = (s > smax) ? 0.f : m_j;
                         const float irho_j =
                             __builtin_amdgcn_rcpf(ldf_o(rho, j));
                         if (SHEP == 1)
@@ -665,7 +762,7 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
                     const float s = dot<D>(r_ij, r_ij);
                     const float q = sqrtf(s) / H;
                     float m_j = ldf_o(m, j);
-                    if (LOOSE) m_j = (s > smax) ? 0.f : m_j;
+                    m_j = (s > smax) ? 0.f : m_j;
                     const float rho_j = ldf_o(rho, j);
                     const float p_j = ldf_o(p, j);
                     const f3 u_ij = sub<D>(ldv_o<D>(u, j), u_i);
@@ -673,33 +770,26 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
                     terms(std::false_type{}, r_ij, q, m_j, rho_j, p_j, u_ij,
                           udr);
             };
-            if constexpr (MATH != 1) {
-                if (fastdiv) {
-                    ring_walk_l<D, SEGW, LOOSE>(
-                        L, lane, total, r_i, act, bmin, bmax, smax, r, imove,
-                        0, flag_el, nearw, pair_fd, w.per);
-                } else {
-                    ring_walk_l<D, SEGW, LOOSE>(
-                        L, lane, total, r_i, act, bmin, bmax, smax, r, imove,
-                        0, flag_el, nearw, pair_ieee, w.per);
-                }
-            } else {
-                ring_walk_l<D, SEGW, false>(L, lane, total, r_i, act, bmin,
-                                           bmax, smax, r, imove, 0, flag_el,
-                                           nearw, pair_ieee, w.per);
-            }
+            if (MATH != 1 && fastdiv)
+                ring_walk_m<D, SEGW, PER>(L, lane, total, r_i, act, bmin,
+                                          bmax, smax, r, imove, 0, flag_el,
+                                          nearw, pair_fd, w.per);
+            else
+                ring_walk_m<D, SEGW, PER>(L, lane, total, r_i, act, bmin,
+                                          bmax, smax, r, imove, 0, flag_el,
+                                          nearw, pair_ieee, w.per);
             // ---- wall elements (boundary-integral Shepard) ------------------
             if (SHEP == 2 && __ballot(nearw) != 0) {
                 bool self_added = false;
                 bool unused = false;
                 const uint32_t total_el =
                     neighbour_table<D, PER>(w, c_i, L, lane, AQ_CELL_ELEM);
-                ring_walk_l<D, SEGW, LOOSE>(
+                ring_walk_m<D, SEGW, PER>(
                     L, lane, total_el, r_i, act && nearw, bmin, bmax, smax,
                     r, imove, 1, false, unused, [&](uint32_t j, uint32_t kl) {
                         const f3 r_ij = sub<D>(rjof(j, kl), r_i);
                         const float s = dot<D>(r_ij, r_ij);
-                        if (LOOSE && s > smax) return;
+                        if (s > smax) return;
                         const float q = sqrtf(s) / H;
                         const f3 n_j = ldv_o<D>(normal, j);
                         const f3 t_j = ldv_o<D>(tangent, j);
@@ -804,9 +894,9 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
                   int nrq, const uint32_t* __restrict__ olist,
                   uint32_t count_word)
 {
-    __shared__ WaveLds<SEGW, false> lds[WC_WAVES];
+    __shared__ WaveLds<SEGW> lds[WC_WAVES];
     const int lane = threadIdx.x & 63;
-    WaveLds<SEGW, false>& L = lds[threadIdx.x >> 6];
+    WaveLds<SEGW>& L = lds[threadIdx.x >> 6];
     if (w.status && (*w.status & 1u)) return;
     const uint32_t n_heads =
         olist ? uni(w.n_heads[count_word]) : uni(*w.n_heads);
@@ -854,13 +944,11 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
             if (nrq)
                 ring_walk<D, SEGW, NB>(
                     L, lane, total, r_i, act, bmin, bmax, smax, r, imove,
-                    Pol::KIND, false, unused,
-                    BatchPair<Pol, true>{ pol, i, r_i, st }, w.per);
+                    Pol::KIND, BatchPair<Pol, true>{ pol, i, r_i, st });
             else
                 ring_walk<D, SEGW, NB>(
                     L, lane, total, r_i, act, bmin, bmax, smax, r, imove,
-                    Pol::KIND, false, unused,
-                    BatchPair<Pol, false>{ pol, i, r_i, st }, w.per);
+                    Pol::KIND, BatchPair<Pol, false>{ pol, i, r_i, st });
             if (act) pol.finish(i, st);
             __builtin_amdgcn_wave_barrier();
         }
