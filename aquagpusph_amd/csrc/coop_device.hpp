@@ -61,6 +61,11 @@ template <int Q, int B, bool PER> struct CoopLds {
     uint32_t list[64 / Q][CAP];
     uint32_t owns[64 / Q];
     float4 shift[PER ? 27 : 1];
+    __device__ __forceinline__ void set_shift(int k, const float4& v)
+    {
+        shift[k] = v;
+    }
+    __device__ __forceinline__ float4 get_shift(int k) { return shift[k]; }
 };
 
 // Relative squared distances by v_mfma_f32_16x16x4_f32: with a point
@@ -234,7 +239,7 @@ coop_list_walk(CoopLds<Q, B, PER>& L, int lane, uint32_t total,
             PER ? (j | ((uint32_t)klj << PER_KL_SHIFT)) : j;
         if (cb + (uint32_t)lane < total) {
             if constexpr (PER) {
-                const float4 sh = L.shift[klj];
+                const float4 sh = L.get_shift(klj);
                 rj = per_shift<D>(rj, f3{ sh.x, sh.y, sh.z }, per);
             }
             is_el = (im_j == -3);

@@ -59,7 +59,7 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
     auto rjof = [&](uint32_t j, uint32_t kl) {
         f3 v = ldv_o<D>(r, j);
         if constexpr (PER) {
-            const float4 s = L.shift[kl];
+            const float4 s = L.get_shift((int)kl);
             v = per_shift<D>(v, f3{ s.x, s.y, s.z }, w.per);
         }
         return v;

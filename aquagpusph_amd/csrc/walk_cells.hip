@@ -62,24 +62,37 @@ __device__ __forceinline__ uint32_t next_cell(const WalkArgs& w,
 
 // Shared state of one wavefront of the fused walk: neighbour-cell table,
 // staged candidates (two chunks of 64, see dist_tile) and the ring of tested
-// chunks (candidate words, SEGW words of accept bits per lane).
+// chunks (SEGW words of accept bits per lane; positions and indices of their
+// candidates, with one chunk more for the survivors staged ahead).
 template <int SEGW, bool PER = false> struct RingLds {
+    static constexpr uint32_t NCH = SEGW / 2 + 1;  // chunks of `ring`
     uint32_t start[27];
     uint32_t cum[28];
     float4 stage[2][80];
-    uint32_t cand[SEGW * 32];
+    float4 ring[NCH * 64];
     uint32_t bits[SEGW][64];
-    // periodic box: the shift of each neighbour cell's particles
-    float4 shift[PER ? 27 : 1];
+    // periodic box: the shift of each neighbour cell's particles, in the
+    // gaps of the staged records
+    __device__ __forceinline__ float4* shift_slot(uint32_t k)
+    {
+        return &stage[k >> 4][20u * ((k >> 2) & 3u) + 16u + (k & 3u)];
+    }
+    __device__ __forceinline__ void set_shift(int k, const float4& v)
+    {
+        *shift_slot((uint32_t)k) = v;
+    }
+    __device__ __forceinline__ float4 get_shift(int k)
+    {
+        return *shift_slot((uint32_t)k);
+    }
 };
 
 // Walk the accepted candidates of one particle per lane.  `kind` selects
 // the candidates (0: fluid particles, imove == 1; 1: wall elements,
 // imove == -3); with kind 0 and `flag_el`, wall elements in range are also
-// tested and reported through `el_near`.  pair(j, kl) is called for the
-// accepted candidates of each lane in increasing candidate order; kl is the
-// neighbour-table entry the candidate came from (its shift in a periodic
-// walk; 0 otherwise).
+// tested and reported through `el_near`.  pair(j, r_j) is called for the
+// accepted candidates of each lane in increasing candidate order, r_j the
+// candidate's position (at its nearest image in a periodic box).
 //
 // (A branch-free variant, calling pair() on every lane at every step with a
 // dummy index on the idle lanes, measured 25% slower on the 3D dam break:
@@ -100,7 +113,10 @@ template <int SEGW, bool PER = false> struct RingLds {
 // more lines than the cache holds for 16 wavefronts.  3D dam break, 1.2 M /
 // 4.5 M particles, walk in us by survivors in the ring: 128: 1867 / 6439,
 // 192: 1816 / 6439, 256: 1789 / 6382, 384: 2099 / 7567, 512: 2359 / 8936
-// (two slots of 256 list entries, refilled whole: 2014 / 6924).
+// (two slots of 256 list entries, refilled whole: 2014 / 6924).  The
+// positions of the ring's candidates are kept in LDS beside their indices,
+// which takes the widest of the five gathers of a pair off the cache: 1592 /
+// 5534 with 256.  (39.8 KB per workgroup: four per CU, with 1 KB to spare.)
 //
 // Test: the squared distances of a chunk to the 64 particles by matrix
 // instructions (dist_tile), on coordinates relative to the box centre c:
@@ -149,6 +165,8 @@ ring_walk_m(RingLds<SEGW, PER>& L, int lane, uint32_t total, const f3& r_i,
     int kl = 0;        // per-lane cursor: neighbour cell of a candidate
     uint32_t nw = 0;   // next word to load (the current one is nw - 1)
     uint32_t bw = 0;   // remaining bits of the current word
+    constexpr uint32_t NCH = RingLds<SEGW, PER>::NCH;
+    uint32_t wb = NCH * 64 - 32;  // its first candidate's place in the ring
     uint32_t wt = 0;   // words tested
     uint32_t cb = 0;   // candidates read
     uint32_t ns = 0;   // survivors staged
@@ -160,6 +178,7 @@ ring_walk_m(RingLds<SEGW, PER>& L, int lane, uint32_t total, const f3& r_i,
         while (bw == 0 && nw < tw) {
             bw = L.bits[nw % RING][lane];
             nw++;
+            wb = wb == NCH * 64 - 32 ? 0u : wb + 32;
         }
     };
     // consume while no chunk can be refilled (a lane still reads from the
@@ -178,28 +197,28 @@ ring_walk_m(RingLds<SEGW, PER>& L, int lane, uint32_t total, const f3& r_i,
             if (bw != 0) {
                 const uint32_t b = __builtin_clz(bw);
                 bw ^= 0x80000000u >> b;
-                const uint32_t cw = L.cand[((nw - 1) % RING) * 32 + b];
-                if constexpr (PER)
-                    pair(cw & PER_J_MASK, cw >> PER_KL_SHIFT);
-                else
-                    pair(cw, 0u);
+                const float4 c = L.ring[wb + b];
+                pair(__float_as_uint(c.w), f3{ c.x, c.y, c.z });
             }
         }
         if (done) break;  // and no lane has a candidate left
-        // stage survivors up to a whole chunk (or the candidates' end)
+        // stage survivors up to a whole chunk (or the candidates' end); the
+        // ring has room for two (the oldest chunk and the one before it)
+        const uint32_t k0 = wt >> 1;  // the chunk
+        const uint32_t in0 = (k0 % NCH) * 64, in1 = ((k0 + 1) % NCH) * 64;
         while (ns < wt * 32 + 64 && cb < total) {
             const uint32_t t = cb + (uint32_t)lane;
             bool take = false, is_el = false;
-            uint32_t word = 0;
+            uint32_t j = 0;
+            f3 rj = { 0.f, 0.f, 0.f };
             float4 st = make_float4(0.f, 0.f, 0.f, 0.f);
             if (t < total) {
                 while (t >= L.cum[kl + 1]) kl++;
-                const uint32_t j = L.start[kl] + (t - L.cum[kl]);
-                f3 rj = ldv_o<D>(r, j);
+                j = L.start[kl] + (t - L.cum[kl]);
+                rj = ldv_o<D>(r, j);
                 const int im_j = ldi_o(imove, j);
-                word = PER ? (j | ((uint32_t)kl << PER_KL_SHIFT)) : j;
                 if constexpr (PER) {
-                    const float4 sh = L.shift[kl];
+                    const float4 sh = L.get_shift(kl);
                     rj = per_shift<D>(rj, f3{ sh.x, sh.y, sh.z }, per);
                 }
                 is_el = (im_j == -3);
@@ -226,9 +245,9 @@ ring_walk_m(RingLds<SEGW, PER>& L, int lane, uint32_t total, const f3& r_i,
                          (uint32_t)(tm >> 32),
                          __builtin_amdgcn_mbcnt_lo((uint32_t)tm, 0u));
             if (take) {
-                float4* sg = L.stage[(rank >> 6) & 1];
-                sg[dist_slot(rank & 63u)] = st;
-                *dist_word<4>(sg, rank & 63u) = word;
+                L.stage[(rank >> 6) & 1][dist_slot(rank & 63u)] = st;
+                L.ring[((rank >> 6) == k0 ? in0 : in1) + (rank & 63u)] =
+                    make_float4(rj.x, rj.y, rj.z, __uint_as_float(j));
             }
             if (!kind) {
                 uint64_t e = __ballot(take && is_el);
@@ -251,8 +270,7 @@ ring_walk_m(RingLds<SEGW, PER>& L, int lane, uint32_t total, const f3& r_i,
             // the chunk's accept bits: candidates 16 g .. in the upper (g
             // even) or lower half of word wt + g / 2
             const uint32_t hf = (wt >> 1) & 1;
-            float4* sg = L.stage[hf];
-            const float* row = dist_row(sg, lane);
+            const float* row = dist_row(L.stage[hf], lane);
             const float A[4] = { row[0], row[16], row[32], row[48] };
             const uint64_t valid =
                 have < 64 ? (1ull << have) - 1ull : ~0ull;
@@ -267,8 +285,6 @@ ring_walk_m(RingLds<SEGW, PER>& L, int lane, uint32_t total, const f3& r_i,
                 // one tile's results live at a time (registers)
                 __builtin_amdgcn_sched_barrier(0);
             }
-            L.cand[(wt % RING) * 32 + (uint32_t)lane] =
-                *dist_word<4>(sg, (uint32_t)lane);
             lds_order();
             const uint64_t em = hf ? elm[1] : elm[0];
             if (!kind && em != 0) {
@@ -595,15 +611,6 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
     const int lane = threadIdx.x & 63;
     const int wv = threadIdx.x >> 6;
     RingLds<SEGW, PER>& L = lds[wv];
-    // a candidate's position, at its nearest image in a periodic box
-    auto rjof = [&](uint32_t j, uint32_t kl) {
-        f3 v = ldv_o<D>(r, j);
-        if constexpr (PER) {
-            const float4 sh = L.shift[kl];
-            v = per_shift<D>(v, f3{ sh.x, sh.y, sh.z }, w.per);
-        }
-        return v;
-    };
     if (w.status && (*w.status & 1u)) return;
     const uint32_t n_heads = uni(*w.n_heads);
     const float eps = 1E-8f * H;
@@ -706,8 +713,8 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
             // terms are then +-0 (finite fields), and adding +-0 leaves the
             // sums unchanged, since they are never -0 (they start at +0, or
             // 1, and an exact cancellation rounds to +0).
-            auto pair_fd = [&](uint32_t j, uint32_t kl) {
-                const f3 r_ij = sub<D>(rjof(j, kl), r_i);
+            auto pair_fd = [&](uint32_t j, const f3& r_j) {
+                const f3 r_ij = sub<D>(r_j, r_i);
                 const float s = dot<D>(r_ij, r_ij);
                 const float qf = div_nr(sqrt_nr(s), RH);
                 float m_j = ldf_o(m, j);
@@ -725,12 +732,12 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
                     terms(std::false_type{}, r_ij, sqrtf(s) / H, m_j, rho_j,
                           p_j, u_ij, udr);
             };
-            auto pair_ieee = [&](uint32_t j, uint32_t kl) {
+            auto pair_ieee = [&](uint32_t j, const f3& r_j) {
                     if constexpr (FAST) {
                         // OpenCL C default accuracy: reciprocal-based
                         // division, hardware square root, contracted
                         // multiply-adds
-                        const f3 r_ij = sub<D>(rjof(j, kl), r_i);
+                        const f3 r_ij = sub<D>(r_j, r_i);
                         const float s = fdot<D>(r_ij, r_ij);
                         const float q = __builtin_amdgcn_sqrtf(s) * iH;
                         float m_j = ldf_o(m, j);
@@ -758,7 +765,7 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
                         if (LAPP) lp = fmaf(p_j - p_i, f_ij * irho_j, lp);
                         return;
                     }
-                    const f3 r_ij = sub<D>(rjof(j, kl), r_i);
+                    const f3 r_ij = sub<D>(r_j, r_i);
                     const float s = dot<D>(r_ij, r_ij);
                     const float q = sqrtf(s) / H;
                     float m_j = ldf_o(m, j);
@@ -786,8 +793,8 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
                     neighbour_table<D, PER>(w, c_i, L, lane, AQ_CELL_ELEM);
                 ring_walk_m<D, SEGW, PER>(
                     L, lane, total_el, r_i, act && nearw, bmin, bmax, smax,
-                    r, imove, 1, false, unused, [&](uint32_t j, uint32_t kl) {
-                        const f3 r_ij = sub<D>(rjof(j, kl), r_i);
+                    r, imove, 1, false, unused, [&](uint32_t j, const f3& r_j) {
+                        const f3 r_ij = sub<D>(r_j, r_i);
                         const float s = dot<D>(r_ij, r_ij);
                         if (s > smax) return;
                         const float q = sqrtf(s) / H;
@@ -1028,7 +1035,8 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
                     const uint32_t j = PER ? cw[0] & PER_J_MASK : cw[0];
                     auto c = pol.load(j);
                     if constexpr (PER) {
-                        const float4 sh = L.shift[cw[0] >> PER_KL_SHIFT];
+                        const float4 sh =
+                            L.get_shift((int)(cw[0] >> PER_KL_SHIFT));
                         c.r = per_shift<D>(c.r, f3{ sh.x, sh.y, sh.z },
                                            w.per);
                     }

@@ -91,7 +91,7 @@ __device__ __forceinline__ uint32_t neighbour_table(const WalkArgs& w,
         if constexpr (PER) {
             f3 sh;
             c = per_neighbour<D>(c_i, ci, cj, ck, w.n_cells, w.per, sh);
-            L.shift[lane] = make_float4(sh.x, sh.y, sh.z, 0.f);
+            L.set_shift(lane, make_float4(sh.x, sh.y, sh.z, 0.f));
         } else {
             c = c_i + (uint32_t)ci + (uint32_t)cj * nx +
                 (uint32_t)ck * nx * ny;
