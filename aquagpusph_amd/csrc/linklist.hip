@@ -731,7 +731,7 @@ void linklist_all(int dims, const float* r, uint32_t N, float* r_min,
 // ---- the link-list without allocation -------------------------------------
 // Scratch of aq_linklist_noalloc: the workspace aq_linklist takes as an
 // argument (min/max partials, the radix sort's key and value buffers, digit
-// counts and scan sums) for up to AQ_LINKLIST_NOALLOC_MAX_N particles, in a
+// counts and totals) for up to AQ_LINKLIST_NOALLOC_MAX_N particles, in a
 // file-scope device array.  Each GPU holds its own copy, at its own
 // address, until the process ends; host code uses that address, looked up
 // once per device, never the array's name.  Every call on one GPU shares

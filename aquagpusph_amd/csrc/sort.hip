@@ -2,16 +2,16 @@
 //
 // Replaces the reference RadixSort tool (aquagpusph/CalcServer/RadixSort.cpp
 // :129-303, kernels RadixSort.cl.in:35-323), which sorts 4-bit digits with
-// 1024 work-items that each scan a contiguous chunk serially.  Here each
-// pass is reduce-then-scan over tiles of 4096 keys:
-//   1. rs_hist    : per-tile digit histogram (wave-aggregated LDS counters),
-//                   stored digit-major so one exclusive scan yields, for each
-//                   (digit, tile), the first output slot;
-//   2. scan       : three-kernel exclusive scan of the digit-major table;
-//   3. rs_scatter : tiles re-read their keys in index order; a key's rank
-//                   among equal digits of its 256-key row comes from eight
-//                   wavefront ballots (match-any), rows are processed in
-//                   order, so equal digits keep their input order (stable).
+// 1024 work-items that each scan a contiguous chunk serially.  Here an array
+// of one workgroup's size is sorted by one launch (rs_small); beyond it each
+// pass is reduce-then-scan over tiles:
+//   1. rs_hist    : per-tile digit histogram (wave-aggregated LDS counters);
+//   2. rs_rows    : the first slot of each (digit, tile) within its digit and
+//                   the digits' totals (few tiles: rs_scatter adds the table
+//                   up itself, RS_DIRECT);
+//   3. rs_scatter : ranks the tile's keys, brings them into digit order in
+//                   LDS and writes each digit's run; the last pass writes the
+//                   inverse permutation as well.
 // No kernel waits on another workgroup, so every wave always finishes.
 #include <algorithm>
 
@@ -20,8 +20,6 @@
 namespace aq {
 
 constexpr int RS_BS = 256;  // threads per tile (4 wave64)
-constexpr int RS_IPT = 16;  // keys per thread
-constexpr int RS_TILE = RS_BS * RS_IPT;
 constexpr int SC_BS = 256;
 constexpr int SC_IPT = 4;
 constexpr int SC_TILE = SC_BS * SC_IPT;
@@ -39,67 +37,6 @@ __device__ __forceinline__ uint64_t match_digit(uint32_t d, uint64_t active)
         m &= bit ? bb : ~bb;
     }
     return m;
-}
-
-__global__ void __launch_bounds__(RS_BS)
-    rs_hist(const uint32_t* __restrict__ keys, uint32_t n, int shift,
-            uint32_t* __restrict__ counts, uint32_t ntiles)
-{
-    __shared__ uint32_t h[256];
-    const int tid = threadIdx.x;
-    h[tid] = 0;
-    __syncthreads();
-    const size_t base = (size_t)blockIdx.x * RS_TILE;
-    const uint64_t lt = (1ull << lane_id()) - 1ull;
-#pragma unroll 4
-    for (int it = 0; it < RS_IPT; it++) {
-        const size_t idx = base + (size_t)it * RS_BS + tid;
-        const bool valid = idx < n;
-        const uint32_t d = valid ? (keys[idx] >> shift) & 255u : 0u;
-        const uint64_t act = __ballot(valid);
-        const uint64_t peers = match_digit(d, act);
-        if (valid && (peers & lt) == 0)
-            atomicAdd(&h[d], (uint32_t)__popcll(peers));
-    }
-    __syncthreads();
-    counts[(size_t)tid * ntiles + blockIdx.x] = h[tid];
-}
-
-__global__ void __launch_bounds__(RS_BS)
-    rs_scatter(const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
-               uint32_t* __restrict__ kout, uint32_t* __restrict__ vout,
-               uint32_t n, int shift, const uint32_t* __restrict__ offs,
-               uint32_t ntiles)
-{
-    __shared__ uint32_t base[256];
-    __shared__ uint32_t wc[4][256];
-    const int tid = threadIdx.x;
-    const int w = tid >> 6;
-    const uint64_t lt = (1ull << lane_id()) - 1ull;
-    base[tid] = offs[(size_t)tid * ntiles + blockIdx.x];
-    const size_t tile = (size_t)blockIdx.x * RS_TILE;
-    for (int it = 0; it < RS_IPT; it++) {
-#pragma unroll
-        for (int k = 0; k < 4; k++) wc[k][tid] = 0;
-        __syncthreads();
-        const size_t idx = tile + (size_t)it * RS_BS + tid;
-        const bool valid = idx < n;
-        const uint32_t key = valid ? kin[idx] : 0u;
-        const uint32_t d = (key >> shift) & 255u;
-        const uint64_t act = __ballot(valid);
-        const uint64_t peers = match_digit(d, act);
-        const uint32_t rank = (uint32_t)__popcll(peers & lt);
-        if (valid && (peers & lt) == 0) wc[w][d] = (uint32_t)__popcll(peers);
-        __syncthreads();
-        if (valid) {
-            uint32_t pos = base[d] + rank;
-            for (int k = 0; k < w; k++) pos += wc[k][d];
-            kout[pos] = key;
-            vout[pos] = vin ? vin[idx] : (uint32_t)idx;
-        }
-        __syncthreads();
-        base[tid] += wc[0][tid] + wc[1][tid] + wc[2][tid] + wc[3][tid];
-    }
 }
 
 // ---- exclusive scan of uint32 ----------------------------------------------
@@ -212,14 +149,241 @@ void exclusive_scan(const uint32_t* in, uint32_t* out, uint32_t m,
                        sums);
 }
 
-// ---- permutations -----------------------------------------------------------
-__global__ void inverse_perm(const uint32_t* __restrict__ perm,
-                             uint32_t* __restrict__ inv, uint32_t n)
+// ---- radix sort --------------------------------------------------------------
+// Ranks a wavefront's IPT rows of 64 keys among its keys of equal digit, in
+// row and lane order (stable), counting them in wc (the wavefront's own
+// counters, zero at the start): a row's rank comes from eight ballots
+// (match-any), the counter carries the rows before it.  The wavefront's LDS
+// operations take effect in order, so no barrier is needed.
+template <int IPT>
+__device__ __forceinline__ void rank_rows(const uint32_t (&key)[IPT],
+                                          uint32_t nrow, int shift,
+                                          uint32_t* wc, uint32_t (&rank)[IPT])
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) inv[perm[i]] = i;
+    const uint32_t lane = lane_id();
+    const uint64_t lt = (1ull << lane) - 1ull;
+#pragma unroll
+    for (int k = 0; k < 4; k++) wc[k * 64 + lane] = 0;
+#pragma unroll
+    for (int it = 0; it < IPT; it++) {
+        const bool valid = (uint32_t)it * 64u + lane < nrow;
+        const uint32_t d = (key[it] >> shift) & 255u;
+        const uint64_t peers = match_digit(d, __ballot(valid));
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        const uint32_t before = wc[d];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        rank[it] = before + (uint32_t)__popcll(peers & lt);
+        if (valid && (peers & lt) == 0)
+            wc[d] = before + (uint32_t)__popcll(peers);
+    }
 }
 
+// keys of the calling wavefront's rows, of which the first `base` of the
+// array belong to others
+__device__ __forceinline__ uint32_t rows_left(uint32_t n, size_t base,
+                                              uint32_t most)
+{
+    return base >= n ? 0u : (uint32_t)min((size_t)most, (size_t)n - base);
+}
+
+// counts: digit-major rows of ntiles (rs_rows), or tile-major (direct)
+template <int IPT>
+__global__ void __launch_bounds__(RS_BS)
+    rs_hist(const uint32_t* __restrict__ keys, uint32_t n, int shift,
+            uint32_t* __restrict__ counts, uint32_t ntiles, int direct)
+{
+    __shared__ uint32_t h[256];
+    const int tid = threadIdx.x;
+    h[tid] = 0;
+    const size_t base = (size_t)blockIdx.x * (RS_BS * IPT);
+    const uint64_t lt = (1ull << lane_id()) - 1ull;
+    uint32_t key[IPT];
+#pragma unroll
+    for (int it = 0; it < IPT; it++) {
+        const size_t idx = base + (size_t)it * RS_BS + tid;
+        key[it] = idx < n ? keys[idx] : 0u;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < IPT; it++) {
+        const bool valid = base + (size_t)it * RS_BS + tid < n;
+        const uint32_t d = (key[it] >> shift) & 255u;
+        const uint64_t peers = match_digit(d, __ballot(valid));
+        if (valid && (peers & lt) == 0)
+            atomicAdd(&h[d], (uint32_t)__popcll(peers));
+    }
+    __syncthreads();
+    counts[direct ? (size_t)blockIdx.x * 256 + tid
+                  : (size_t)tid * ntiles + blockIdx.x] = h[tid];
+}
+
+// one workgroup per digit: exclusive scan of its row, total to totals[digit]
+__global__ void __launch_bounds__(RS_BS)
+    rs_rows(uint32_t* counts, uint32_t ntiles, uint32_t* __restrict__ totals)
+{
+    __shared__ uint32_t ws[RS_BS / 64];
+    uint32_t* row = counts + (size_t)blockIdx.x * ntiles;
+    uint32_t carry = 0;
+    for (uint32_t b = 0; b < ntiles; b += RS_BS) {
+        const uint32_t i = b + threadIdx.x;
+        const uint32_t v = i < ntiles ? row[i] : 0u;
+        uint32_t tot;
+        const uint32_t ex = block_excl_scan(v, ws, &tot);
+        if (i < ntiles) row[i] = carry + ex;
+        carry += tot;
+    }
+    if (threadIdx.x == 0) totals[blockIdx.x] = carry;
+}
+
+template <int IPT>
+__global__ void __launch_bounds__(RS_BS)
+    rs_scatter(const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
+               uint32_t* __restrict__ kout, uint32_t* __restrict__ vout,
+               uint32_t* __restrict__ inv, uint32_t n, int shift,
+               const uint32_t* __restrict__ counts,
+               const uint32_t* __restrict__ totals, uint32_t ntiles,
+               int direct)
+{
+    constexpr uint32_t TILE = RS_BS * IPT;
+    __shared__ uint32_t wc[RS_BS / 64][256];
+    __shared__ uint32_t dbase[256];
+    __shared__ uint32_t ws[RS_BS / 64];
+    __shared__ uint32_t sk[TILE], sv[TILE];
+    const int tid = threadIdx.x;
+    const uint32_t w = (uint32_t)tid >> 6, lane = lane_id();
+    // a wavefront ranks a contiguous part of the tile
+    const size_t tile = (size_t)blockIdx.x * TILE;
+    const size_t wbase = tile + (size_t)w * (64 * IPT);
+    const uint32_t nrow = rows_left(n, wbase, 64 * IPT);
+    uint32_t key[IPT], val[IPT], rank[IPT];
+#pragma unroll
+    for (int it = 0; it < IPT; it++) {
+        const uint32_t o = (uint32_t)it * 64u + lane;
+        key[it] = o < nrow ? kin[wbase + o] : 0u;
+        val[it] = (vin && o < nrow) ? vin[wbase + o] : (uint32_t)wbase + o;
+    }
+    // the digit's total, and its keys in the tiles before this one
+    uint32_t tot = 0, pre = 0;
+    if (direct) {
+#pragma unroll 8
+        for (uint32_t t = 0; t < ntiles; t++) {
+            const uint32_t c = counts[(size_t)t * 256 + tid];
+            tot += c;
+            pre += t < blockIdx.x ? c : 0u;
+        }
+    } else {
+        tot = totals[tid];
+        pre = counts[(size_t)tid * ntiles + blockIdx.x];
+    }
+    rank_rows<IPT>(key, nrow, shift, wc[w], rank);
+    uint32_t all;
+    const uint32_t start = block_excl_scan(tot, ws, &all) + pre;
+    uint32_t c[RS_BS / 64], cnt = 0;
+#pragma unroll
+    for (int k = 0; k < RS_BS / 64; k++) {
+        c[k] = cnt;
+        cnt += wc[k][tid];
+    }
+    const uint32_t ls = block_excl_scan(cnt, ws, &all);
+#pragma unroll
+    for (int k = 0; k < RS_BS / 64; k++) wc[k][tid] = ls + c[k];
+    dbase[tid] = start - ls;
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < IPT; it++) {
+        if ((uint32_t)it * 64u + lane < nrow) {
+            const uint32_t q = wc[w][(key[it] >> shift) & 255u] + rank[it];
+            sk[q] = key[it];
+            sv[q] = val[it];
+        }
+    }
+    __syncthreads();
+    const uint32_t nt = rows_left(n, tile, TILE);
+#pragma unroll
+    for (int it = 0; it < IPT; it++) {
+        const uint32_t q = (uint32_t)it * RS_BS + tid;
+        if (q < nt) {
+            const uint32_t k = sk[q], v = sv[q];
+            const uint32_t pos = dbase[(k >> shift) & 255u] + q;
+            kout[pos] = k;
+            vout[pos] = v;
+            if (inv) inv[v] = pos;
+        }
+    }
+}
+
+// All passes over at most 1024 * IPT keys by one workgroup, the keys in
+// registers and reordered through LDS.
+constexpr int RS_SMALL_BS = 1024;
+template <int IPT>
+__global__ void __launch_bounds__(RS_SMALL_BS)
+    rs_small(uint32_t* keys, uint32_t* __restrict__ perm,
+             uint32_t* __restrict__ inv, uint32_t n, int passes)
+{
+    constexpr int NW = RS_SMALL_BS / 64;
+    __shared__ uint32_t wc[NW][256];
+    __shared__ uint32_t ws[NW];
+    __shared__ uint32_t sk[RS_SMALL_BS * IPT], sv[RS_SMALL_BS * IPT];
+    const int tid = threadIdx.x;
+    const uint32_t w = (uint32_t)tid >> 6, lane = lane_id();
+    const uint32_t wbase = w * (64 * IPT);
+    const uint32_t nrow = rows_left(n, wbase, 64 * IPT);
+    uint32_t key[IPT], val[IPT], rank[IPT];
+#pragma unroll
+    for (int it = 0; it < IPT; it++) {
+        const uint32_t o = (uint32_t)it * 64u + lane;
+        key[it] = o < nrow ? keys[wbase + o] : 0u;
+        val[it] = wbase + o;
+    }
+    for (int p = 0; p < passes; p++) {
+        const int shift = 8 * p;
+        rank_rows<IPT>(key, nrow, shift, wc[w], rank);
+        __syncthreads();
+        uint32_t c[NW], cnt = 0;
+        if (tid < 256) {
+#pragma unroll
+            for (int k = 0; k < NW; k++) {
+                c[k] = cnt;
+                cnt += wc[k][tid];
+            }
+        }
+        uint32_t all;
+        const uint32_t ls = block_excl_scan(cnt, ws, &all);
+        if (tid < 256) {
+#pragma unroll
+            for (int k = 0; k < NW; k++) wc[k][tid] = ls + c[k];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int it = 0; it < IPT; it++) {
+            if ((uint32_t)it * 64u + lane < nrow) {
+                const uint32_t q = wc[w][(key[it] >> shift) & 255u] + rank[it];
+                sk[q] = key[it];
+                sv[q] = val[it];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int it = 0; it < IPT; it++) {
+            const uint32_t o = (uint32_t)it * 64u + lane;
+            if (o < nrow) {
+                key[it] = sk[wbase + o];
+                val[it] = sv[wbase + o];
+            }
+        }
+    }
+#pragma unroll
+    for (int it = 0; it < IPT; it++) {
+        const uint32_t o = (uint32_t)it * 64u + lane;
+        if (o < nrow) {
+            keys[wbase + o] = key[it];
+            perm[wbase + o] = val[it];
+            if (inv) inv[val[it]] = wbase + o;
+        }
+    }
+}
+
+// ---- permutations -----------------------------------------------------------
 template <typename T>
 __global__ void permute_k(const T* __restrict__ src, T* __restrict__ dst,
                           const uint32_t* __restrict__ perm, uint32_t n)
@@ -231,52 +395,100 @@ __global__ void permute_k(const T* __restrict__ src, T* __restrict__ dst,
 // ---- driver -------------------------------------------------------------
 static inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
+// Largest array one workgroup sorts: launches bound the short sorts (two or
+// three a pass).  A copy and a sort of uniform keys, us, one launch / passes
+// of two: 500 keys of 8 bits 8.5 / 17.0, 2000 of 12 bits 9.5 / 23.4, 4000 of
+// 16 bits 13.2 / 23.9, 8000 21.4 / 24.1.  (Tiles of 4096 keys ranked row by
+// row between barriers and scattered unordered, three scan launches and an
+// inverse permutation of its own took 20.2, 38.8, 49.0 and 54.9.)
+constexpr uint32_t RS_SMALL = 8 * RS_SMALL_BS;
+// Tiles up to which rs_scatter adds up the table of counts itself, a
+// coalesced column walk that costs less than the launch of rs_rows: 65 k keys
+// of 20 bits 34.5 / 36.4 us, 131 k 41.6 / 43.4.
+constexpr uint32_t RS_DIRECT = 64;
+
+// Keys per thread of a tile of n keys.  Short tiles keep every CU busy, long
+// ones write longer runs and shorter tables.  Copy and sort, us, with 4 or 8
+// keys per thread / with twice as many (with the earlier passes): 131 k keys
+// of 20 bits 41.6 / 51.5 (112.7), 1 M 70.1 / 95.3 (127.4), 4 M 185.8 / 162.8
+// (297.1), 4 M of 24 bits 199.0 / 169.8 (339.1).  A pass of 4 M keys moves
+// 84 MB, 18 us at the rate of a large copy; beyond that it is the scattered
+// runs, of 16 keys (64 B) for uniform digits.
+static inline int rs_ipt(uint32_t n)
+{
+    return n <= 65536u ? 4 : n <= 2097152u ? 8 : 16;
+}
+
 size_t radix_sort_workspace(uint32_t n)
 {
-    const size_t nt = blocks_for(n, RS_TILE);
-    const size_t m = nt * 256;
-    return align256((size_t)n * 4) * 2 + align256(m * 4) +
-           align256(scan_workspace((uint32_t)m));
+    const size_t nt = blocks_for(n, RS_BS * rs_ipt(n));
+    return align256((size_t)n * 4) * 2 + align256(nt * 256 * 4) +
+           align256(256 * 4);
 }
 
 void radix_sort(uint32_t* keys, uint32_t* perm, uint32_t* inv, uint32_t n,
                 unsigned key_bits, void* workspace, hipStream_t s)
 {
     if (n == 0) return;
-    const uint32_t nt = blocks_for(n, RS_TILE);
-    const uint32_t m = nt * 256;
+    const int passes = key_bits == 0 ? 1 : (int)((key_bits + 7) / 8);
+    if (n <= RS_SMALL) {
+#define AQ_RS(IPT)                                                             \
+    hipLaunchKernelGGL(rs_small<IPT>, dim3(1), dim3(RS_SMALL_BS), 0, s, keys,  \
+                       perm, inv, n, passes)
+        if (n <= 1 * RS_SMALL_BS) AQ_RS(1);
+        else if (n <= 2 * RS_SMALL_BS) AQ_RS(2);
+        else if (n <= 4 * RS_SMALL_BS) AQ_RS(4);
+        else AQ_RS(8);
+#undef AQ_RS
+        return;
+    }
+    const int ipt = rs_ipt(n);
+    const uint32_t nt = blocks_for(n, RS_BS * ipt);
+    const int direct = nt <= RS_DIRECT;
     char* w = (char*)workspace;
     uint32_t* kb = (uint32_t*)w;
     w += align256((size_t)n * 4);
     uint32_t* vb = (uint32_t*)w;
     w += align256((size_t)n * 4);
     uint32_t* counts = (uint32_t*)w;
-    w += align256((size_t)m * 4);
-    uint32_t* sums = (uint32_t*)w;
-    const int passes = key_bits == 0 ? 1 : (int)((key_bits + 7) / 8);
-    // The keys alternate between kb (even passes: the first cannot write
-    // keys in place) and keys; the values between vb and perm, chosen so
-    // that the last pass writes perm (the first pass reads no values).
-    uint32_t *kin = keys, *vin = nullptr, *kout = kb, *vout = nullptr;
+    w += align256((size_t)nt * 256 * 4);
+    uint32_t* totals = (uint32_t*)w;
+    // The keys alternate between kb and keys, ending in keys; of three passes
+    // the first writes them into inv, which only the last pass fills.  The
+    // values alternate between vb and perm, chosen so that the last pass
+    // writes perm (the first pass reads no values).
+    uint32_t *kin = keys, *vin = nullptr;
     for (int p = 0; p < passes; p++) {
-        const int shift = 8 * p;
-        kout = (p % 2 == 0) ? kb : keys;
-        vout = ((passes - 1 - p) % 2 == 0) ? perm : vb;
-        hipLaunchKernelGGL(rs_hist, dim3(nt), dim3(RS_BS), 0, s, kin, n,
-                           shift, counts, nt);
-        exclusive_scan(counts, counts, m, sums, s);
-        hipLaunchKernelGGL(rs_scatter, dim3(nt), dim3(RS_BS), 0, s, kin, vin,
-                           kout, vout, n, shift, counts, nt);
+        const int shift = 8 * p, left = passes - 1 - p;
+        uint32_t* kout = left % 2 == 0 ? keys : kb;
+        if (passes % 2 == 1) {
+            if (passes == 3 && inv) kout = p == 0 ? inv : p == 1 ? kb : keys;
+            else kout = p % 2 == 0 ? kb : keys;
+        }
+        uint32_t* vout = left % 2 == 0 ? perm : vb;
+        uint32_t* iout = left == 0 ? inv : nullptr;
+#define AQ_RS(IPT)                                                             \
+    do {                                                                       \
+        hipLaunchKernelGGL(rs_hist<IPT>, dim3(nt), dim3(RS_BS), 0, s, kin, n,  \
+                           shift, counts, nt, direct);                         \
+        if (!direct)                                                           \
+            hipLaunchKernelGGL(rs_rows, dim3(256), dim3(RS_BS), 0, s, counts,  \
+                               nt, totals);                                    \
+        hipLaunchKernelGGL(rs_scatter<IPT>, dim3(nt), dim3(RS_BS), 0, s, kin,  \
+                           vin, kout, vout, iout, n, shift, counts, totals,    \
+                           nt, direct);                                        \
+    } while (0)
+        if (ipt == 4) AQ_RS(4);
+        else if (ipt == 8) AQ_RS(8);
+        else AQ_RS(16);
+#undef AQ_RS
         kin = kout;
         vin = vout;
     }
-    // the sorted keys are in kb after an odd number of passes
+    // one pass (or three without an inverse): the sorted keys are in kb
     if (kin != keys)
         AQ_HIP(hipMemcpyAsync(keys, kin, (size_t)n * 4,
                               hipMemcpyDeviceToDevice, s));
-    if (inv)
-        hipLaunchKernelGGL(inverse_perm, dim3(blocks_for(n, 256)), dim3(256),
-                           0, s, perm, inv, n);
 }
 
 struct alignas(16) Words8 {

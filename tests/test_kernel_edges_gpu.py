@@ -47,6 +47,40 @@ def test_ihoc_table_of_wide_grids(cuda, cells, cap):
     assert (got[cells:] == -7).all()
 
 
+# one workgroup's sizes, the tile sizes and their remainders, the line of the
+# separate scan, and one to four passes (three write through the inverse)
+@pytest.mark.parametrize("bits", [4, 16, 20, 32])
+@pytest.mark.parametrize("n", [1, 63, 1024, 1025, 2049, 4097, 8192, 8193,
+                               65536, 65537, 131072, 131073, 2_097_152,
+                               2_097_153])
+def test_radix_sort_edges(cuda, n, bits):
+    """Keys, permutation and its inverse (with and without it asked for)
+    against a stable sort of the digits in use, whole passes of 8 bits."""
+    L = _lib.lib()
+    rng = np.random.default_rng(n + bits)
+    keys = rng.integers(0, 1 << 32, n, dtype=np.uint32)
+    keys[n // 3: 2 * n // 3] &= np.uint32(0xFF00FF0F)
+    mask = np.uint32((1 << (8 * ((bits + 7) // 8))) - 1)
+    want = np.argsort(keys & mask, kind="stable").astype(np.uint32)
+    size = int(L.aq_radix_sort_workspace(ctypes.c_uint32(n)))
+    for with_inv in (True, False):
+        kd = _dev(keys.view(np.int32))
+        pd, iv = (torch.full((n + 1,), -7, dtype=torch.int32, device="cuda")
+                  for _ in range(2))
+        ws = torch.full((size + 64,), 123, dtype=torch.uint8, device="cuda")
+        _lib.call("aq_radix_sort", _dp(kd), _dp(pd),
+                  _dp(iv) if with_inv else None, n, bits, _dp(ws), _stream())
+        np.testing.assert_array_equal(pd[:n].cpu().numpy(), want)
+        np.testing.assert_array_equal(kd.cpu().numpy().view(np.uint32),
+                                      keys[want])
+        if with_inv:
+            inv = np.empty(n, np.int32)
+            inv[want] = np.arange(n)
+            np.testing.assert_array_equal(iv[:n].cpu().numpy(), inv)
+        assert int(pd[n]) == -7 and int(iv[n]) == -7
+        assert bool((ws[size:] == 123).all())
+
+
 def _run(tmp_path, case, presets, tag, steps=3):
     from aquagpusph_amd import casefiles
     from aquagpusph_amd.sim import Simulation
