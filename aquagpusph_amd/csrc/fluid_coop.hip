@@ -278,24 +278,24 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
 // one lane / 4 lanes / 16 lanes, on dam breaks with their walls:
 //   2D      2 k 107 / 34 / 27     8 k 104 / 35 / 28    31 k 101 / 38 / 45
 //         184 k 185 / 92 / 159   1.1 M 820 / 435 / 869
-//   3D      9 k 513 / 120 / 71   20 k 532 / 126 / 115   38 k 533 / 146 / 162
-//         135 k 634 / 326 / 440  240 k 651 / 535 / 714  394 k 880 / 791 / -
-//         627 k 1144 / 1269 / -
+//   3D     11 k - / 114 / 72     23 k - / 128 / 122     40 k - / 139 / 158
+//         135 k 487 / 301 / -    240 k 502 / 497 / -    314 k 534 / 635 / -
+//         394 k 705 / 747 / -    764 k 1109 / 1381 / -
 // A 2D cell has 16 particles, so four lanes each fill a wavefront at any
 // size; a 3D cell has 64, and one lane each wins once the cells fill the
-// chip: 4096 wavefronts, 262 k fluid particles, where four still gain on a
-// flow out of lattice order and lose on the lattice (periodic cube of 262 k:
-// 764 / 669 and 584 / 633).  The
-// compensated sums (math == 2) take their six operations per term on every
-// lane of the group, which moves that line down (135 k 693 / 455, 240 k
-// 746 / 760); 16 lanes pay it 16 times (2D 8 k 109 / 39 / 37, 31 k 107 / 44
-// / 72; 3D 9 k 558 / 154 / 114, 20 k 576 / 165 / 192).
+// chip: 4096 wavefronts, 262 k fluid particles (periodic cube of 262 k on the
+// lattice 467 / 583, out of lattice order 846 / 943; of 195 k 778 / 663 and
+// 873 / 729).  The compensated sums (math == 2) take their six operations per
+// term on every lane of the group, which moves that line down (135 k on the
+// lattice 503 / 503, out of it 888 / 819; 193 k 502 / 782 and 902 / 1186); 16
+// lanes pay it 16 times (2D 8 k 109 / 39 / 37, 31 k 107 / 44 / 72; 3D 11 k
+// - / 147 / 111, 23 k - / 171 / 242).
 int fluid_coop_lanes(int dims, uint32_t N, int math)
 {
     const bool comp = math == 2;
     if (dims == 2) return N <= (comp ? 8000u : 16000u) ? 16 : 4;
     if (N <= (comp ? 12000u : 24000u)) return 16;
-    return N <= (comp ? 200000u : 250000u) ? 4 : 0;
+    return N <= (comp ? 150000u : 250000u) ? 4 : 0;
 }
 
 void launch_fluid_coop(int dims, int shep, bool lapp, int q,

@@ -11,8 +11,8 @@
 //
 // The per-particle kernels are bound by latency and divergence: each lane
 // reads its own candidates one at a time (256 accepted of 1728 in 3D).  At
-// 150 k particles in 3D: Shepard 841 -> 425 us, interactions 1278 ->
-// 555 us, lap p 935 -> 448 us.
+// 150 k particles in 3D: Shepard 841 -> 376 us, interactions 1278 ->
+// 523 us, lap p 935 -> 412 us.
 #include "aq_device.hpp"
 #include "aq_internal.hpp"
 #include "coop_device.hpp"

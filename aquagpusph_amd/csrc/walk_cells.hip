@@ -4,17 +4,18 @@
 // per lane); the candidates of the 27 (3D) / 9 (2D) neighbour cells are
 // enumerated in the reference order (x offset outermost, then y, then z;
 // sorted index inside a cell, types/3D.h:197-219), which is the same list
-// for every particle of the cell.  The list is cut in segments of SEG
-// candidates, tested into a ring of two LDS slots:
+// for every particle of the cell.  The list is staged 64 candidates at a time
+// and goes through a ring:
 //
-//   test     the lanes load 64 candidates at a time (coalesced) into LDS;
-//            the candidate loop reads them back by broadcast and every lane
-//            shifts in one accept bit per candidate (q < 2 and the wanted
-//            particle type);
+//   test     the lanes load 64 candidates (coalesced) into LDS, those out of
+//            reach of the wave's box are dropped, and chunks of 64 survivors
+//            are tested against the 64 particles by matrix instructions
+//            (dist_tile), which leave each lane a word of accept bits per 32
+//            candidates (q < 2 and the wanted particle type);
 //   consume  every lane walks its own accepted candidates in increasing
-//            order and evaluates the pair terms.  A lane that finishes a
-//            segment goes on with the next one while slower lanes finish
-//            theirs; the oldest slot is refilled once no lane needs it.
+//            order and evaluates the pair terms.  Lanes run ahead as far as
+//            the ring has been tested; the oldest chunk is replaced once no
+//            lane needs it.
 //
 // The fluid sums (grad p, lap u, div u, lap p, and the cfd Shepard sum) and
 // the boundary-integral Shepard sum take their terms from disjoint candidate
