@@ -394,7 +394,7 @@ def main():
         "peak_non_packed": PEAK_FP32_NONPACKED_TFLOPS,
         "frac_non_packed": (achieved / PEAK_FP32_NONPACKED_TFLOPS
                             if flops else None),
-        "note": "FP32 vector ALU work, no matrix instructions (bound: the "
+        "note": "FP32 vector ALU work, distance tests on FP32 matrix instructions (bound: the "
                 "VALU). peak is the published MI355X FP32 vector figure, "
                 "which counts packed FP32; this build emits none, so "
                 "peak_non_packed (one FMA per lane and cycle) is the "
