@@ -414,16 +414,28 @@ constexpr uint32_t RS_DIRECT = 64;
 // (297.1), 4 M of 24 bits 199.0 / 169.8 (339.1).  A pass of 4 M keys moves
 // 84 MB, 18 us at the rate of a large copy; beyond that it is the scattered
 // runs, of 16 keys (64 B) for uniform digits.
+constexpr uint32_t RS_IPT4 = 65536, RS_IPT8 = 2097152;
 static inline int rs_ipt(uint32_t n)
 {
-    return n <= 65536u ? 4 : n <= 2097152u ? 8 : 16;
+    return n <= RS_IPT4 ? 4 : n <= RS_IPT8 ? 8 : 16;
 }
 
-size_t radix_sort_workspace(uint32_t n)
+// What a sort of exactly n keys uses
+static size_t rs_bytes(uint32_t n)
 {
     const size_t nt = blocks_for(n, RS_BS * rs_ipt(n));
     return align256((size_t)n * 4) * 2 + align256(nt * 256 * 4) +
            align256(256 * 4);
+}
+
+// The table of counts halves beyond each line of rs_ipt, so just above one a
+// sort uses less than at it; a workspace holds every sort of up to n keys.
+size_t radix_sort_workspace(uint32_t n)
+{
+    size_t b = rs_bytes(n);
+    for (const uint32_t line : { RS_IPT4, RS_IPT8 })
+        if (n > line) b = std::max(b, rs_bytes(line));
+    return b;
 }
 
 void radix_sort(uint32_t* keys, uint32_t* perm, uint32_t* inv, uint32_t n,

@@ -102,7 +102,8 @@ AQ_API int aq_linklist(int dims, const float* r, uint32_t N, float* r_min,
                        uint32_t* id_unsorted, uint32_t* id_sorted,
                        uint32_t* ihoc, uint32_t ihoc_capacity,
                        uint32_t* status, void* workspace, void* stream);
-/* Bytes of device workspace aq_linklist / aq_linklist_grid need for N. */
+/* Bytes of device workspace aq_linklist / aq_linklist_grid need for up to N
+ * particles (never fewer for a larger N). */
 AQ_API size_t aq_linklist_workspace(uint32_t N);
 
 /* aq_linklist without a workspace argument and without any allocation.
@@ -129,10 +130,12 @@ AQ_API int aq_linklist_noalloc(int dims, const float* r, uint32_t N,
  * (RadixSort::_execute, RadixSort.cpp:129-303).  keys is sorted in place;
  * perm[k] = original index of sorted key k (id_unsorted); inv_perm[perm[k]]
  * = k (id_sorted, RadixSort.cl.in:313-323).  inv_perm may be NULL.
- * workspace: aq_radix_sort_workspace(n). */
+ * workspace: aq_radix_sort_workspace(n) bytes, or those of a larger count. */
 AQ_API int aq_radix_sort(uint32_t* keys, uint32_t* perm, uint32_t* inv_perm,
                          uint32_t n, unsigned key_bits, void* workspace,
                          void* stream);
+/* Bytes of device workspace for sorts of up to n keys (never fewer for a
+ * larger n). */
 AQ_API size_t aq_radix_sort_workspace(uint32_t n);
 /* Key bits the reference processes for max_val (RadixSort.cpp:152-176). */
 AQ_API unsigned aq_radix_key_bits(uint64_t max_val);

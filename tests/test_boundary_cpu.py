@@ -29,6 +29,21 @@ def test_error_reporting_without_gpu():
     assert L.aq_strerror(-6) == b"assertion failed"
 
 
+@pytest.mark.parametrize("fn", ["aq_radix_sort_workspace",
+                                "aq_linklist_workspace"])
+def test_workspace_holds_every_shorter_sort(fn):
+    """A workspace sized for n serves any smaller count: its size never
+    falls as n grows, the lines where the sort's tiles double among them
+    (65536 and 2097152 keys)."""
+    f = getattr(_lib.lib(), fn)
+    ns = sorted({n for c in (1024, 8192, 65536, 131072, 2097152)
+                 for n in [*range(max(1, c - 300), c + 300),
+                           *range(c, c + 80000, 251)]})
+    sizes = [f(n) for n in ns]
+    assert all(a <= b for a, b in zip(sizes, sizes[1:]))
+    assert f(0) <= sizes[0] and f(ctypes.c_uint32(2 ** 32 - 1)) > sizes[-1]
+
+
 def _resolve(xml, dims):
     L = _lib.lib()
     L.aq_xml_resolve.argtypes = [ctypes.c_char_p, ctypes.c_int,

@@ -81,6 +81,27 @@ def test_radix_sort_edges(cuda, n, bits):
         assert bool((ws[size:] == 123).all())
 
 
+@pytest.mark.parametrize("n,most", [(65536, 65537), (65000, 65600),
+                                    (2_097_152, 2_097_153),
+                                    (2_097_000, 2_100_000)])
+def test_radix_sort_in_a_larger_sorts_workspace(cuda, n, most):
+    """A sort of n keys in the workspace of a sort of `most`, across the
+    lines where the tiles double: nothing behind the workspace is written."""
+    f = _lib.lib().aq_radix_sort_workspace
+    # allocated so that even a sort that overran it would stay in bounds
+    size, room = f(most), max(f(most), f(n)) + 64
+    keys = np.random.default_rng(n).integers(0, 1 << 20, n, dtype=np.uint32)
+    want = np.argsort(keys, kind="stable").astype(np.uint32)
+    kd = _dev(keys.view(np.int32))
+    pd, iv = (torch.empty(n, dtype=torch.int32, device="cuda")
+              for _ in range(2))
+    ws = torch.full((room,), 123, dtype=torch.uint8, device="cuda")
+    _lib.call("aq_radix_sort", _dp(kd), _dp(pd), _dp(iv), n, 20, _dp(ws),
+              _stream())
+    np.testing.assert_array_equal(pd.cpu().numpy(), want)
+    assert bool((ws[size:] == 123).all())
+
+
 def _run(tmp_path, case, presets, tag, steps=3):
     from aquagpusph_amd import casefiles
     from aquagpusph_amd.sim import Simulation
