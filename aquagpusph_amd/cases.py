@@ -139,8 +139,8 @@ def dam_break(dims, dr, L=None, D=0.6, B=0.6, H=0.3, W=0.6, hfac=2.0,
     if tait_gamma is None:
         rho = refd + press / cs ** 2
     else:
-        B = refd * cs ** 2 / tait_gamma
-        rho = refd * (press / B + 1.0) ** (1.0 / tait_gamma)
+        bulk = refd * cs ** 2 / tait_gamma  # (B is the column's width)
+        rho = refd * (press / bulk + 1.0) ** (1.0 / tait_gamma)
     rho[nf:] = refd
     m = np.empty(N)
     m[:nf] = refd * dr ** dims

@@ -124,3 +124,24 @@ def test_tait_wall_inverse_returns_the_density():
     np.testing.assert_allclose(p[el], p_true[el], rtol=1e-13)
     np.testing.assert_allclose(r_out[el], rho[el], rtol=1e-13)
     np.testing.assert_array_equal(r_out[~el], 5.0)
+
+
+@pytest.mark.parametrize("dims,bc", [(2, "BI"), (3, "BI"), (2, "GP")])
+def test_tait_dam_break_differs_in_its_density_only(dims, bc):
+    """cases.dam_break with tait_gamma: the tank, its domain box and every
+    parameter of the linear case; the water's density by the Tait law."""
+    from aquagpusph_amd import cases
+    lin = cases.dam_break(dims, 0.05, bc=bc)
+    tait = cases.dam_break(dims, 0.05, bc=bc, tait_gamma=7.0)
+    assert tait["params"] == lin["params"]
+    assert tait.keys() == lin.keys()
+    for k, v in lin.items():
+        if isinstance(v, np.ndarray) and k != "rho":
+            np.testing.assert_array_equal(tait[k], v, err_msg=k)
+    cs, refd = lin["params"]["cs"], lin["params"]["refd"][0]
+    nf = lin["n_fluid"]
+    press = (lin["rho"][:nf] - refd) * cs ** 2
+    np.testing.assert_allclose(
+        tait["rho"][:nf], refd * (press * 7.0 / (refd * cs ** 2) + 1) **
+        (1 / 7.0), rtol=1e-12)
+    np.testing.assert_array_equal(tait["rho"][nf:], lin["rho"][nf:])
