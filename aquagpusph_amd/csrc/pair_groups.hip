@@ -93,9 +93,10 @@ __device__ __forceinline__ uint32_t run_table(const RunArgs& w, uint32_t c_i,
 }
 
 // Policies: KIND of the candidates (coop_list_walk), owner(im), State,
-// init(i, st), load(j) (Cand: position r, mass m, ...), term(cand, r_ij, s,
-// st) (carries the mass as a factor), add_group<Q>(st, term), finish(i, st);
-// NO_SELF: a particle is not its own candidate.
+// init(i, st), load(j) (Cand: position r, ...), term(cand, r_ij, s, st),
+// add_group<Q>(st, term), finish(i, st); none(): the term of a lane without
+// a candidate, -0 (x + -0 is x for every x); NO_SELF: a particle is not its
+// own candidate.
 template <int D, int Q, class Pol>
 __global__ void __launch_bounds__(64 * WC_WAVES)
     run_group_k(Pol pol, const int* __restrict__ imove,
@@ -139,13 +140,17 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
             typename Pol::Term t = Pol::none();
             if ((uint32_t)q < n) {
                 const uint32_t j = cw[0];
-                typename Pol::Cand cd = pol.load(j);
+                const typename Pol::Cand cd = pol.load(j);
                 const f3 r_ij = sub<D>(cd.r, r_i);
                 const float s = dot<D>(r_ij, r_ij);
-                // the walk's test accepts a thin shell beyond: no mass (a
-                // select, so that every load of the pair is issued at once)
-                if (s > smax || (Pol::NO_SELF && j == i)) cd.m = 0.f;
+                // the walk's test accepts a thin shell beyond: such a
+                // candidate adds nothing, whatever its fields hold (the term
+                // is selected, so that every load of the pair is issued at
+                // once)
+                const bool out =
+                    (s > smax) | (Pol::NO_SELF && j == i);
                 t = pol.term(cd, r_ij, s, st);
+                if (out) t = Pol::none();
             }
             pol.template add_group<Q>(st, t);
         };
@@ -193,7 +198,7 @@ template <int D, int K> struct PolShepard {
     {
         return kernelW<D>(sqrtf(s) / H) * CONW * c.m / c.rho;
     }
-    __device__ static Term none() { return 0.f; }
+    __device__ static Term none() { return -0.f; }
     template <int Q>
     __device__ void add_group(State& st, const Term& t) const
     {
@@ -254,7 +259,7 @@ template <int D> struct PolInteractions {
     }
     __device__ static Term none()
     {
-        return Term{ f3{ 0.f, 0.f, 0.f }, f3{ 0.f, 0.f, 0.f }, 0.f };
+        return Term{ f3{ -0.f, -0.f, -0.f }, f3{ -0.f, -0.f, -0.f }, -0.f };
     }
     template <int Q>
     __device__ void add_group(State& st, const Term& t) const
@@ -307,7 +312,7 @@ template <int D> struct PolLapP {
         const float f_ij = kernelF<D>(sqrtf(s) / H) * CONF * c.m / c.rho;
         return (c.p - st.p_i) * f_ij;
     }
-    __device__ static Term none() { return 0.f; }
+    __device__ static Term none() { return -0.f; }
     template <int Q>
     __device__ void add_group(State& st, const Term& t) const
     {

@@ -977,6 +977,8 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
 // pure function of the owner and the candidate) and add_group<Q>(st, term),
 // which adds the terms of the group's lanes in lane order on all of them:
 // every owner's sums take the terms of the one-lane walk in the same order.
+// A lane without a candidate adds Pol::none(), which holds -0: x + -0 is x
+// for every x.
 // PER: the candidate's position is moved to its periodic image first.
 // olist as in cell_kernel_k, its count in n_heads[count_word].
 // ---------------------------------------------------------------------------
@@ -1042,15 +1044,15 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
                                            w.per);
                     }
                     // the walk's test accepts a thin shell beyond: such a
-                    // candidate gets no weight (a select, so that every
-                    // load of the pair is issued at once)
+                    // candidate adds nothing, whatever its fields hold (the
+                    // term is selected, so that every load of the pair is
+                    // issued at once)
                     const f3 r_ij = sub<D>(c.r, r_i);
-                    const bool out = dot<D>(r_ij, r_ij) > smax ||
+                    const bool out = (dot<D>(r_ij, r_ij) > smax) |
                                      (Pol::NO_SELF && j == i);
-                    pol.weigh(c, out);
                     t = nrq ? pol.template term<true>(i, j, c, r_i, st)
                             : pol.template term<false>(i, j, c, r_i, st);
-                    pol.weigh(t, out);
+                    if (out) t = Pol::none();
                 }
                 pol.template add_group<Q>(st, t);
             };
@@ -1070,15 +1072,6 @@ template <int Q> __device__ __forceinline__ void add_lanes(float& a, float v)
 {
     each_lane<Q>(v, [&](float x) { a += x; });
 }
-
-// weigh(x, out): takes the weight of an `out` candidate (its mass or area,
-// which every product of the term carries) or of its term
-#define AQ_POL_WEIGH_MASS                                                      \
-    __device__ static void weigh(Cand& c, bool out)                            \
-    {                                                                          \
-        c.m = out ? 0.f : c.m;                                                 \
-    }                                                                          \
-    __device__ static void weigh(Term&, bool) {}
 
 // The element-owner policies below split each pair into load(j) (the
 // candidate's fields), term<NRQ>(i, j, cand, r_i, st) (a pure function of
@@ -1164,11 +1157,6 @@ template <int D> struct PolBiShepard {
         }
     }
     __device__ static Term none() { return Term{ 0.f, 2u }; }
-    __device__ static void weigh(Cand&, bool) {}
-    __device__ static void weigh(Term& t, bool out)
-    {
-        if (out) t = none();
-    }
     template <int Q>
     __device__ void add_group(State& st, const Term& t) const
     {
@@ -1258,8 +1246,10 @@ template <int D> struct PolBiLapU {
         st.lu.y += t.v.y;
         if constexpr (D == 3) st.lu.z += t.v.z;
     }
-    __device__ static Term none() { return Term{ f3{ 0.f, 0.f, 0.f }, 0u }; }
-    AQ_POL_WEIGH_MASS
+    __device__ static Term none()
+    {
+        return Term{ f3{ -0.f, -0.f, -0.f }, 0u };
+    }
     template <int Q>
     __device__ void add_group(State& st, const Term& t) const
     {
@@ -1318,8 +1308,7 @@ template <int D> struct PolBiInterp {
         return (c.p - dot<D>(st.gp_i, r_ij)) * w_ij;
     }
     __device__ void add(State& st, const Term& t) const { st.acc += t; }
-    __device__ static Term none() { return 0.f; }
-    AQ_POL_WEIGH_MASS
+    __device__ static Term none() { return -0.f; }
     template <int Q>
     __device__ void add_group(State& st, const Term& t) const
     {
@@ -1389,12 +1378,10 @@ template <int D> struct PolBiInteractions {
         st.gp = add3<D>(st.gp, t.g);
         st.dv += t.d;
     }
-    __device__ static Term none() { return Term{ f3{ 0.f, 0.f, 0.f }, 0.f }; }
-    __device__ static void weigh(Cand& c, bool out)
+    __device__ static Term none()
     {
-        c.area = out ? 0.f : c.area;
+        return Term{ f3{ -0.f, -0.f, -0.f }, -0.f };
     }
-    __device__ static void weigh(Term&, bool) {}
     template <int Q>
     __device__ void add_group(State& st, const Term& t) const
     {
@@ -1472,10 +1459,9 @@ template <int D> struct PolLesGradU {
     {
         Term t;
 #pragma unroll
-        for (int k = 0; k < D * D; k++) t.g[k] = 0.f;
+        for (int k = 0; k < D * D; k++) t.g[k] = -0.f;
         return t;
     }
-    AQ_POL_WEIGH_MASS
     template <int Q>
     __device__ void add_group(State& st, const Term& t) const
     {
@@ -1541,8 +1527,7 @@ template <int D> struct PolLesInteractions {
             f * (st.mu_i + c.rho * c.nu) / (st.rho_i * c.rho);
         return scl<D>(sc, sub<D>(c.u, st.u_i));
     }
-    __device__ static Term none() { return f3{ 0.f, 0.f, 0.f }; }
-    AQ_POL_WEIGH_MASS
+    __device__ static Term none() { return f3{ -0.f, -0.f, -0.f }; }
     template <int Q>
     __device__ void add_group(State& st, const Term& t) const
     {

@@ -211,34 +211,39 @@ def test_les_groups_match_oracle(cuda, tmp_path, dims, n):
     sim.close()
 
 
-# around the line between 16 and 4 lanes per particle, single particles and
-# cells of more than 64
-@pytest.mark.parametrize("dims,n,cell,lap", [
-    (2, 1, 3, 1), (2, 65, 3, 2), (2, 16384, 4, 1), (2, 16385, 4, 2),
-    (2, 30011, 12, 1), (3, 1, 3, 1), (3, 63, 2, 1), (3, 5000, 6, 2),
-    (3, 16384, 4, 1), (3, 20011, 4, 1)])
-def test_abi_pair_kernels_match_oracle(cuda, dims, n, cell, lap):
-    """aq_shepard (both variants), aq_interactions and aq_lapp on disordered
-    particles of every kind, about cell^dims of them per cell, against the
-    oracle's float32 walk, bit for bit, accumulating onto given values."""
-    from oracle import pipeline as op
-    rng = np.random.default_rng(n + dims)
-    vs = 2 if dims == 2 else 4
-    side = max(1.0, (n / cell ** dims) ** (1 / dims))  # in cells
-    h = np.float32(0.05)
-    r = np.zeros((n, vs), np.float32)
-    r[:, :dims] = rng.uniform(0, side * 2 * h, (n, dims))
-    u = np.zeros_like(r)
-    u[:, :dims] = rng.normal(0, 1, (n, dims))
-    f32 = lambda a: np.ascontiguousarray(a, np.float32)  # noqa: E731
-    rho = f32(1000 + rng.normal(0, 5, n))
-    m = f32(rng.uniform(0.5, 1.5, n))
-    p = f32(rng.normal(0, 100, n))
-    im = rng.choice(np.array([1, 1, 1, 1, 1, 0, -3, 2, 3, -256], np.int32), n)
-    cap = int(side + 8) ** dims
+@pytest.mark.parametrize("dims,n", [(2, 23), (2, 150), (3, 17), (3, 30)])
+def test_les_gradient_of_an_empty_particle(cuda, tmp_path, dims, n):
+    """A particle of zero density is no neighbour of itself: its own velocity
+    gradient stays finite (16 and 4 lanes per particle)."""
+    from aquagpusph_amd import casefiles, cases
+    from aquagpusph_amd.sim import Simulation
+    case = _stir(cases.periodic_box(dims, n), 5)
+    # one in every 500, none a neighbour of another
+    empty = np.arange(0, case["N"], 500)
+    if dims == 2:
+        empty = empty[:1]
+    case["rho"][empty] = 0
+    sim = Simulation(casefiles.write_case(
+        case, str(tmp_path), load=False, presets=casefiles.PPER_PRESETS +
+        ("resources/Presets/cfd/LES-smagorinsky.xml",)), dims)
+    casefiles.upload(sim, case)
+    sim.step(1)
+    g, ids = sim.get("grad_u").reshape(case["N"], -1), sim.get("id")
+    sim.close()
+    mine = np.isin(ids, empty)
+    assert mine.sum() == empty.size
+    assert np.isfinite(g[mine]).all()
+
+
+def _abi_linklist(dims, r, h):
+    """Device link-list (icell, ihoc, n_cells) of the positions r, and the
+    permutation that sorts them."""
+    n, vs = r.shape
+    extent = (r.max(0) - r.min(0))[:dims]
+    cap = int(np.prod(np.floor(extent / (2 * h)) + 8))
     d = {k: _dev(v) for k, v in dict(
         lo=np.zeros(vs, np.float32), hi=np.zeros(vs, np.float32),
-        sup=f32([2]), h=f32([h]), nc=np.zeros(4, np.int32),
+        sup=np.float32([2]), h=np.float32([h]), nc=np.zeros(4, np.int32),
         ic=np.zeros(n, np.int32), pu=np.zeros(n, np.int32),
         ps=np.zeros(n, np.int32), hoc=np.zeros(cap, np.int32),
         st=np.zeros(1, np.int32), r=r).items()}
@@ -248,8 +253,17 @@ def test_abi_pair_kernels_match_oracle(cuda, dims, n, cell, lap):
               _dp(d["hi"]), _dp(d["sup"]), _dp(d["h"]), _dp(d["nc"]),
               _dp(d["ic"]), _dp(d["pu"]), _dp(d["ps"]), _dp(d["hoc"]), cap,
               _dp(d["st"]), _dp(ws), _stream())
-    perm = d["pu"].cpu().numpy()
     assert int(d["st"].item()) == 0
+    return d, d["pu"].cpu().numpy()
+
+
+def _check_abi_pair_kernels(rng, dims, lap, h, r, u, rho, m, p, im):
+    """aq_shepard (both variants), aq_interactions and aq_lapp against the
+    oracle's float32 walk, bit for bit, accumulating onto given values."""
+    from oracle import pipeline as op
+    f32 = lambda a: np.ascontiguousarray(a, np.float32)  # noqa: E731
+    n, vs = r.shape
+    d, perm = _abi_linklist(dims, r, h)
     r, u, rho, m, p, im = (np.ascontiguousarray(a[perm])
                            for a in (r, u, rho, m, p, im))
     H = op.definition(h)
@@ -287,3 +301,61 @@ def test_abi_pair_kernels_match_oracle(cuda, dims, n, cell, lap):
                op._p(w[3]), cu(n), *oll, cf(H), cf(CONF))
     for a, b in zip(t, w):
         np.testing.assert_array_equal(a.cpu().numpy(), b)
+
+
+# around the line between 16 and 4 lanes per particle, single particles and
+# cells of more than 64
+@pytest.mark.parametrize("dims,n,cell,lap", [
+    (2, 1, 3, 1), (2, 65, 3, 2), (2, 16384, 4, 1), (2, 16385, 4, 2),
+    (2, 30011, 12, 1), (3, 1, 3, 1), (3, 63, 2, 1), (3, 5000, 6, 2),
+    (3, 16384, 4, 1), (3, 20011, 4, 1)])
+def test_abi_pair_kernels_match_oracle(cuda, dims, n, cell, lap):
+    """The pair kernels of the C ABI on disordered particles of every kind,
+    about cell^dims of them per cell."""
+    rng = np.random.default_rng(n + dims)
+    vs = 2 if dims == 2 else 4
+    side = max(1.0, (n / cell ** dims) ** (1 / dims))  # in cells
+    h = np.float32(0.05)
+    r = np.zeros((n, vs), np.float32)
+    r[:, :dims] = rng.uniform(0, side * 2 * h, (n, dims))
+    u = np.zeros_like(r)
+    u[:, :dims] = rng.normal(0, 1, (n, dims))
+    f32 = lambda a: np.ascontiguousarray(a, np.float32)  # noqa: E731
+    rho = f32(1000 + rng.normal(0, 5, n))
+    m = f32(rng.uniform(0.5, 1.5, n))
+    p = f32(rng.normal(0, 100, n))
+    im = rng.choice(np.array([1, 1, 1, 1, 1, 0, -3, 2, 3, -256], np.int32), n)
+    _check_abi_pair_kernels(rng, dims, lap, h, r, u, rho, m, p, im)
+
+
+@pytest.mark.parametrize("dims,sites,lap", [(2, 60, 1), (2, 800, 2),
+                                            (3, 60, 2), (3, 800, 1)])
+def test_abi_pairs_at_the_edge_of_the_support(cuda, dims, sites, lap):
+    """Pairs within 4e-5 of the support radius (the walk's distance test
+    accepts some of those beyond it) whose neighbour has an infinite, NaN or
+    zero field, and particles that meet themselves with such a field: a pair
+    out of reach, or a particle with itself, adds nothing.  Each site is a
+    bunch of 24 particles and a broken one a support radius away; 60 sites
+    run with 16 lanes per particle, 800 with 4."""
+    rng = np.random.default_rng(sites + dims)
+    vs = 2 if dims == 2 else 4
+    h = np.float32(0.05)
+    k, B = np.arange(sites), 25
+    n = sites * B
+    r = np.zeros((sites, B, vs))
+    r[:, :, 0] = (0.61 * (k % 20))[:, None]
+    r[:, :, 1] = (0.61 * (k // 20))[:, None]
+    r[:, :-1, 1] += 1e-3 * h * rng.uniform(-1, 1, (sites, B - 1))
+    r[:, -1, 0] += 2 * h * (1 + 4e-5 * rng.uniform(-1, 1, sites))
+    r = np.ascontiguousarray(r.reshape(n, vs), np.float32)
+    u = np.zeros_like(r)
+    u[:, :dims] = rng.normal(0, 1, (n, dims))
+    f32 = lambda a: np.ascontiguousarray(a, np.float32)  # noqa: E731
+    rho, m, p = (f32(1000 + rng.normal(0, 5, n)),
+                 f32(rng.uniform(0.5, 1.5, n)), f32(rng.normal(0, 100, n)))
+    last = np.arange(sites) * B + B - 1
+    for kind, (a, v) in enumerate([(p, np.inf), (p, np.nan), (rho, 0),
+                                   (m, np.inf), (u, np.nan)]):
+        a[last[kind::5]] = v
+    _check_abi_pair_kernels(rng, dims, lap, h, r, u, rho, m, p,
+                            np.ones(n, np.int32))
