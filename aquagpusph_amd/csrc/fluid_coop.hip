@@ -159,6 +159,10 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
                         const f3 v = lapf == AQ_LAP_MONAGHAN ? r_ij : u_ij;
                         g = scl<D>(t.sg, r_ij);
                         l = scl<D>(t.sl, v);
+                        if (PER && s > smax) {
+                            t = PairTerms{ 0.f, 0.f, 0.f, 0.f, 0.f };
+                            g = l = f3{ 0.f, 0.f, 0.f };
+                        }
                     }
                     if constexpr (SHEP == 1)
                         each_lane<Q>(t.sh, [&](float x) { sh += x; });

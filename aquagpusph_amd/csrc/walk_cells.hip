@@ -713,10 +713,13 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
             // branch, so every load of the pair is issued at once): its
             // terms are then +-0 (finite fields), and adding +-0 leaves the
             // sums unchanged, since they are never -0 (they start at +0, or
-            // 1, and an exact cancellation rounds to +0).
+            // 1, and an exact cancellation rounds to +0).  SKIP: it is
+            // passed over, whatever its fields hold.
+            constexpr bool SKIP = PER || FAST;
             auto pair_fd = [&](uint32_t j, const f3& r_j) {
                 const f3 r_ij = sub<D>(r_j, r_i);
                 const float s = dot<D>(r_ij, r_ij);
+                if (SKIP && s > smax) return;
                 const float qf = div_nr(sqrt_nr(s), RH);
                 float m_j = ldf_o(m, j);
                 m_j = (s > smax) ? 0.f : m_j;
@@ -740,9 +743,9 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
                         // multiply-adds
                         const f3 r_ij = sub<D>(r_j, r_i);
                         const float s = fdot<D>(r_ij, r_ij);
+                        if (SKIP && s > smax) return;
                         const float q = __builtin_amdgcn_sqrtf(s) * iH;
-                        float m_j = ldf_o(m, j);
-                        m_j = (s > smax) ? 0.f : m_j;
+                        const float m_j = ldf_o(m, j);
                         const float irho_j =
                             __builtin_amdgcn_rcpf(ldf_o(rho, j));
                         if (SHEP == 1)
@@ -768,6 +771,7 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
                     }
                     const f3 r_ij = sub<D>(r_j, r_i);
                     const float s = dot<D>(r_ij, r_ij);
+                    if (SKIP && s > smax) return;
                     const float q = sqrtf(s) / H;
                     float m_j = ldf_o(m, j);
                     m_j = (s > smax) ? 0.f : m_j;

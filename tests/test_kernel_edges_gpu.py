@@ -168,6 +168,48 @@ def test_lanes_per_particle_are_bit_identical(cuda, tmp_path, monkeypatch,
         np.testing.assert_array_equal(got[k], want[k], err_msg=k)
 
 
+# 16, 4 and one lane per particle in a periodic box, one with relaxed math
+@pytest.mark.parametrize("dims,n,relaxed", [
+    (2, 60, False), (2, 150, False), (3, 17, False), (3, 30, False),
+    (3, 64, False), (2, 60, True), (3, 30, True)])
+def test_fluid_pairs_at_the_edge_of_the_support(cuda, tmp_path, dims, n,
+                                                relaxed):
+    """Neighbours of zero density up to 2e-5 beyond the support radius (the
+    walk's distance test accepts some of them): they add nothing, so the
+    sums of the particle they are out of reach of stay finite."""
+    from aquagpusph_amd import casefiles, cases
+    from aquagpusph_amd.sim import Simulation
+    case = cases.periodic_box(dims, n, seed=2)
+    # a row of particles i, 11 apart, and their neighbours j, 4 spacings on
+    x, dr, h = case["r"], case["params"]["dr"], case["params"]["h"]
+    x[:, :dims] = x[:, :dims].astype(np.float32)
+    key = np.lexsort(np.round(x[:, :dims] / dr, 2).T)
+    row = key[:n] if dims == 2 else key[n * (n // 2):][:n]
+    i = row[np.arange(2, n - 6, 11)]
+    j = row[np.arange(2, n - 6, 11) + 4]
+    assert np.allclose(x[j, 0] - x[i, 0], 4 * dr, rtol=1e-4)
+    assert np.allclose(2 * h, 4 * dr, rtol=1e-6)
+    x[j] = x[i]
+    x[j, 0] += 2 * h * (1 + np.linspace(2e-6, 2e-5, len(i)))
+    case["rho"][j] = 0
+    case["u"][:] = 0  # the predictor leaves the positions
+    kw = {}
+    if relaxed:
+        kw["extra_xml"] = ('<Settings><Device platform="0" device="0" '
+                           'compile_flags="-cl-fast-relaxed-math" />'
+                           '</Settings>')
+    sim = Simulation(casefiles.write_case(
+        case, str(tmp_path), load=False, presets=casefiles.PPER_PRESETS,
+        **kw), dims)
+    casefiles.upload(sim, case)
+    sim.step(1)
+    ids = sim.get("id")
+    mine = np.isin(ids, i)
+    for k in ("grad_p", "lap_u", "div_u", "lap_p", "shepard"):
+        assert np.isfinite(sim.get(k).reshape(len(ids), -1)[mine]).all(), k
+    sim.close()
+
+
 # element kernels: 16 lanes per owner below 100 k (2D) / 600 k (3D)
 # particles, 4 above; wall edges and corners hold more than one group
 @pytest.mark.parametrize("dims,dr,hfac", [(2, 0.06, 2.0), (2, 0.011, 2.0),
