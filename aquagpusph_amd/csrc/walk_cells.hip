@@ -1071,6 +1071,75 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
     }
 }
 
+// One owner per lane through the fused walk's ring (ring_walk_m), for fluid
+// owners once their cells fill the chip.  Policies as in cell_group_k, with
+// add(st, term) for one term; hand-out as in cell_kernel_k.
+template <int D, class Pol, bool PER>
+__global__ void __launch_bounds__(64 * WC_WAVES)
+    cell_lane_k(Pol pol, const int* __restrict__ imove,
+                const float* __restrict__ r, WalkArgs w, float smax, int nrq,
+                const uint32_t* __restrict__ olist, uint32_t count_word)
+{
+    __shared__ RingLds<8, PER> lds[WC_WAVES];
+    const int lane = threadIdx.x & 63;
+    RingLds<8, PER>& L = lds[threadIdx.x >> 6];
+    if (w.status && (*w.status & 1u)) return;
+    const uint32_t n_heads =
+        olist ? uni(w.n_heads[count_word]) : uni(*w.n_heads);
+    const uint32_t nwv = gridDim.x * WC_WAVES;
+    for (uint32_t hk = blockIdx.x * WC_WAVES + (threadIdx.x >> 6);
+         hk < n_heads; hk += nwv) {
+        uint32_t cstart, c_i, ce;
+        if (olist) {
+            cstart = uni(olist[3 * hk]);
+            c_i = uni(olist[3 * hk + 1]);
+            ce = uni(olist[3 * hk + 2]);
+        } else {
+            cstart = uni(w.heads[hk]);
+            c_i = uni(w.icell[cstart]);
+            ce = uni(w.cell_end[c_i]);
+        }
+        const uint32_t cend = ce & AQ_CELL_END;
+        if (w.flagged && Pol::OWNERS && !(ce & Pol::OWNERS)) continue;
+        for (uint32_t i0 = cstart; i0 < cend; i0 += 64) {
+            const uint32_t i = i0 + lane;
+            const bool act = (i < cend) && pol.owner(i, imove[i]);
+            if (__ballot(act) == 0) continue;
+            const uint32_t total = neighbour_table<D, PER>(
+                w, c_i, L, lane, Pol::KIND ? AQ_CELL_ELEM : AQ_CELL_FLUID);
+            typename Pol::State st{};
+            f3 r_i = { 0.f, 0.f, 0.f };
+            if (act) {
+                r_i = ldv<D>(r, i);
+                pol.init(i, r_i, st);
+            }
+            f3 bmin, bmax;
+            wave_box<D>(r_i, act, bmin, bmax);
+            auto walk = [&](auto fd) {
+                constexpr bool NRQ = decltype(fd)::value;
+                auto pair = [&](uint32_t j, const f3& r_j) {
+                    auto c = pol.load(j);
+                    c.r = r_j;
+                    const f3 r_ij = sub<D>(r_j, r_i);
+                    const bool out = (dot<D>(r_ij, r_ij) > smax) |
+                                     (Pol::NO_SELF && j == i);
+                    auto t = pol.template term<NRQ>(i, j, c, r_i, st);
+                    if (out) t = Pol::none();
+                    pol.add(st, t);
+                };
+                bool unused = false;
+                ring_walk_m<D, 8, PER>(L, lane, total, r_i, act, bmin, bmax,
+                                       smax, r, imove, Pol::KIND, false,
+                                       unused, pair, w.per);
+            };
+            if (nrq) walk(std::true_type{});
+            else walk(std::false_type{});
+            if (act) pol.finish(i, st);
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+}
+
 // a += the values v of the group's lanes, in lane order
 template <int Q> __device__ __forceinline__ void add_lanes(float& a, float v)
 {
@@ -1410,7 +1479,7 @@ template <int D> struct PolBiInteractions {
 //   G_i = sum_j m_j / rho_j (u_j - u_i) (x) F_ij r_ij,
 // grad_u[a n + b] = du_a / dx_b (row stride n = 2 in 2D, 4 in 3D), summed
 // in the walk order.  The non-fluid particles' rows are cleared by the
-// launcher.  (Group kernel only.)
+// launcher.
 template <int D> struct PolLesGradU {
     static constexpr int KIND = 0;
     static constexpr bool NO_SELF = true;
@@ -1465,6 +1534,11 @@ template <int D> struct PolLesGradU {
 #pragma unroll
         for (int k = 0; k < D * D; k++) t.g[k] = -0.f;
         return t;
+    }
+    __device__ void add(State& st, const Term& t) const
+    {
+#pragma unroll
+        for (int k = 0; k < D * D; k++) st.G[k] += t.g[k];
     }
     template <int Q>
     __device__ void add_group(State& st, const Term& t) const
@@ -1532,6 +1606,10 @@ template <int D> struct PolLesInteractions {
         return scl<D>(sc, sub<D>(c.u, st.u_i));
     }
     __device__ static Term none() { return f3{ -0.f, -0.f, -0.f }; }
+    __device__ void add(State& st, const Term& t) const
+    {
+        st.acc = add3<D>(st.acc, t);
+    }
     template <int Q>
     __device__ void add_group(State& st, const Term& t) const
     {
@@ -1792,13 +1870,12 @@ static void launch_bi_cells(const Pol& pol, const int32_t* imove,
 //                        1.2 M 57 / 62   4.5 M 113 / 126
 //                    2D  21 k 13 / 11   1.2 M (64 tanks) 23 / 28
 //   BI Interactions  3D  29 k 25 / 34   1.2 M 72 / 126   4.5 M 136 / 245
-//   LES grad u       3D  9 k 219 / 101   64 k 204 / 248   262 k 570 / 862
 // The elements are few and hold a fifth of their neighbours' particles each,
 // so 16 lanes pay as long as latency rules; fluid owners fill the chip much
-// earlier.  (Before, in us at 4.5 M / 1.2 M / 29 k: 4 lanes with the terms
+// earlier (les_lanes for the LES kernels).  (Before, in us at 4.5 M / 1.2 M / 29 k: 4 lanes with the terms
 // through LDS and a full wait per segment, LapU 240 / 134 / 127,
 // Interpolation 200 / 119 / 113; one lane per owner, Interactions 132 / 75 /
-// 65; LES grad u at 262 k one lane 667.)
+// 65.)
 template <int D, class Pol, bool PER = false>
 static void launch_groups(const Pol& pol, const int32_t* imove,
                           const float* r, const CellArgs& c, float smax,
@@ -1936,19 +2013,57 @@ void launch_bi_interactions_cells(int dims, const int32_t* imove,
            std::integral_constant<int, 3>{});
 }
 
-// LES kernels: groups over every cell
+// Lanes per particle of the LES kernels for N particles; 0: one lane each
+// (cell_lane_k).  Both kernels of a step in us, 16 / 4 / one, on the lattice
+// and with the particles displaced by up to 0.4 of their spacing:
+//   3D   22 k  230 /  302 /  889     242 /  344 / 1094
+//        47 k  279 /  200 /  445     322 /  242 /  570
+//       195 k 1507 /  997 / 1101    1848 / 1083 / 1259
+//       262 k 1360 /  843 /  645    1502 /  956 /  835
+//       373 k 2001 / 1190 / 1111    2103 / 1277 / 1347
+//       512 k 2740 / 1740 / 1325    2879 / 1799 / 1622
+//       2.1 M  11610 / 7078 / 5148  12289 / 7330 / 6157
+//   2D   16 k   40 /   54 /   64      45 /   57 /   74
+//        40 k   54 /   42 /   74      59 /   48 /   88
+//       1.0 M 1006 /  620 / 1123    1422 /  848 / 1227
+// One lane each wins, as in the fused walk, once the 3D cells fill the chip
+// (4096 wavefronts, 262 k particles).
+static int les_lanes(int dims, uint32_t N)
+{
+    if (N <= (dims == 2 ? 16000u : 24000u)) return 16;
+    return dims == 3 && N > 250000u ? 0 : 4;
+}
+
+// LES kernels over every cell
+template <int D, class Pol, bool PER>
+static void launch_les_form(const Pol& pol, const int32_t* imove,
+                            const float* r, const CellArgs& c, float smax,
+                            const float* per, hipStream_t s)
+{
+    const int q = les_lanes(D, c.N);
+    if (q) {
+        launch_groups<D, Pol, PER>(pol, imove, r, c, smax, s, q == 16,
+                                   nullptr, 0, D == 2 ? 16 : 64, per);
+        return;
+    }
+    AQ_REQUIRE(c.N < (1u << 28), "cell-parallel walk: more than 2^28 particles");
+    WalkArgs w{ c.icell,   c.ihoc,   c.n_cells, c.cell_end, c.heads,
+                c.n_heads, nullptr,  c.status,  c.N,        c.flagged,
+                walk_ranges(), per };
+    auto* ker = cell_lane_k<D, Pol, PER>;
+    const int nrq = (pol.H >= 0x1p-40f && pol.H <= 0x1p40f) ? 1 : 0;
+    hipLaunchKernelGGL(ker, dim3(walk_grid((const void*)ker, c)),
+                       dim3(64 * WC_WAVES), 0, s, pol, imove, r, w, smax, nrq,
+                       c.blist, 0u);
+}
+
 template <int D, class Pol>
 static void launch_les(const Pol& pol, const int32_t* imove, const float* r,
                        const CellArgs& c, float smax, const float* per,
                        hipStream_t s)
 {
-    const bool wide = c.N <= (D == 2 ? 16000u : 24000u);
-    const uint32_t full = D == 2 ? 16 : 64;
-    if (per)
-        launch_groups<D, Pol, true>(pol, imove, r, c, smax, s, wide, nullptr,
-                                    0, full, per);
-    else
-        launch_groups<D>(pol, imove, r, c, smax, s, wide, nullptr, 0, full);
+    if (per) launch_les_form<D, Pol, true>(pol, imove, r, c, smax, per, s);
+    else launch_les_form<D, Pol, false>(pol, imove, r, c, smax, nullptr, s);
 }
 
 void launch_les_gradu_cells(int dims, const int32_t* imove, const float* r,

@@ -229,11 +229,13 @@ def test_element_groups_match_one_lane_walks(cuda, tmp_path, monkeypatch,
         np.testing.assert_array_equal(got[k], want[k], err_msg=k)
 
 
-@pytest.mark.parametrize("dims,n", [(2, 23), (2, 150), (3, 17), (3, 30)])
+@pytest.mark.parametrize("dims,n", [(2, 23), (2, 150), (3, 17), (3, 30),
+                                    (3, 63)])
 def test_les_groups_match_oracle(cuda, tmp_path, dims, n):
     """The LES gradient and viscous term (periodic box, Smagorinsky) with 16
     and with 4 lanes per particle (2D above 16 k, 3D above 24 k particles)
-    against the oracle's float32 walk, bit for bit."""
+    and with one (3D above 250 k: 63^3 = 250,047) against the oracle's
+    float32 walk, bit for bit."""
     from aquagpusph_amd import casefiles, cases
     from aquagpusph_amd.sim import Simulation
     from oracle import pipeline as op
@@ -244,26 +246,50 @@ def test_les_groups_match_oracle(cuda, tmp_path, dims, n):
     casefiles.upload(sim, case)
     o = op.OracleSim(case, bi=False, domain=False, les={"Cs": 0.15},
                      periodic=case["params"]["periodic"])
-    for _ in range(2):
+    steps = 2 if n < 60 or dims == 2 else 1
+    for _ in range(steps):
         o.step()
-    sim.step(2)
+    sim.step(steps)
     for k in ("grad_u", "nu_t", "dudt", "u", "r"):
         np.testing.assert_array_equal(sim.get(k).ravel(), o.f[k].ravel(),
                                       err_msg=k)
     sim.close()
 
 
-@pytest.mark.parametrize("dims,n", [(2, 23), (2, 150), (3, 17), (3, 30)])
+# 16, 4 and one lane per particle inside walls (particles with the elements)
+@pytest.mark.parametrize("dims,dr,lo,hi", [
+    (2, 0.011, 0, 16000), (3, 0.0187, 24000, 250000),
+    (3, 0.0083, 250000, 1 << 28)])
+def test_les_walls_match_oracle(cuda, tmp_path, dims, dr, lo, hi):
+    """The LES kernels of a dam break with its walls (no periodic images)
+    against the oracle's float32 walk, bit for bit."""
+    from aquagpusph_amd import casefiles, cases
+    from aquagpusph_amd.sim import Simulation
+    from oracle import pipeline as op
+    case = _stir(cases.dam_break(dims, dr), 5)
+    assert lo < case["N"] <= hi
+    sim = Simulation(casefiles.write_case(
+        case, str(tmp_path), load=False, presets=casefiles.PBI_PRESETS +
+        ("resources/Presets/cfd/LES-smagorinsky.xml",)), dims)
+    casefiles.upload(sim, case)
+    o = op.OracleSim(case, les={"Cs": 0.15})
+    o.step()
+    sim.step(1)
+    for k in ("grad_u", "nu_t", "dudt", "u", "r"):
+        np.testing.assert_array_equal(sim.get(k).ravel(), o.f[k].ravel(),
+                                      err_msg=k)
+    sim.close()
+
+
+@pytest.mark.parametrize("dims,n", [(2, 23), (2, 150), (3, 17), (3, 30),
+                                    (3, 63)])
 def test_les_gradient_of_an_empty_particle(cuda, tmp_path, dims, n):
     """A particle of zero density is no neighbour of itself: its own velocity
-    gradient stays finite (16 and 4 lanes per particle)."""
+    gradient stays finite (16, 4 and one lane per particle)."""
     from aquagpusph_amd import casefiles, cases
     from aquagpusph_amd.sim import Simulation
     case = _stir(cases.periodic_box(dims, n), 5)
-    # one in every 500, none a neighbour of another
-    empty = np.arange(0, case["N"], 500)
-    if dims == 2:
-        empty = empty[:1]
+    empty = np.array([case["N"] // 2])
     case["rho"][empty] = 0
     sim = Simulation(casefiles.write_case(
         case, str(tmp_path), load=False, presets=casefiles.PPER_PRESETS +
