@@ -294,9 +294,11 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
 // lattice 503 / 503, out of it 888 / 819; 193 k 502 / 782 and 902 / 1186); 16
 // lanes pay it 16 times (2D 8 k 109 / 39 / 37, 31 k 107 / 44 / 72; 3D 11 k
 // - / 147 / 111, 23 k - / 171 / 242).
-int fluid_coop_lanes(int dims, uint32_t N, int math)
+// A periodic box of more particles than the group walk can name: one lane.
+int fluid_coop_lanes(int dims, uint32_t N, int math, bool per)
 {
     const bool comp = math == 2;
+    if (per && N > PER_GROUP_MAX_N) return 0;
     if (dims == 2) return N <= (comp ? 8000u : 16000u) ? 16 : 4;
     if (N <= (comp ? 12000u : 24000u)) return 16;
     return N <= (comp ? 150000u : 250000u) ? 4 : 0;
@@ -312,6 +314,8 @@ void launch_fluid_coop(int dims, int shep, bool lapp, int q,
                        float smax, int math, const uint32_t* rec,
                        hipStream_t s)
 {
+    AQ_REQUIRE(!w.per || w.N <= PER_GROUP_MAX_N,
+               "periodic box: more than 2^27 particles in a group walk");
     // a 2D cell holds one group of 16 particles, a 3D cell four
     const uint32_t S = q == 16 ? (dims == 2 ? 4u : 16u)
                                : (dims == 2 ? 1u : 4u);

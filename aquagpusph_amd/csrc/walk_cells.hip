@@ -1727,7 +1727,7 @@ static unsigned walk_grid(const void* ker, const CellArgs& c)
     return std::min(res, std::max(1u, side_wgs_per_cu()) * cu_count());
 }
 
-int fluid_coop_lanes(int dims, uint32_t N, int math);
+int fluid_coop_lanes(int dims, uint32_t N, int math, bool per);
 void launch_fluid_coop(int dims, int shep, bool lapp, int q,
                        const int32_t* imove, const float* r, const float* u,
                        const float* rho, const float* m, const float* p,
@@ -1789,7 +1789,7 @@ void launch_fluid_pass_cells(int dims, int shep, bool lapp,
     // only: an explicit segment width or grid asks for the one-lane walk)
     if (const int q = segw == 8 && !nblocks && ranges != 1 && !reserve_per_cu
                               && math != 1
-                          ? fluid_coop_lanes(dims, N, math)
+                          ? fluid_coop_lanes(dims, N, math, per != nullptr)
                           : 0) {
         launch_fluid_coop(dims, shep, lapp, q, imove, r, u, rho, m, p, normal,
                           tangent, binormal, shepard, grad_p, lap_u, div_u,
@@ -1884,6 +1884,8 @@ static void launch_groups(const Pol& pol, const int32_t* imove,
                           const float* per = nullptr)
 {
     AQ_REQUIRE(c.N < (1u << 28), "cell-parallel walk: more than 2^28 particles");
+    AQ_REQUIRE(!PER || c.N <= PER_GROUP_MAX_N,
+               "periodic box: more than 2^27 particles in a group walk");
     WalkArgs w{ c.icell,   c.ihoc,   c.n_cells, c.cell_end, c.heads,
                 c.n_heads, nullptr,  c.status,  c.N,        c.flagged,
                 walk_ranges(), per };
@@ -1904,6 +1906,12 @@ static void launch_groups(const Pol& pol, const int32_t* imove,
     else launch(cell_group_k<D, 4, Pol, PER>, 4);
 }
 
+// Lanes per wall element or sensor of the owner-list walks (launch_groups)
+static int elem_lanes(int dims, uint32_t N)
+{
+    return N <= (dims == 2 ? 100000u : 600000u) ? 16 : 4;
+}
+
 // list: 0 every non-empty cell (one owner per lane), 1 the owner cells,
 // 2 the wet owner cells (group kernel)
 template <int D, class Pol>
@@ -1919,7 +1927,7 @@ static void launch_bi_coop(const Pol& pol, const int32_t* imove,
         launch_bi_cells<D>(pol, imove, r, c, smax, s);
     else
         launch_groups<D>(pol, imove, r, c, smax, s,
-                         c.N <= (D == 2 ? 100000u : 600000u), ol,
+                         elem_lanes(D, c.N) == 16, ol,
                          list == 1 ? AQ_CL_NOCELLS : AQ_CL_NWCELLS,
                          AQ_OWNER_CHUNK);
 }
@@ -2028,8 +2036,10 @@ void launch_bi_interactions_cells(int dims, const int32_t* imove,
 //       1.0 M 1006 /  620 / 1123    1422 /  848 / 1227
 // One lane each wins, as in the fused walk, once the 3D cells fill the chip
 // (4096 wavefronts, 262 k particles).
-static int les_lanes(int dims, uint32_t N)
+// A periodic box of more particles than the group walk can name: one lane.
+static int les_lanes(int dims, uint32_t N, bool per)
 {
+    if (per && N > PER_GROUP_MAX_N) return 0;
     if (N <= (dims == 2 ? 16000u : 24000u)) return 16;
     return dims == 3 && N > 250000u ? 0 : 4;
 }
@@ -2040,7 +2050,7 @@ static void launch_les_form(const Pol& pol, const int32_t* imove,
                             const float* r, const CellArgs& c, float smax,
                             const float* per, hipStream_t s)
 {
-    const int q = les_lanes(D, c.N);
+    const int q = les_lanes(D, c.N, PER);
     if (q) {
         launch_groups<D, Pol, PER>(pol, imove, r, c, smax, s, q == 16,
                                    nullptr, 0, D == 2 ? 16 : 64, per);
@@ -2102,3 +2112,21 @@ void launch_les_interactions_cells(int dims, const int32_t* imove,
 }
 
 }  // namespace aq
+
+using namespace aq;
+
+extern "C" AQ_API int aq_walk_lanes(int kernel, int dims, uint32_t N,
+                                    int periodic)
+{
+    if ((dims != 2 && dims != 3) || N >= (1u << 28)) return AQ_EINVAL;
+    const bool per = periodic != 0;
+    switch (kernel) {
+    case AQ_WALK_FLUID:
+        return std::max(1, fluid_coop_lanes(dims, N, 0, per));
+    case AQ_WALK_COMPENSATED:
+        return std::max(1, fluid_coop_lanes(dims, N, 2, per));
+    case AQ_WALK_ELEMENTS: return per ? AQ_EINVAL : elem_lanes(dims, N);
+    case AQ_WALK_LES: return std::max(1, les_lanes(dims, N, per));
+    default: return AQ_EINVAL;
+    }
+}

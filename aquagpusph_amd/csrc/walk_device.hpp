@@ -61,6 +61,9 @@ struct WalkArgs {
 // bits and the neighbour-table entry (0..26) in the top 5.
 constexpr uint32_t PER_KL_SHIFT = 27;
 constexpr uint32_t PER_J_MASK = (1u << PER_KL_SHIFT) - 1u;
+// Particles such a word can name (the group walks; the one-lane walks keep
+// the index alone)
+constexpr uint32_t PER_GROUP_MAX_N = 1u << PER_KL_SHIFT;
 
 // Candidate table of cell c_i: start and prefix count of each neighbour
 // cell in walk order.  Cells known to hold none of the `want` kinds

@@ -445,6 +445,15 @@ AQ_API int aq_check_nr_arith(uint64_t n, uint64_t seed, uint64_t* mismatches);
  * the device sequence against the CPU one. */
 AQ_API int aq_clmath_eval(int op, const float* x, float* y, uint32_t n,
                           void* stream);
+/* Lanes of a wavefront that serve one particle in the default launch of a
+ * cell-parallel walk over N particles of every kind: 1, 4 or 16 (the sums are
+ * bit-identical whichever it is), or AQ_EINVAL.  periodic: in a periodic box.
+ * For tests and tuning. */
+#define AQ_WALK_FLUID 0       /* fused fluid walk */
+#define AQ_WALK_COMPENSATED 1 /* fused fluid walk with compensated sums */
+#define AQ_WALK_ELEMENTS 2    /* boundary-integral kernels of the elements */
+#define AQ_WALK_LES 3         /* LES closure kernels */
+AQ_API int aq_walk_lanes(int kernel, int dims, uint32_t N, int periodic);
 /* Registry keys ("cfd/Interactions.cl:entry", ...) of the HIP kernels. */
 AQ_API int aq_sim_n_registered_kernels(void);
 AQ_API const char* aq_sim_registered_kernel(int i);

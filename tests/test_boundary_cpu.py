@@ -44,6 +44,24 @@ def test_workspace_holds_every_shorter_sort(fn):
     assert f(0) <= sizes[0] and f(ctypes.c_uint32(2 ** 32 - 1)) > sizes[-1]
 
 
+def test_lanes_per_particle_of_the_walks():
+    """Several lanes per particle only where the group walk can name every
+    candidate: 27 bits of a candidate word in a periodic box."""
+    f = _lib.lib().aq_walk_lanes
+    fluid, comp, elem, les = range(4)
+    for kernel in (fluid, comp, les):
+        for dims in (2, 3):
+            for n in (1 << 27, (1 << 27) + 1, (1 << 28) - 1):
+                lanes = f(kernel, dims, n, 1)
+                assert lanes == (4 if n <= 1 << 27 and dims == 2 else 1)
+            assert f(kernel, dims, 1000, 1) == 16
+    assert f(fluid, 2, (1 << 28) - 1, 0) == 4
+    assert [f(les, 3, n, 0) for n in (24000, 24001, 250000, 250001)] == \
+        [16, 4, 4, 1]
+    assert f(elem, 3, 1000, 1) == f(fluid, 4, 1000, 0) == -1
+    assert f(fluid, 3, 1 << 28, 0) == f(9, 3, 1000, 0) == -1
+
+
 def _resolve(xml, dims):
     L = _lib.lib()
     L.aq_xml_resolve.argtypes = [ctypes.c_char_p, ctypes.c_int,
