@@ -11,8 +11,11 @@
 //
 // The per-particle kernels are bound by latency and divergence: each lane
 // reads its own candidates one at a time (256 accepted of 1728 in 3D).  At
-// 150 k particles in 3D: Shepard 841 -> 376 us, interactions 1278 ->
-// 523 us, lap p 935 -> 412 us.
+// 150 k particles in 3D: Shepard 841 -> 383 us, interactions 1278 ->
+// 519 us, lap p 935 -> 381 us.  A wavefront pays some 2 us per cell among its
+// particles, though, so where they are scattered over many cells, or where
+// the per-particle form fills the chip, that form is the faster one: a large
+// launch comes in both, and the device takes one (pair_groups_edges).
 #include "aq_device.hpp"
 #include "aq_internal.hpp"
 #include "coop_device.hpp"
@@ -22,12 +25,25 @@ namespace aq {
 
 namespace {
 
+// Largest launch with 16 lanes per particle, 4 above.  Shepard /
+// interactions in us, 16 and 4 lanes:
+//   2D, 16 per cell   20 k  19 /  25  34 /  45    48 k  33 /  46   38 /  51
+//                     64 k  40 /  57  53 /  67   150 k  77 / 113   87 / 117
+//   3D, 64 per cell   20 k  79 / 127 138 / 181    48 k 137 / 213  168 / 224
+//                     64 k 163 / 263 183 / 252   150 k 320 / 548  386 / 513
+constexpr uint32_t GROUPS_16 = 50000;
+// Largest launch by groups whatever the cells hold: the per-particle form
+// gains 5 us at most there (20 k particles, 0.3 per cell, 19 against 14 us),
+// about what its launch takes.
+constexpr uint32_t GROUPS_ALL = 16384;
+
 // Link-list of the caller
 struct RunArgs {
     const uint32_t* icell;
     const uint32_t* ihoc;
     const uint32_t* n_cells;
     uint32_t N;
+    uint32_t edges;  // pair_groups_edges
 };
 
 // neighbour_table without a cell list: a cell's particles are the run of
@@ -114,6 +130,7 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
     const uint32_t b = (blockIdx.x % NRANGE) * (gridDim.x / NRANGE) +
                        blockIdx.x / NRANGE;
     if (b >= nblocks) return;
+    if (w.edges && sampled_cells(w.icell, w.N) > w.edges) return;  // sparse
     const uint32_t i = (b * WC_WAVES + (uint32_t)wv) * OW + (uint32_t)o;
     uint32_t c = 0;
     bool own = false;
@@ -324,8 +341,6 @@ template <int D> struct PolLapP {
     }
 };
 
-// 16 lanes per particle while that takes no more wavefronts than the chip
-// holds at once (4096 of 4 particles), 4 above
 template <int D, class Pol>
 void launch_runs(const Pol& pol, const int32_t* imove, const float* r,
                  const RunArgs& w, aq_defs d, hipStream_t s)
@@ -336,11 +351,37 @@ void launch_runs(const Pol& pol, const int32_t* imove, const float* r,
                            dim3(64 * WC_WAVES), 0, s, pol, imove, r, w,
                            support_threshold(d.H), nb);
     };
-    if (w.N <= 16384u) go(run_group_k<D, 16, Pol>, 16);
+    if (w.N <= GROUPS_16) go(run_group_k<D, 16, Pol>, 16);
     else go(run_group_k<D, 4, Pol>, 4);
 }
 
 }  // namespace
+
+// Sampled cell boundaries (sampled_cells) up to which the groups take the
+// launch and above which the per-particle kernels do; 0: always the groups.
+// The line lies at `few` particles per cell.  aq_shepard in us by the groups
+// (4 lanes; 48 k: 16) / per particle, by particles per cell:
+//   2D          0.3       2          6          10         16         30
+//      48 k   36 / 14   32 / 29    28 / 49    29 / 73    33 / 94   43 / 142
+//      64 k   67 / 14   55 / 29    52 / 49    40 / 68    53 / 94   59 / 142
+//     150 k  159 / 19  123 / 35   111 / 65    90 / 82    89 / 115 112 / 171
+//     300 k  279 / 35  213 / 48   143 / 81   161 / 107  151 / 139 194 / 223
+//     1.0 M  853 / 74  629 / 139  425 / 246  433 / 312  437 / 370 576 / 689
+//   3D          0.3       2          5           8         12         64
+//      48 k   64 / 34   59 / 67    56 / 108   60 / 146   57 / 190 147 / 685
+//      64 k  111 / 35  102 / 69    98 / 114   75 / 156   87 / 193 183 / 709
+//     150 k  269 / 40  227 / 89   209 / 168  156 / 213  182 / 248 384 / 780
+//     300 k  472 / 80  371 / 172  315 / 280  277 / 370  298 / 392 674 / 1440
+//     1.0 M 1459 / 180 1089 / 362 875 / 582  787 / 776  798 / 988 2088 / 3357
+// The form not taken adds 2 to 4 us (10 us for the 62 k idle wavefronts of
+// 1 M scattered particles).
+uint32_t pair_groups_edges(int dims, uint32_t N)
+{
+    if (N <= GROUPS_ALL) return 0;
+    const uint32_t few = dims == 2 ? std::min(18u, N / 16000u + 1u)
+                                   : std::min(8u, N / 25000u + 1u);
+    return CELL_SAMPLE / few;
+}
 
 // Each returns false, launching nothing, beyond the 32-bit byte offsets of
 // the candidate loads.
@@ -351,7 +392,7 @@ bool shepard_groups(int dims, const int32_t* imove, const float* r,
                     hipStream_t s)
 {
     if (N >= (1u << 28)) return false;
-    const RunArgs w{ icell, ihoc, n_cells, N };
+    const RunArgs w{ icell, ihoc, n_cells, N, pair_groups_edges(dims, N) };
 #define AQ_SH(DD, KK)                                                          \
     launch_runs<DD>(PolShepard<DD, KK>{ r, rho, m, shepard, d.H, d.CONW },     \
                     imove, r, w, d, s)
@@ -374,7 +415,7 @@ bool interactions_groups(int dims, const int32_t* imove, const float* r,
                          aq_defs d, hipStream_t s)
 {
     if (N >= (1u << 28)) return false;
-    const RunArgs w{ icell, ihoc, n_cells, N };
+    const RunArgs w{ icell, ihoc, n_cells, N, pair_groups_edges(dims, N) };
     if (dims == 2)
         launch_runs<2>(PolInteractions<2>{ r, u, rho, m, p, grad_p, lap_u,
                                            div_u, d.H, d.CONF,
@@ -395,7 +436,7 @@ bool lapp_groups(int dims, const int32_t* imove, const float* r,
                  hipStream_t s)
 {
     if (N >= (1u << 28)) return false;
-    const RunArgs w{ icell, ihoc, n_cells, N };
+    const RunArgs w{ icell, ihoc, n_cells, N, pair_groups_edges(dims, N) };
     if (dims == 2)
         launch_runs<2>(PolLapP<2>{ r, rho, m, p, lap_p, d.H, d.CONF }, imove,
                        r, w, d, s);

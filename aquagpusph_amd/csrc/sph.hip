@@ -938,6 +938,14 @@ struct LLArgs {
     // the kinds each cell holds
     const uint32_t* cell_end = nullptr;
     uint32_t flagged = 0;
+    // not 0: nothing to do unless the cells are sparse, with more sampled
+    // boundaries than this (pair_groups_edges)
+    uint32_t edges = 0;
+    // by whole wavefronts, before any lane returns
+    __device__ __forceinline__ bool dense() const
+    {
+        return edges && sampled_cells(icell, N) <= edges;
+    }
 };
 
 // walk() over the cell list when one is given: the same candidates in the
@@ -1043,6 +1051,7 @@ __global__ void __launch_bounds__(BS)
               float smax, int cfd, Sel sel)
 {
     AQ_STATUS_SKIP;
+    if (ll.dense()) return;
     auto excl = [&](int v) { return (cfd & 1) ? (v != 1) : (v >= 3); };
     // cfd: fluid candidates only
     const uint32_t want = (cfd & 1) ? AQ_CELL_FLUID : 0u;
@@ -1078,6 +1087,7 @@ __global__ void __launch_bounds__(BS)
                    float* __restrict__ div_u, LLArgs ll, float H, float CONF,
                    float smax, int lap)
 {
+    if (ll.dense()) return;
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= ll.N) return;
     AQ_STATUS_SKIP;
@@ -1125,6 +1135,7 @@ __global__ void __launch_bounds__(BS)
            const float* __restrict__ p, float* __restrict__ lap_p, LLArgs ll,
            float H, float CONF, float smax)
 {
+    if (ll.dense()) return;
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= ll.N) return;
     AQ_STATUS_SKIP;
@@ -1828,6 +1839,7 @@ void launch_bi_interp_shepard(const uint32_t* iset, const int32_t* imove,
 }
 
 // pair_groups.hip
+uint32_t pair_groups_edges(int dims, uint32_t N);
 bool shepard_groups(int dims, const int32_t* imove, const float* r,
                     const float* rho, const float* m, float* shepard,
                     uint32_t N, const uint32_t* icell, const uint32_t* ihoc,
@@ -1845,6 +1857,50 @@ bool lapp_groups(int dims, const int32_t* imove, const float* r,
                  const uint32_t* ihoc, const uint32_t* n_cells, aq_defs d,
                  hipStream_t s);
 
+// A pair kernel of the C ABI: its group form, groups(), false where it
+// launched nothing; and its per-particle form, single(ll), where that may be
+// the one for the caller's cells (the device finds out which of the two).
+template <class Groups, class Single>
+static void pairs_by_groups(int dims, uint32_t N, const uint32_t* icell,
+                            const uint32_t* ihoc, const uint32_t* n_cells,
+                            Groups groups, Single single)
+{
+    LLArgs ll = mkll(icell, ihoc, n_cells, nullptr, N);
+    if (groups()) {
+        ll.edges = pair_groups_edges(dims, N);
+        if (!ll.edges) return;
+    }
+    single(ll);
+}
+
+static void shepard_ll(int dims, const int32_t* imove, const float* r,
+                       const float* rho, const float* m, float* shepard,
+                       const LLArgs& ll, const Sel& sel, aq_defs d, int cfd,
+                       hipStream_t s)
+{
+    auto* ker = (dims == 2) ? shepard_k<2> : shepard_k<3>;
+    hipLaunchKernelGGL(ker, sel_grid((const void*)ker, sel, ll.N), dim3(BS),
+                       0, s, imove, r, rho, m, shepard, ll, d.H, d.CONW,
+                       support_threshold(d.H), cfd, sel);
+}
+static void interactions_ll(int dims, const int32_t* imove, const float* r,
+                            const float* u, const float* rho, const float* m,
+                            const float* p, float* grad_p, float* lap_u,
+                            float* div_u, const LLArgs& ll, aq_defs d,
+                            hipStream_t s)
+{
+    AQ_DISPATCH(dims, interactions_k, AQ_GRID(ll.N), imove, r, u, rho, m, p,
+                grad_p, lap_u, div_u, ll, d.H, d.CONF, support_threshold(d.H),
+                d.lap_formulation);
+}
+static void lapp_ll(int dims, const int32_t* imove, const float* r,
+                    const float* rho, const float* m, const float* p,
+                    float* lap_p, const LLArgs& ll, aq_defs d, hipStream_t s)
+{
+    AQ_DISPATCH(dims, lapp_k, AQ_GRID(ll.N), imove, r, rho, m, p, lap_p, ll,
+                d.H, d.CONF, support_threshold(d.H));
+}
+
 void launch_shepard(int dims, const int32_t* imove, const float* r,
                     const float* rho, const float* m, float* shepard,
                     uint32_t N, const uint32_t* icell, const uint32_t* ihoc,
@@ -1852,13 +1908,11 @@ void launch_shepard(int dims, const int32_t* imove, const float* r,
                     aq_defs d, int cfd, hipStream_t s, const PartWalk* pw)
 {
     // with the fluid done elsewhere (cfd & 2) it runs on -3 <= imove <= 0
-    const LLArgs ll = mkll_pw(icell, ihoc, n_cells, status, N, pw);
-    const Sel sel = select_parts((cfd & 2) ? pw : nullptr, imove, nullptr,
-                                 -3, 0, N, s);
-    auto* ker = (dims == 2) ? shepard_k<2> : shepard_k<3>;
-    hipLaunchKernelGGL(ker, sel_grid((const void*)ker, sel, N), dim3(BS), 0,
-                       s, imove, r, rho, m, shepard, ll, d.H, d.CONW,
-                       support_threshold(d.H), cfd, sel);
+    shepard_ll(dims, imove, r, rho, m, shepard,
+               mkll_pw(icell, ihoc, n_cells, status, N, pw),
+               select_parts((cfd & 2) ? pw : nullptr, imove, nullptr, -3, 0,
+                            N, s),
+               d, cfd, s);
 }
 void launch_interactions(int dims, const int32_t* imove, const float* r,
                          const float* u, const float* rho, const float* m,
@@ -1867,9 +1921,8 @@ void launch_interactions(int dims, const int32_t* imove, const float* r,
                          const uint32_t* ihoc, const uint32_t* n_cells,
                          const uint32_t* status, aq_defs d, hipStream_t s)
 {
-    AQ_DISPATCH(dims, interactions_k, AQ_GRID(N), imove, r, u, rho, m, p,
-                grad_p, lap_u, div_u, mkll(icell, ihoc, n_cells, status, N),
-                d.H, d.CONF, support_threshold(d.H), d.lap_formulation);
+    interactions_ll(dims, imove, r, u, rho, m, p, grad_p, lap_u, div_u,
+                    mkll(icell, ihoc, n_cells, status, N), d, s);
 }
 void launch_lapp(int dims, const int32_t* imove, const float* r,
                  const float* rho, const float* m, const float* p,
@@ -1877,9 +1930,8 @@ void launch_lapp(int dims, const int32_t* imove, const float* r,
                  const uint32_t* ihoc, const uint32_t* n_cells,
                  const uint32_t* status, aq_defs d, hipStream_t s)
 {
-    AQ_DISPATCH(dims, lapp_k, AQ_GRID(N), imove, r, rho, m, p, lap_p,
-                mkll(icell, ihoc, n_cells, status, N), d.H, d.CONF,
-                support_threshold(d.H));
+    lapp_ll(dims, imove, r, rho, m, p, lap_p,
+            mkll(icell, ihoc, n_cells, status, N), d, s);
 }
 void launch_sensors(int dims, const int32_t* imove, const float* r,
                     const float* m, float* u, float* rho, float* p,
@@ -2244,11 +2296,18 @@ AQ_API int aq_shepard(int dims, const int32_t* imove, const float* r,
         check_defs(defs);
         if (!N) return;
         AQ_PTRS(imove, r, rho, m, shepard, icell, ihoc, n_cells);
-        if (!shepard_groups(dims, imove, r, rho, m, shepard, N, icell, ihoc,
-                            n_cells, defs, cfd_variant, S(stream)))
-            launch_shepard(dims, imove, r, rho, m, shepard, N, icell, ihoc,
-                           n_cells, nullptr, defs, cfd_variant ? 1 : 0,
-                           S(stream), nullptr);
+        const int cfd = cfd_variant ? 1 : 0;
+        pairs_by_groups(
+            dims, N, icell, ihoc, n_cells,
+            [&] {
+                return shepard_groups(dims, imove, r, rho, m, shepard, N,
+                                      icell, ihoc, n_cells, defs, cfd,
+                                      S(stream));
+            },
+            [&](const LLArgs& ll) {
+                shepard_ll(dims, imove, r, rho, m, shepard, ll,
+                           Sel{ nullptr, nullptr }, defs, cfd, S(stream));
+            });
     });
 }
 
@@ -2265,12 +2324,17 @@ AQ_API int aq_interactions(int dims, const int32_t* imove, const float* r,
         if (!N) return;
         AQ_PTRS(imove, r, u, rho, m, p, grad_p, lap_u, div_u, icell, ihoc,
                 n_cells);
-        if (!interactions_groups(dims, imove, r, u, rho, m, p, grad_p, lap_u,
-                                 div_u, N, icell, ihoc, n_cells, defs,
-                                 S(stream)))
-            launch_interactions(dims, imove, r, u, rho, m, p, grad_p, lap_u,
-                                div_u, N, icell, ihoc, n_cells, nullptr, defs,
-                                S(stream));
+        pairs_by_groups(
+            dims, N, icell, ihoc, n_cells,
+            [&] {
+                return interactions_groups(dims, imove, r, u, rho, m, p,
+                                           grad_p, lap_u, div_u, N, icell,
+                                           ihoc, n_cells, defs, S(stream));
+            },
+            [&](const LLArgs& ll) {
+                interactions_ll(dims, imove, r, u, rho, m, p, grad_p, lap_u,
+                                div_u, ll, defs, S(stream));
+            });
     });
 }
 
@@ -2285,10 +2349,16 @@ AQ_API int aq_lapp(int dims, const int32_t* imove, const float* r,
         check_defs(defs);
         if (!N) return;
         AQ_PTRS(imove, r, rho, m, p, lap_p, icell, ihoc, n_cells);
-        if (!lapp_groups(dims, imove, r, rho, m, p, lap_p, N, icell, ihoc,
-                         n_cells, defs, S(stream)))
-            launch_lapp(dims, imove, r, rho, m, p, lap_p, N, icell, ihoc,
-                        n_cells, nullptr, defs, S(stream));
+        pairs_by_groups(
+            dims, N, icell, ihoc, n_cells,
+            [&] {
+                return lapp_groups(dims, imove, r, rho, m, p, lap_p, N, icell,
+                                   ihoc, n_cells, defs, S(stream));
+            },
+            [&](const LLArgs& ll) {
+                lapp_ll(dims, imove, r, rho, m, p, lap_p, ll, defs,
+                        S(stream));
+            });
     });
 }
 

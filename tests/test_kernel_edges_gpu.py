@@ -371,12 +371,15 @@ def _check_abi_pair_kernels(rng, dims, lap, h, r, u, rho, m, p, im):
         np.testing.assert_array_equal(a.cpu().numpy(), b)
 
 
-# around the line between 16 and 4 lanes per particle, single particles and
-# cells of more than 64
+# single particles, cells of more than 64, around the lines of the launch by
+# groups alone (16384) and between 16 and 4 lanes per particle (50000), and
+# about one particle per cell beyond them (the per-particle form)
 @pytest.mark.parametrize("dims,n,cell,lap", [
     (2, 1, 3, 1), (2, 65, 3, 2), (2, 16384, 4, 1), (2, 16385, 4, 2),
     (2, 30011, 12, 1), (3, 1, 3, 1), (3, 63, 2, 1), (3, 5000, 6, 2),
-    (3, 16384, 4, 1), (3, 20011, 4, 1)])
+    (3, 16384, 4, 1), (3, 20011, 4, 1), (2, 50000, 4, 2), (2, 50001, 5, 1),
+    (3, 50001, 4, 2), (2, 16385, 1, 1), (2, 60001, 1, 2), (3, 50001, 1, 1),
+    (3, 110003, 1, 2)])
 def test_abi_pair_kernels_match_oracle(cuda, dims, n, cell, lap):
     """The pair kernels of the C ABI on disordered particles of every kind,
     about cell^dims of them per cell."""
@@ -396,15 +399,15 @@ def test_abi_pair_kernels_match_oracle(cuda, dims, n, cell, lap):
     _check_abi_pair_kernels(rng, dims, lap, h, r, u, rho, m, p, im)
 
 
-@pytest.mark.parametrize("dims,sites,lap", [(2, 60, 1), (2, 800, 2),
-                                            (3, 60, 2), (3, 800, 1)])
+@pytest.mark.parametrize("dims,sites,lap", [(2, 60, 1), (2, 2100, 2),
+                                            (3, 60, 2), (3, 2100, 1)])
 def test_abi_pairs_at_the_edge_of_the_support(cuda, dims, sites, lap):
     """Pairs within 4e-5 of the support radius (the walk's distance test
     accepts some of those beyond it) whose neighbour has an infinite, NaN or
     zero field, and particles that meet themselves with such a field: a pair
     out of reach, or a particle with itself, adds nothing.  Each site is a
     bunch of 24 particles and a broken one a support radius away; 60 sites
-    run with 16 lanes per particle, 800 with 4."""
+    run with 16 lanes per particle, 2100 with 4."""
     rng = np.random.default_rng(sites + dims)
     vs = 2 if dims == 2 else 4
     h = np.float32(0.05)
