@@ -129,7 +129,15 @@ def _stir(case, seed):
     return case
 
 
-# sizes on both sides of the lines between 16, 4 and one lane per particle
+# aq_walk_lanes: the walks and the lanes per particle of their launches
+FLUID, KAHAN, ELEMENTS, LES = range(4)
+
+
+def _lanes(kernel, case, periodic=0):
+    return _lib.lib().aq_walk_lanes(kernel, case["dims"], case["N"], periodic)
+
+
+# sizes on both sides of the lines between 16 and 4 lanes per particle
 @pytest.mark.parametrize("dims,dr,kind", [
     (2, 0.06, "wall"), (2, 0.011, "wall"), (2, 0.0028, "wall"),
     (2, 0.011, "kahan"), (2, 0.0031, "kahan"), (3, 0.05, "wall"),
@@ -151,6 +159,8 @@ def test_lanes_per_particle_are_bit_identical(cuda, tmp_path, monkeypatch,
         case = cases.dam_break(dims, dr)
         if kind == "kahan":
             pres = pres + ("resources/Presets/precision.xml",)
+    assert _lanes(KAHAN if kind == "kahan" else FLUID, case,
+                  kind == "box") > 1
     case = _stir(case, 7)
     extra = ""
     if kind == "morris":
@@ -166,6 +176,35 @@ def test_lanes_per_particle_are_bit_identical(cuda, tmp_path, monkeypatch,
     want = _run(tmp_path, case, pres, "one")
     for k in want:
         np.testing.assert_array_equal(got[k], want[k], err_msg=k)
+
+
+# just above the lines to one lane per particle
+@pytest.mark.parametrize("dr,kahan", [(0.0083, False), (0.01, True)])
+def test_one_lane_walk_matches_oracle(cuda, tmp_path, dr, kahan):
+    """The fused walk with one lane per particle, as launched by default, and
+    the element kernels over its near list against the oracle's float32
+    walk, bit for bit: 3D dam breaks of 252,576 and, with compensated sums,
+    153,600 particles."""
+    from aquagpusph_amd import casefiles, cases
+    from aquagpusph_amd.sim import Simulation
+    from oracle import pipeline as op
+    case = _stir(cases.dam_break(3, dr), 13)
+    assert _lanes(KAHAN if kahan else FLUID, case) == 1
+    pres = casefiles.PBI_PRESETS
+    if kahan:
+        pres = pres + ("resources/Presets/precision.xml",)
+    sim = Simulation(casefiles.write_case(case, str(tmp_path), load=False,
+                                          presets=pres), 3)
+    casefiles.upload(sim, case)
+    o = op.OracleSim(case, precision=kahan)
+    for _ in range(2):
+        o.step()
+    sim.step(2)
+    for k in ("id", "r", "u", "rho", "p", "dudt", "drhodt", "shepard",
+              "grad_p", "lap_u", "div_u", "lap_p"):
+        np.testing.assert_array_equal(
+            sim.get(k).ravel().view(o.f[k].dtype), o.f[k].ravel(), err_msg=k)
+    sim.close()
 
 
 # 16, 4 and one lane per particle in a periodic box, one with relaxed math
@@ -212,16 +251,18 @@ def test_fluid_pairs_at_the_edge_of_the_support(cuda, tmp_path, dims, n,
 
 # element kernels: 16 lanes per owner below 100 k (2D) / 600 k (3D)
 # particles, 4 above; wall edges and corners hold more than one group
-@pytest.mark.parametrize("dims,dr,hfac", [(2, 0.06, 2.0), (2, 0.011, 2.0),
-                                          (2, 0.00135, 2.0), (3, 0.05, 2.0),
-                                          (3, 0.031, 3.3), (3, 0.0061, 2.0)])
+@pytest.mark.parametrize("dims,dr,hfac,lanes", [
+    (2, 0.06, 2.0, 16), (2, 0.011, 2.0, 16), (2, 0.00135, 2.0, 4),
+    (3, 0.05, 2.0, 16), (3, 0.031, 3.3, 16), (3, 0.0061, 2.0, 16),
+    (3, 0.0059, 2.0, 4)])
 def test_element_groups_match_one_lane_walks(cuda, tmp_path, monkeypatch,
-                                             dims, dr, hfac):
+                                             dims, dr, hfac, lanes):
     """The boundary-integral element kernels with 4 or 16 lanes per owner
     over the owner, wet and near lists against one lane per owner over every
     cell (AQ_BI_WALK=cells), bit for bit."""
     from aquagpusph_amd import casefiles, cases
     case = _stir(cases.dam_break(dims, dr, hfac=hfac), 11)
+    assert _lanes(ELEMENTS, case) == lanes
     got = _run(tmp_path, case, casefiles.PBI_PRESETS, "groups", 2)
     monkeypatch.setenv("AQ_BI_WALK", "cells")
     want = _run(tmp_path, case, casefiles.PBI_PRESETS, "cells", 2)
@@ -229,9 +270,10 @@ def test_element_groups_match_one_lane_walks(cuda, tmp_path, monkeypatch,
         np.testing.assert_array_equal(got[k], want[k], err_msg=k)
 
 
-@pytest.mark.parametrize("dims,n", [(2, 23), (2, 150), (3, 17), (3, 30),
-                                    (3, 63)])
-def test_les_groups_match_oracle(cuda, tmp_path, dims, n):
+@pytest.mark.parametrize("dims,n,lanes", [(2, 23, 16), (2, 150, 4),
+                                          (3, 17, 16), (3, 30, 4),
+                                          (3, 63, 1)])
+def test_les_groups_match_oracle(cuda, tmp_path, dims, n, lanes):
     """The LES gradient and viscous term (periodic box, Smagorinsky) with 16
     and with 4 lanes per particle (2D above 16 k, 3D above 24 k particles)
     and with one (3D above 250 k: 63^3 = 250,047) against the oracle's
@@ -240,6 +282,7 @@ def test_les_groups_match_oracle(cuda, tmp_path, dims, n):
     from aquagpusph_amd.sim import Simulation
     from oracle import pipeline as op
     case = _stir(cases.periodic_box(dims, n), 5)
+    assert _lanes(LES, case, 1) == lanes
     sim = Simulation(casefiles.write_case(
         case, str(tmp_path), load=False, presets=casefiles.PPER_PRESETS +
         ("resources/Presets/cfd/LES-smagorinsky.xml",)), dims)
@@ -256,18 +299,16 @@ def test_les_groups_match_oracle(cuda, tmp_path, dims, n):
     sim.close()
 
 
-# 16, 4 and one lane per particle inside walls (particles with the elements)
-@pytest.mark.parametrize("dims,dr,lo,hi", [
-    (2, 0.011, 0, 16000), (3, 0.0187, 24000, 250000),
-    (3, 0.0083, 250000, 1 << 28)])
-def test_les_walls_match_oracle(cuda, tmp_path, dims, dr, lo, hi):
+@pytest.mark.parametrize("dims,dr,lanes", [(2, 0.011, 16), (3, 0.0187, 4),
+                                           (3, 0.0083, 1)])
+def test_les_walls_match_oracle(cuda, tmp_path, dims, dr, lanes):
     """The LES kernels of a dam break with its walls (no periodic images)
     against the oracle's float32 walk, bit for bit."""
     from aquagpusph_amd import casefiles, cases
     from aquagpusph_amd.sim import Simulation
     from oracle import pipeline as op
     case = _stir(cases.dam_break(dims, dr), 5)
-    assert lo < case["N"] <= hi
+    assert _lanes(LES, case) == lanes
     sim = Simulation(casefiles.write_case(
         case, str(tmp_path), load=False, presets=casefiles.PBI_PRESETS +
         ("resources/Presets/cfd/LES-smagorinsky.xml",)), dims)
