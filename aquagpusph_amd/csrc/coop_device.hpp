@@ -8,7 +8,7 @@
 //            instructions (dist_tile); Q == 16: lane q tests the survivors
 //            q, q + 16, ..., their places in the list from ballots.
 //   consume  when a list has no room for another chunk (and at the end),
-//            the lanes of every particle with Q B listed take its next Q B,
+//            the lanes of every particle with Q listed take its next Q,
 //            evaluate their terms, and all Q lanes add the terms in list
 //            order, each term broadcast from its lane by a DPP modifier of
 //            the addition: the Q copies of the sums stay equal, and every
@@ -50,7 +50,7 @@ __device__ __forceinline__ void each_lane(float v, F f)
     }
 }
 
-template <int Q, int B, bool PER> struct CoopLds {
+template <int Q, bool PER> struct CoopLds {
     uint32_t start[27];
     uint32_t cum[28];
     // Q == 4: see dist_tile; the gap after each 16 records holds their
@@ -155,11 +155,11 @@ __device__ __forceinline__ uint32_t dist_bits(uint64_t m, int g)
 // The test runs on coordinates relative to the box centre with the margin of
 // ring_walk's LOOSE form, so it accepts a thin shell beyond the support:
 // the callers repeat the exact test (s <= smax) on every pair.
-// round(n, cw): one round, in which lane q of the group takes the list
-// entries q + Q b < n (cw[b]); called by every lane.
-template <int D, int Q, int B, bool PER, class Round>
+// round(n, cw): one round, in which lane q of the group takes the list entry
+// q < n (cw); called by every lane.
+template <int D, int Q, bool PER, class Round>
 __device__ __forceinline__ void
-coop_list_walk(CoopLds<Q, B, PER>& L, int lane, uint32_t total,
+coop_list_walk(CoopLds<Q, PER>& L, int lane, uint32_t total,
                const f3& r_i, bool act, const f3& bmin, const f3& bmax,
                float smax, const float* __restrict__ r,
                const int* __restrict__ imove, int kind, bool flag_el,
@@ -181,7 +181,7 @@ coop_list_walk(CoopLds<Q, B, PER>& L, int lane, uint32_t total,
     const float ai = dot<D>(rio, rio);
     int kl = 0;         // neighbour cell of the lane's next candidate
     uint32_t head = 0, pend = 0;  // the particle's ring: first entry, entries
-    constexpr uint32_t CAP = CoopLds<Q, B, PER>::CAP;
+    constexpr uint32_t CAP = CoopLds<Q, PER>::CAP;
     bool eln = false;
     // Q == 4, lane (g, o16): the B operand and threshold of particle o16
     // and the entries its list has taken
@@ -219,13 +219,8 @@ coop_list_walk(CoopLds<Q, B, PER>& L, int lane, uint32_t total,
     auto consume = [&](uint32_t most, uint32_t least) {
         if (__ballot(pend >= most) == 0) return;
         do {
-            const uint32_t n =
-                pend >= least ? min(pend, (uint32_t)(Q * B)) : 0u;
-            uint32_t cw[B];
-#pragma unroll
-            for (int b = 0; b < B; b++)
-                cw[b] = list[(head + (uint32_t)(q + Q * b)) & (CAP - 1)];
-            round(n, cw);
+            const uint32_t n = pend >= least ? min(pend, (uint32_t)Q) : 0u;
+            round(n, list[(head + (uint32_t)q) & (CAP - 1)]);
             head += n;
             pend -= n;
         } while (__ballot(pend >= most) != 0);
@@ -350,7 +345,7 @@ coop_list_walk(CoopLds<Q, B, PER>& L, int lane, uint32_t total,
             }
         }
         lds_order();
-        consume(CAP - 63, Q * B);  // room for the next chunk
+        consume(CAP - 63, Q);  // room for the next chunk
     }
     consume(1, 1);
     // every lane of the group learns what one of its lanes saw

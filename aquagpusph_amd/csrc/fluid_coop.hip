@@ -23,7 +23,7 @@ namespace {
 // 1 for t = 0, 1, ..., OW = 64 / Q.  nlist gets one entry per item with a
 // near particle: the runs of particles of different items do not overlap,
 // so BI Interactions meets every near particle once.
-template <int D, int SHEP, int MATH, bool PER, int Q, int B>
+template <int D, int SHEP, int MATH, bool PER, int Q>
 __global__ void __launch_bounds__(64 * WC_WAVES)
     fluid_coop_k(const int* __restrict__ imove, const float* __restrict__ r,
                  const float* __restrict__ u, const float* __restrict__ rho,
@@ -40,11 +40,11 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
 {
     constexpr int OW = 64 / Q;
     const bool lapp = lapp_ != 0;
-    __shared__ CoopLds<Q, B, PER> lds[WC_WAVES];
+    __shared__ CoopLds<Q, PER> lds[WC_WAVES];
     const int lane = threadIdx.x & 63;
     const int wv = threadIdx.x >> 6;
     const int q = lane & (Q - 1), o = lane / Q;
-    CoopLds<Q, B, PER>& L = lds[wv];
+    CoopLds<Q, PER>& L = lds[wv];
     if (w.status && (*w.status & 1u)) return;
     const uint32_t n_items = uni(*w.n_heads) * S;
     const float eps = 1E-8f * H;
@@ -120,63 +120,52 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
             // of the relative test's shell beyond the support (zero mass):
             // the sums are never -0 (they start at +0, or 1, and an exact
             // cancellation rounds to +0), so +-0 leaves them unchanged.
-            auto round = [&](uint32_t n, const uint32_t (&cw)[B]) {
-                f3 rc[B], uc[B];
-                float mc[B], rhoc[B], pc[B];
-#pragma unroll
-                for (int b = 0; b < B; b++) {
-                    if ((uint32_t)(q + Q * b) >= n) continue;
-                    const uint32_t j = PER ? cw[b] & PER_J_MASK : cw[b];
-                    rc[b] = rjof(j, PER ? cw[b] >> PER_KL_SHIFT : 0u);
-                    mc[b] = ldf_o(m, j);
-                    rhoc[b] = ldf_o(rho, j);
-                    pc[b] = ldf_o(p, j);
-                    uc[b] = ldv_o<D>(u, j);
-                }
-#pragma unroll
-                for (int b = 0; b < B; b++) {
-                    PairTerms t{ 0.f, 0.f, 0.f, 0.f, 0.f };
-                    f3 g = { 0.f, 0.f, 0.f }, l = { 0.f, 0.f, 0.f };
-                    if ((uint32_t)(q + Q * b) < n) {
-                        const f3 r_ij = sub<D>(rc[b], r_i);
-                        const float s = dot<D>(r_ij, r_ij);
-                        float m_j = mc[b];
-                        m_j = (s > smax) ? 0.f : m_j;
-                        const f3 u_ij = sub<D>(uc[b], u_i);
-                        const float udr = dot<D>(u_ij, r_ij);
-                        const bool fd =
-                            fastdiv && !(((s < 0x1p-96f) & (s != 0.f)) |
-                                         ((udr != 0.f) & (fabsf(udr) < fdT)));
-                        if (fd)
-                            t = fluid_pair<D, SHEP, true>(
-                                lapf, lapp, div_nr(sqrt_nr(s), RH), m_j,
-                                rhoc[b], pc[b], udr, p_i, rho_i, H, CONW,
-                                CONF);
-                        else
-                            t = fluid_pair<D, SHEP, false>(
-                                lapf, lapp, sqrtf(s) / H, m_j, rhoc[b], pc[b],
-                                udr, p_i, rho_i, H, CONW, CONF);
-                        const f3 v = lapf == AQ_LAP_MONAGHAN ? r_ij : u_ij;
-                        g = scl<D>(t.sg, r_ij);
-                        l = scl<D>(t.sl, v);
-                        if (PER && s > smax) {
-                            t = PairTerms{ 0.f, 0.f, 0.f, 0.f, 0.f };
-                            g = l = f3{ 0.f, 0.f, 0.f };
-                        }
+            auto round = [&](uint32_t n, uint32_t cw) {
+                PairTerms t{ 0.f, 0.f, 0.f, 0.f, 0.f };
+                f3 g = { 0.f, 0.f, 0.f }, l = { 0.f, 0.f, 0.f };
+                if ((uint32_t)q < n) {
+                    const uint32_t j = PER ? cw & PER_J_MASK : cw;
+                    const f3 r_ij =
+                        sub<D>(rjof(j, PER ? cw >> PER_KL_SHIFT : 0u), r_i);
+                    const float s = dot<D>(r_ij, r_ij);
+                    float m_j = ldf_o(m, j);
+                    const float rho_j = ldf_o(rho, j);
+                    const float p_j = ldf_o(p, j);
+                    const f3 u_j = ldv_o<D>(u, j);
+                    m_j = (s > smax) ? 0.f : m_j;
+                    const f3 u_ij = sub<D>(u_j, u_i);
+                    const float udr = dot<D>(u_ij, r_ij);
+                    const bool fd =
+                        fastdiv && !(((s < 0x1p-96f) & (s != 0.f)) |
+                                     ((udr != 0.f) & (fabsf(udr) < fdT)));
+                    if (fd)
+                        t = fluid_pair<D, SHEP, true>(
+                            lapf, lapp, div_nr(sqrt_nr(s), RH), m_j, rho_j,
+                            p_j, udr, p_i, rho_i, H, CONW, CONF);
+                    else
+                        t = fluid_pair<D, SHEP, false>(
+                            lapf, lapp, sqrtf(s) / H, m_j, rho_j, p_j, udr,
+                            p_i, rho_i, H, CONW, CONF);
+                    const f3 v = lapf == AQ_LAP_MONAGHAN ? r_ij : u_ij;
+                    g = scl<D>(t.sg, r_ij);
+                    l = scl<D>(t.sl, v);
+                    if (PER && s > smax) {
+                        t = PairTerms{ 0.f, 0.f, 0.f, 0.f, 0.f };
+                        g = l = f3{ 0.f, 0.f, 0.f };
                     }
-                    if constexpr (SHEP == 1)
-                        each_lane<Q>(t.sh, [&](float x) { sh += x; });
-                    acc1(gp.x, cgp.x, g.x);
-                    acc1(gp.y, cgp.y, g.y);
-                    if constexpr (D == 3) acc1(gp.z, cgp.z, g.z);
-                    acc1(lu.x, clu.x, l.x);
-                    acc1(lu.y, clu.y, l.y);
-                    if constexpr (D == 3) acc1(lu.z, clu.z, l.z);
-                    acc1(dv, cdv, t.td);
-                    acc1(lp, clp, t.tl);  // zeros without lap p
                 }
+                if constexpr (SHEP == 1)
+                    each_lane<Q>(t.sh, [&](float x) { sh += x; });
+                acc1(gp.x, cgp.x, g.x);
+                acc1(gp.y, cgp.y, g.y);
+                if constexpr (D == 3) acc1(gp.z, cgp.z, g.z);
+                acc1(lu.x, clu.x, l.x);
+                acc1(lu.y, clu.y, l.y);
+                if constexpr (D == 3) acc1(lu.z, clu.z, l.z);
+                acc1(dv, cdv, t.td);
+                acc1(lp, clp, t.tl);  // zeros without lap p
             };
-            coop_list_walk<D, Q, B, PER>(
+            coop_list_walk<D, Q, PER>(
                 L, lane, total, r_i, act, bmin, bmax, smax, r, imove, 0,
                 flag_el, nearw, w.per, round);
             // ---- wall elements (boundary-integral Shepard) ------------------
@@ -185,63 +174,57 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
                     bool self_added = false, unused = false;
                     const uint32_t total_el =
                         neighbour_table<D, PER>(w, c_i, L, lane, AQ_CELL_ELEM);
-                    auto round_el = [&](uint32_t n, const uint32_t (&cw)[B]) {
-#pragma unroll
-                        for (int b = 0; b < B; b++) {
-                            // v: the element's part; on: the particle lies on
-                            // the element (1/2, once)
-                            float v = 0.f;
-                            bool on = false;
-                            if ((uint32_t)(q + Q * b) < n) {
-                                const uint32_t j = cw[b];
-                                const f3 r_ij = sub<D>(ldv_o<D>(r, j), r_i);
-                                const float s = dot<D>(r_ij, r_ij);
-                                const f3 n_j = ldv_o<D>(normal, j);
-                                const f3 t_j = ldv_o<D>(tangent, j);
-                                const f3 b_j = ldv_o<D>(binormal, j);
-                                const float area_j = ldf_o(m, j);
-                                const float qq = sqrtf(s) / H;
-                                const float r_n = dot<D>(r_ij, n_j);
-                                const float r_t = fabsf(dot<D>(r_ij, t_j));
-                                const float r_b = fabsf(dot<D>(r_ij, b_j));
-                                if (s > smax) {
-                                } else if ((r_n > -eps) && (r_n < eps)) {
-                                    const float dr =
-                                        0.55f *
-                                        pow_cl(area_j, 1.f / (DIMS - 1.f));
-                                    on = (r_t <= dr) && (r_b <= dr);
-                                } else {
-                                    v = r_n * CONW * kernelS_P<D>(qq) *
-                                            area_j +
-                                        kernelS_D<D>(fabsf(r_n), r_t, r_b,
-                                                     area_j);
-                                }
-                            }
-                            if (__ballot(on) == 0) {
-                                each_lane<Q>(v, [&](float x) { sh += x; });
+                    auto round_el = [&](uint32_t n, uint32_t j) {
+                        // v: the element's part; on: the particle lies on
+                        // the element (1/2, once)
+                        float v = 0.f;
+                        bool on = false;
+                        if ((uint32_t)q < n) {
+                            const f3 r_ij = sub<D>(ldv_o<D>(r, j), r_i);
+                            const float s = dot<D>(r_ij, r_ij);
+                            const f3 n_j = ldv_o<D>(normal, j);
+                            const f3 t_j = ldv_o<D>(tangent, j);
+                            const f3 b_j = ldv_o<D>(binormal, j);
+                            const float area_j = ldf_o(m, j);
+                            const float qq = sqrtf(s) / H;
+                            const float r_n = dot<D>(r_ij, n_j);
+                            const float r_t = fabsf(dot<D>(r_ij, t_j));
+                            const float r_b = fabsf(dot<D>(r_ij, b_j));
+                            if (s > smax) {
+                            } else if ((r_n > -eps) && (r_n < eps)) {
+                                const float dr =
+                                    0.55f * pow_cl(area_j, 1.f / (DIMS - 1.f));
+                                on = (r_t <= dr) && (r_b <= dr);
                             } else {
-                                // the half angle in its place in the order
-                                float f = on ? 1.f : 0.f;
-                                float xs[Q], fs[Q];
-                                int k = 0;
-                                each_lane<Q>(v, [&](float x) { xs[k++] = x; });
-                                k = 0;
-                                each_lane<Q>(f, [&](float x) { fs[k++] = x; });
+                                v = r_n * CONW * kernelS_P<D>(qq) * area_j +
+                                    kernelS_D<D>(fabsf(r_n), r_t, r_b,
+                                                 area_j);
+                            }
+                        }
+                        if (__ballot(on) == 0) {
+                            each_lane<Q>(v, [&](float x) { sh += x; });
+                        } else {
+                            // the half angle in its place in the order
+                            const float f = on ? 1.f : 0.f;
+                            float xs[Q], fs[Q];
+                            int k = 0;
+                            each_lane<Q>(v, [&](float x) { xs[k++] = x; });
+                            k = 0;
+                            each_lane<Q>(f, [&](float x) { fs[k++] = x; });
 #pragma unroll
-                                for (int e = 0; e < Q; e++) {
-                                    if (fs[e] != 0.f) {
-                                        if (!self_added) {
-                                            self_added = true;
-                                            sh -= 0.5f;
-                                        }
-                                    } else {
-                                        sh += xs[e];
+                            for (int e = 0; e < Q; e++) {
+                                if (fs[e] != 0.f) {
+                                    if (!self_added) {
+                                        self_added = true;
+                                        sh -= 0.5f;
                                     }
+                                } else {
+                                    sh += xs[e];
                                 }
                             }
                         }
                     };
-                    coop_list_walk<D, Q, B, PER>(
+                    coop_list_walk<D, Q, PER>(
                         L, lane, total_el, r_i, act && nearw, bmin, bmax,
                         smax, r, imove, 1, false, unused, w.per, round_el);
                 }
@@ -319,9 +302,9 @@ void launch_fluid_coop(int dims, int shep, bool lapp, int q,
     // a 2D cell holds one group of 16 particles, a 3D cell four
     const uint32_t S = q == 16 ? (dims == 2 ? 4u : 16u)
                                : (dims == 2 ? 1u : 4u);
-#define AQ_CO4(DD, SH, MM, PR, QQ, BB)                                         \
+#define AQ_CO4(DD, SH, MM, PR, QQ)                                             \
     do {                                                                       \
-        auto* ker = fluid_coop_k<DD, SH, MM, PR, QQ, BB>;                      \
+        auto* ker = fluid_coop_k<DD, SH, MM, PR, QQ>;                          \
         const unsigned nb =                                                    \
             std::min(resident_blocks((const void*)ker, 64 * WC_WAVES),         \
                      std::max(1u, blocks_for((size_t)w.N * QQ * 2,             \
@@ -334,8 +317,8 @@ void launch_fluid_coop(int dims, int shep, bool lapp, int q,
     } while (0)
 #define AQ_CO3(DD, SH, MM, PR)                                                 \
     do {                                                                       \
-        if (q == 16) AQ_CO4(DD, SH, MM, PR, 16, 1);                            \
-        else AQ_CO4(DD, SH, MM, PR, 4, 1);                                     \
+        if (q == 16) AQ_CO4(DD, SH, MM, PR, 16);                               \
+        else AQ_CO4(DD, SH, MM, PR, 4);                                        \
     } while (0)
 #define AQ_CO2(DD, SH, MM)                                                     \
     do {                                                                       \

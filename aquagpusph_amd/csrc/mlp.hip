@@ -19,7 +19,8 @@
 //
 // Training is deterministic: every wave sums the gradients of its own
 // fixed tiles in registers and writes one partial per wave; a second
-// kernel adds the partials in wave order; Adam then updates the master copy.
+// kernel adds the partials in one fixed order (mlp_reduce_k); Adam then
+// updates the master copy.
 #include "aq_device.hpp"
 #include "aq_internal.hpp"
 

@@ -120,11 +120,11 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
                 uint32_t nblocks)
 {
     constexpr uint32_t OW = 64 / Q;
-    __shared__ CoopLds<Q, 1, false> lds[WC_WAVES];
+    __shared__ CoopLds<Q, false> lds[WC_WAVES];
     const int lane = threadIdx.x & 63;
     const int wv = threadIdx.x >> 6;
     const int q = lane & (Q - 1), o = lane / Q;
-    CoopLds<Q, 1, false>& L = lds[wv];
+    CoopLds<Q, false>& L = lds[wv];
     // one contiguous stretch of the particles per XCD (workgroup b runs on
     // XCD b % 8), so that the neighbourhoods in flight share its L2
     const uint32_t b = (blockIdx.x % NRANGE) * (gridDim.x / NRANGE) +
@@ -153,10 +153,9 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
         }
         f3 bmin, bmax;
         wave_box<D>(r_i, act, bmin, bmax);
-        auto round = [&](uint32_t n, const uint32_t (&cw)[1]) {
+        auto round = [&](uint32_t n, uint32_t j) {
             typename Pol::Term t = Pol::none();
             if ((uint32_t)q < n) {
-                const uint32_t j = cw[0];
                 const typename Pol::Cand cd = pol.load(j);
                 const f3 r_ij = sub<D>(cd.r, r_i);
                 const float s = dot<D>(r_ij, r_ij);
@@ -172,7 +171,7 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
             pol.template add_group<Q>(st, t);
         };
         bool unused = false;
-        coop_list_walk<D, Q, 1, false>(
+        coop_list_walk<D, Q, false>(
             L, lane, total, r_i, act, bmin, bmax, smax, r, imove, Pol::KIND,
             false, unused, nullptr, round);
         if (act && q == 0) pol.finish(i, st);

@@ -995,11 +995,11 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
 {
     constexpr int OW = 64 / Q;
     using Term = typename Pol::Term;
-    __shared__ CoopLds<Q, 1, PER> lds[WC_WAVES];
+    __shared__ CoopLds<Q, PER> lds[WC_WAVES];
     const int lane = threadIdx.x & 63;
     const int wv = threadIdx.x >> 6;
     const int q = lane & (Q - 1), o = lane / Q;
-    CoopLds<Q, 1, PER>& L = lds[wv];
+    CoopLds<Q, PER>& L = lds[wv];
     if (w.status && (*w.status & 1u)) return;
     const uint32_t n_items =
         (olist ? uni(w.n_heads[count_word]) : uni(*w.n_heads)) * S;
@@ -1036,14 +1036,14 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
             }
             f3 bmin, bmax;
             wave_box<D>(r_i, act, bmin, bmax);
-            auto round = [&](uint32_t n, const uint32_t (&cw)[1]) {
+            auto round = [&](uint32_t n, uint32_t cw) {
                 Term t = Pol::none();
                 if ((uint32_t)q < n) {
-                    const uint32_t j = PER ? cw[0] & PER_J_MASK : cw[0];
+                    const uint32_t j = PER ? cw & PER_J_MASK : cw;
                     auto c = pol.load(j);
                     if constexpr (PER) {
                         const float4 sh =
-                            L.get_shift((int)(cw[0] >> PER_KL_SHIFT));
+                            L.get_shift((int)(cw >> PER_KL_SHIFT));
                         c.r = per_shift<D>(c.r, f3{ sh.x, sh.y, sh.z },
                                            w.per);
                     }
@@ -1061,7 +1061,7 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
                 pol.template add_group<Q>(st, t);
             };
             bool unused = false;
-            coop_list_walk<D, Q, 1, PER>(
+            coop_list_walk<D, Q, PER>(
                 L, lane, total, r_i, act, bmin, bmax, smax, r, imove,
                 Pol::KIND, false, unused, w.per, round);
             if (act && q == 0) pol.finish(i, st);
@@ -1659,8 +1659,8 @@ static uint32_t walk_ranges()
 }
 
 // Workgroups of `ker` that fit on the device at once (all CUs), cached per
-// kernel: the walk hands cells out dynamically, so a grid of exactly that
-// many workgroups keeps every slot busy until the cells run out.
+// kernel: the grid of the walks, which hand out their cells to the wavefronts
+// there are (the one-lane fused walk by counters, the others by stride).
 unsigned resident_blocks(const void* ker, int block)
 {
     static std::mutex mu;

@@ -87,7 +87,8 @@ AQ_API int aq_linklist_icell(int dims, uint32_t* icell, const float* r,
                              void* stream);
 
 /* iHoc + linkList kernels, LinkList.cl.in:32-42 and 92-113, on sorted icell.
- * Launches over ihoc_capacity cells; only cells < n_cells.w are written. */
+ * Only the cells below n_cells.w (and ihoc_capacity) are visited and
+ * written. */
 AQ_API int aq_linklist_ihoc(const uint32_t* icell, uint32_t* ihoc,
                             uint32_t N, const uint32_t* n_cells,
                             uint32_t ihoc_capacity, const uint32_t* status,
