@@ -1845,12 +1845,14 @@ void launch_fluid_pass_cells(int dims, int shep, bool lapp,
 
 
 // ---- launchers of the generic cell kernels ---------------------------------
-// One owner per lane over every non-empty cell (in blocked order when the
-// link-list built it), batched loads.
+// One owner per lane over `olist` (its count in n_heads[count_word]; nullptr:
+// every non-empty cell, in blocked order when the link-list built it),
+// batched loads.
 template <int D, class Pol>
 static void launch_bi_cells(const Pol& pol, const int32_t* imove,
                             const float* r, const CellArgs& c, float smax,
-                            hipStream_t s)
+                            hipStream_t s, const uint32_t* olist = nullptr,
+                            uint32_t count_word = 0)
 {
     AQ_REQUIRE(c.N < (1u << 28), "cell-parallel walk: more than 2^28 particles");
     WalkArgs w{ c.icell,   c.ihoc,   c.n_cells, c.cell_end, c.heads,
@@ -1859,8 +1861,12 @@ static void launch_bi_cells(const Pol& pol, const int32_t* imove,
     auto* ker = cell_kernel_k<D, 8, Pol, Pol::BATCH>;
     const unsigned nb = walk_grid((const void*)ker, c);
     const int nrq = (pol.H >= 0x1p-40f && pol.H <= 0x1p40f) ? 1 : 0;
+    if (!olist) {
+        olist = c.blist;
+        count_word = 0;
+    }
     hipLaunchKernelGGL(ker, dim3(nb), dim3(64 * WC_WAVES), 0, s, pol, imove,
-                       r, w, smax, nrq, c.blist, 0u);
+                       r, w, smax, nrq, olist, count_word);
 }
 
 // The group kernel with `wide` ? 16 : 4 lanes per owner over `olist`
@@ -1869,13 +1875,13 @@ static void launch_bi_cells(const Pol& pol, const int32_t* imove,
 //   BI LapU          3D  29 k particles 46 / 25   394 k 52 / 34
 //                        1.2 M 57 / 62   4.5 M 113 / 126
 //                    2D  21 k 13 / 11   1.2 M (64 tanks) 23 / 28
-//   BI Interactions  3D  29 k 25 / 34   1.2 M 72 / 126   4.5 M 136 / 245
+//   BI Interactions  3D  29 k 26 / 34
 // The elements are few and hold a fifth of their neighbours' particles each,
 // so 16 lanes pay as long as latency rules; fluid owners fill the chip much
-// earlier (les_lanes for the LES kernels).  (Before, in us at 4.5 M / 1.2 M / 29 k: 4 lanes with the terms
-// through LDS and a full wait per segment, LapU 240 / 134 / 127,
-// Interpolation 200 / 119 / 113; one lane per owner, Interactions 132 / 75 /
-// 65.)
+// earlier (les_lanes; launch_bi_interactions_cells).  (Before, in us at 4.5 M
+// / 1.2 M / 29 k: 4 lanes with the terms through LDS and a full wait per
+// segment, LapU 240 / 134 / 127, Interpolation 200 / 119 / 113; one lane per
+// owner, Interactions at 29 k 65.)
 template <int D, class Pol, bool PER = false>
 static void launch_groups(const Pol& pol, const int32_t* imove,
                           const float* r, const CellArgs& c, float smax,
@@ -2003,9 +2009,17 @@ void launch_bi_interactions_cells(int dims, const int32_t* imove,
 {
     // with the near flags, only the cells the fused walk listed as near
     const uint32_t* ol = (near && c.flagged) ? c.nlist : nullptr;
+    // A near cell holds few near particles, but above a million particles in
+    // 3D there are cells enough for one lane each.  4 lanes / one, us, on the
+    // lattice and displaced by up to 0.4 of the spacing: 29 k 26 / 56, 27 /
+    // 58; 394 k 49 / 67, 50 / 71; 1.2 M 84 / 78, 89 / 83; 4.5 M 159 / 136,
+    // 166 / 148; 11 M 328 / 303, 355 / 336; 2D 507 k 11 / 13.
+    const bool one = dims == 3 && c.N > 1000000u;
     auto go = [&](const auto& pol, auto dim) {
         constexpr int D = decltype(dim)::value;
-        if (ol)
+        if (ol && one)
+            launch_bi_cells<D>(pol, imove, r, c, smax, s, ol, AQ_CL_NNCELLS);
+        else if (ol)
             launch_groups<D>(pol, imove, r, c, smax, s, false, ol,
                              AQ_CL_NNCELLS, D == 2 ? 16 : 64);
         else

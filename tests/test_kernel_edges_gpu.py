@@ -250,11 +250,12 @@ def test_fluid_pairs_at_the_edge_of_the_support(cuda, tmp_path, dims, n,
 
 
 # element kernels: 16 lanes per owner below 100 k (2D) / 600 k (3D)
-# particles, 4 above; wall edges and corners hold more than one group
+# particles, 4 above (one for BI Interactions above 1 M in 3D, the last case);
+# wall edges and corners hold more than one group
 @pytest.mark.parametrize("dims,dr,hfac,lanes", [
     (2, 0.06, 2.0, 16), (2, 0.011, 2.0, 16), (2, 0.00135, 2.0, 4),
     (3, 0.05, 2.0, 16), (3, 0.031, 3.3, 16), (3, 0.0061, 2.0, 16),
-    (3, 0.0059, 2.0, 4)])
+    (3, 0.0059, 2.0, 4), (3, 0.005, 2.0, 4)])
 def test_element_groups_match_one_lane_walks(cuda, tmp_path, monkeypatch,
                                              dims, dr, hfac, lanes):
     """The boundary-integral element kernels with 4 or 16 lanes per owner
