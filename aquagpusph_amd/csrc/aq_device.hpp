@@ -329,22 +329,23 @@ __device__ __forceinline__ float kernelS_D(float d, float t, float b, float s)
 }
 
 // ---- neighbour walk (types/3D.h:197-219, types/2D.h:174-193) --------------
-// Cell boundaries in four runs of 64 sorted particles spread over the array
-// (252 neighbouring pairs): a measure of the particles per cell, the same for
-// every wavefront of every launch on that array.  N >= 64; called by all 64
-// lanes.
-constexpr uint32_t CELL_SAMPLE = 4 * 63;
+// Cell boundaries in 16 runs of 16 sorted particles spread over the array (240
+// neighbouring pairs): a measure of the particles per cell, the same for
+// every wavefront of every launch on that array.  (Fewer and longer runs are
+// misled where one meets a thin row of cells at the domain's edge.)  N >= 16;
+// called by all 64 lanes.
+constexpr uint32_t CELL_SAMPLE = 16 * 15;
 __device__ __forceinline__ uint32_t
 sampled_cells(const uint32_t* __restrict__ icell, uint32_t N)
 {
-    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t g = (threadIdx.x >> 4) & 3u, o = threadIdx.x & 15u;
     bool edge[4];
 #pragma unroll
     for (uint32_t k = 0; k < 4; k++) {
         // fractions of the golden ratio: no stride the cells could share
-        const uint32_t f = (k + 1u) * 0x9E3779B9u;
-        const uint32_t i = __umulhi(f, N - 63u) + lane;
-        edge[k] = lane != 0 && icell[i] != icell[i - 1];
+        const uint32_t f = (4u * k + g + 1u) * 0x9E3779B9u;
+        const uint32_t i = __umulhi(f, N - 15u) + o;
+        edge[k] = o != 0 && icell[i] != icell[i - 1];
     }
     uint32_t n = 0;
 #pragma unroll

@@ -11,8 +11,8 @@
 //
 // The per-particle kernels are bound by latency and divergence: each lane
 // reads its own candidates one at a time (256 accepted of 1728 in 3D).  At
-// 150 k particles in 3D: Shepard 841 -> 383 us, interactions 1278 ->
-// 519 us, lap p 935 -> 381 us.  A wavefront pays some 2 us per cell among its
+// 150 k particles in 3D: Shepard 841 -> 380 us, interactions 1278 ->
+// 510 us, lap p 935 -> 386 us.  A wavefront pays some 2 us per cell among its
 // particles, though, so where they are scattered over many cells, or where
 // the per-particle form fills the chip, that form is the faster one: a large
 // launch comes in both, and the device takes one (pair_groups_edges).
@@ -369,16 +369,17 @@ void launch_runs(const Pol& pol, const int32_t* imove, const float* r,
 //   3D          0.3       2          5           8         12         64
 //      48 k   64 / 34   59 / 67    56 / 108   60 / 146   57 / 190 147 / 685
 //      64 k  111 / 35  102 / 69    98 / 114   75 / 156   87 / 193 183 / 709
+//     100 k                      156 / 120  146 / 159  145 / 210 293 / 736
 //     150 k  269 / 40  227 / 89   209 / 168  156 / 213  182 / 248 384 / 780
 //     300 k  472 / 80  371 / 172  315 / 280  277 / 370  298 / 392 674 / 1440
 //     1.0 M 1459 / 180 1089 / 362 875 / 582  787 / 776  798 / 988 2088 / 3357
-// The form not taken adds 2 to 4 us (10 us for the 62 k idle wavefronts of
+// The form not taken adds 3 to 5 us (13 us for the 62 k idle wavefronts of
 // 1 M scattered particles).
 uint32_t pair_groups_edges(int dims, uint32_t N)
 {
     if (N <= GROUPS_ALL) return 0;
-    const uint32_t few = dims == 2 ? std::min(18u, N / 16000u + 1u)
-                                   : std::min(8u, N / 25000u + 1u);
+    const uint32_t few = dims == 2 ? std::min(22u, N / 16000u + 1u)
+                                   : std::min(8u, N / 20000u + 1u);
     return CELL_SAMPLE / few;
 }
 
