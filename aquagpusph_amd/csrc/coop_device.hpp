@@ -358,6 +358,18 @@ coop_list_walk(CoopLds<Q, PER>& L, int lane, uint32_t total,
     lds_order();
 }
 
+// Items (groups of 64 / Q particles) a cell is handed out as, S in a full one.
+// Sparse cells, under 16 of the N particles each on average (a spray): items
+// for half as many particles again, since the others would find none.
+template <int Q>
+__device__ __forceinline__ uint32_t items_per_cell(uint32_t S,
+                                                   uint32_t n_heads,
+                                                   uint32_t N)
+{
+    if ((uint64_t)n_heads * 16 <= N) return S;
+    return min(S, (N + N / 2) / n_heads / (64 / Q) + 1u);
+}
+
 // Owners of one group: the owner(i, imove)s of the particles [cstart, cend)
 // with ranks lo .. lo + 64 / Q - 1 into L.owns; returns their number.
 template <int Q, class Lds, class Owner>

@@ -46,7 +46,14 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
     const int q = lane & (Q - 1), o = lane / Q;
     CoopLds<Q, PER>& L = lds[wv];
     if (w.status && (*w.status & 1u)) return;
-    const uint32_t n_items = uni(*w.n_heads) * S;
+    // 3D walk in us with S items per cell / with items_per_cell's (one lane per
+    // particle), at 64, 8 and 1 particles per cell of the fluid:
+    //    8 k (16 lanes)  139 / 138 ( 912)   91 /  51 (268)  109 /  44 (194)
+    //   29 k (4 lanes)   252 / 253 ( 914)  157 / 118 (261)  200 / 113 (219)
+    //  177 k (4 lanes)   786 / 796 (1015)  478 / 234 (397)  701 / 294 (456)
+    const uint32_t n_heads = uni(*w.n_heads);
+    S = items_per_cell<Q>(S, n_heads, w.N);
+    const uint32_t n_items = n_heads * S;
     const float eps = 1E-8f * H;
     const bool flag_el = (SHEP == 2) || (near != nullptr);
     const uint32_t nwv = gridDim.x * WC_WAVES;

@@ -984,7 +984,7 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
 // A lane without a candidate adds Pol::none(), which holds -0: x + -0 is x
 // for every x.
 // PER: the candidate's position is moved to its periodic image first.
-// olist as in cell_kernel_k, its count in n_heads[count_word].
+// olist as in cell_kernel_k, its count in n_heads[count_word] (0: the cells).
 // ---------------------------------------------------------------------------
 template <int D, int Q, class Pol, bool PER>
 __global__ void __launch_bounds__(64 * WC_WAVES)
@@ -1001,8 +1001,10 @@ __global__ void __launch_bounds__(64 * WC_WAVES)
     const int q = lane & (Q - 1), o = lane / Q;
     CoopLds<Q, PER>& L = lds[wv];
     if (w.status && (*w.status & 1u)) return;
-    const uint32_t n_items =
-        (olist ? uni(w.n_heads[count_word]) : uni(*w.n_heads)) * S;
+    const uint32_t n_heads =
+        olist ? uni(w.n_heads[count_word]) : uni(*w.n_heads);
+    if (count_word == 0) S = items_per_cell<Q>(S, n_heads, w.N);
+    const uint32_t n_items = n_heads * S;
     const uint32_t nwv = gridDim.x * WC_WAVES;
     for (uint32_t item = blockIdx.x * WC_WAVES + (uint32_t)wv; item < n_items;
          item += nwv) {

@@ -129,6 +129,23 @@ def _stir(case, seed):
     return case
 
 
+def _spray(case, seed, factor):
+    """The fluid scattered over `factor` times its extent along each axis, in
+    a wider domain box: cells of one or a few particles."""
+    rng = np.random.default_rng(seed)
+    fl, D = case["imove"] == 1, case["dims"]
+    x = case["r"][fl, :D]
+    lo, ext = x.min(0), x.max(0) - x.min(0)
+    case["r"][fl, :D] = lo + ext * (
+        0.5 + factor * (rng.random(x.shape) - 0.5))
+    P = case["params"]
+    P["domain_min"] = [a - factor * e for a, e in zip(P["domain_min"], ext)]
+    P["domain_max"] = [a + factor * e for a, e in zip(P["domain_max"], ext)]
+    P["dt_min"] = 1e-9
+    case["u"][fl, :D] = rng.normal(0, 0.3, x.shape)
+    return case
+
+
 # aq_walk_lanes: the walks and the lanes per particle of their launches
 FLUID, KAHAN, ELEMENTS, LES = range(4)
 
@@ -144,7 +161,8 @@ def _lanes(kernel, case, periodic=0):
     (3, 0.031, "wall"), (3, 0.0187, "wall"), (3, 0.031, "kahan"),
     (3, 0.0187, "kahan"), (2, 1 / 41, "box"), (2, 1 / 160, "box"),
     (3, 1 / 17, "box"), (3, 1 / 33, "box"), (2, 0.011, "morris"),
-    (3, 0.031, "morris")])
+    (3, 0.031, "morris"), (2, 0.011, "spray"), (2, 0.0028, "spray"),
+    (3, 0.031, "spray"), (3, 0.0187, "spray"), (3, 0.0187, "cloud")])
 def test_lanes_per_particle_are_bit_identical(cuda, tmp_path, monkeypatch,
                                               dims, dr, kind):
     """The fused walk with 4 or 16 lanes per particle against the one-lane
@@ -161,7 +179,10 @@ def test_lanes_per_particle_are_bit_identical(cuda, tmp_path, monkeypatch,
             pres = pres + ("resources/Presets/precision.xml",)
     assert _lanes(KAHAN if kind == "kahan" else FLUID, case,
                   kind == "box") > 1
-    case = _stir(case, 7)
+    if kind in ("spray", "cloud"):
+        case = _spray(case, 7, 5.0 if kind == "spray" else 2.0)
+    else:
+        case = _stir(case, 7)
     extra = ""
     if kind == "morris":
         from aquagpusph_amd import casefiles as cf
@@ -300,15 +321,17 @@ def test_les_groups_match_oracle(cuda, tmp_path, dims, n, lanes):
     sim.close()
 
 
-@pytest.mark.parametrize("dims,dr,lanes", [(2, 0.011, 16), (3, 0.0187, 4),
-                                           (3, 0.0083, 1)])
-def test_les_walls_match_oracle(cuda, tmp_path, dims, dr, lanes):
-    """The LES kernels of a dam break with its walls (no periodic images)
-    against the oracle's float32 walk, bit for bit."""
+@pytest.mark.parametrize("dims,dr,lanes,spray", [
+    (2, 0.011, 16, 0), (3, 0.0187, 4, 0), (3, 0.0083, 1, 0), (3, 0.031, 16, 4),
+    (3, 0.0187, 4, 2), (3, 0.0187, 4, 5)])
+def test_les_walls_match_oracle(cuda, tmp_path, dims, dr, lanes, spray):
+    """The LES kernels of a dam break with its walls (no periodic images), as
+    a flow and as a spray, against the oracle's float32 walk, bit for bit."""
     from aquagpusph_amd import casefiles, cases
     from aquagpusph_amd.sim import Simulation
     from oracle import pipeline as op
-    case = _stir(cases.dam_break(dims, dr), 5)
+    case = cases.dam_break(dims, dr)
+    case = _spray(case, 5, spray) if spray else _stir(case, 5)
     assert _lanes(LES, case) == lanes
     sim = Simulation(casefiles.write_case(
         case, str(tmp_path), load=False, presets=casefiles.PBI_PRESETS +
